@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "galp.h"
+#include "device_common.hpp"
 #include "internal.hpp"
 
 namespace galp {
@@ -360,7 +361,7 @@ static int upload_impl(galp_graph *g, const galp_csr_view *c) {
     if (!ooc) GALP_TRY(dev_alloc(g, &g->d_nbr, m));
     GALP_TRY(dev_alloc(g, &g->d_lab[0], n));
     GALP_TRY(dev_alloc(g, &g->d_lab[1], n));
-    GALP_TRY(dev_alloc(g, &g->d_counter, 1));
+    GALP_TRY(dev_alloc(g, &g->d_counter, kCountShards * kCountStride));
     GALP_TRY(dev_alloc(g, &g->d_stop, 1));
     GALP_TRY(dev_alloc(g, &g->d_iters_done, 1));
     GALP_TRY(dev_alloc(g, &g->d_err, 1));

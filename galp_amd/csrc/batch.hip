@@ -174,6 +174,8 @@ k_batch_stop(unsigned long long *__restrict__ gcount, const int64_t *__restrict_
         sactive = 0;
         sstopped = 0;
     }
+    // the class kernels' whole-graph count is not used in batched runs
+    if (threadIdx.x < kCountShards) counter[threadIdx.x * kCountStride] = 0ull;
     __syncthreads();
     unsigned long long tot = 0;
     int active = 0, stopped = 0;
@@ -197,7 +199,6 @@ k_batch_stop(unsigned long long *__restrict__ gcount, const int64_t *__restrict_
     if (threadIdx.x == 0) {
         iter_counts[it] = (long long)stotal;
         *iters_done = it + 1;
-        *counter = 0ull;   // the class kernels' whole-graph count is not used in batched runs
         if (!sactive) *stop = 1;
         if (rebuild) *rebuild = sstopped;
     }

@@ -197,13 +197,27 @@ __device__ __forceinline__ int block_exclusive_scan(int x, int *scratch) {
     return before + inc - x;
 }
 
-// Adds a per-thread count into *counter with one atomic per block of NW waves.
+// The change counter is kept in kCountShards words, one 128-byte line each, and
+// a block adds to the shard of its index: atomics on one word serialise at
+// the L2 at about 14 ns each, so a 280 K-edge class kernel of 1716 blocks took
+// 25 us, nearly all of it its atomics; with the shards its graph's ten
+// iterations (PP-16K) went from 399 to 256 us, RMAT-18 from 2503 to 1966 us,
+// LFR-1M from 3.67 to 2.79 ms.  The sum is taken once per iteration
+// (k_iter_end).
+constexpr int kCountShards = 64;
+constexpr int kCountStride = 16;
+__device__ __forceinline__ unsigned long long *count_shard(unsigned long long *counter) {
+    return counter + (blockIdx.x & (kCountShards - 1)) * kCountStride;
+}
+
+// Adds a per-thread count into its shard of the change counter with one
+// atomic per block of NW waves.
 template <int NW>
 __device__ __forceinline__ void block_count_add(uint32_t mine, unsigned long long *counter,
                                                 uint32_t *scratch) {
     uint32_t s = wave_sum_u32(mine);
     if constexpr (NW == 1) {
-        if (lane_id() == 0 && s) atomicAdd(counter, (unsigned long long)s);
+        if (lane_id() == 0 && s) atomicAdd(count_shard(counter), (unsigned long long)s);
     } else {
         const int w = (int)(threadIdx.x / kWave);
         __syncthreads();
@@ -213,7 +227,7 @@ __device__ __forceinline__ void block_count_add(uint32_t mine, unsigned long lon
             unsigned long long t = 0;
 #pragma unroll
             for (int i = 0; i < NW; ++i) t += scratch[i];
-            if (t) atomicAdd(counter, t);
+            if (t) atomicAdd(count_shard(counter), t);
         }
     }
 }

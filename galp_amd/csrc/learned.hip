@@ -549,7 +549,7 @@ k_cand(const E *__restrict__ off, const int32_t *__restrict__ nbr, const int32_t
     run(std::integral_constant<int, 4>{}, 1, nt[1], nullptr);
     run(std::integral_constant<int, 2>{}, 0, nt[0], nullptr);
     const uint32_t s = wave_sum_u32(changed);
-    if (lane_id() == 0 && s) atomicAdd(counter, (unsigned long long)s);
+    if (lane_id() == 0 && s) atomicAdd(count_shard(counter), (unsigned long long)s);
 }
 
 constexpr int kMergeU = 8;   // entry batches per load round in k_cand_merge
@@ -681,7 +681,7 @@ k_cand_merge(const E *__restrict__ off, const int32_t *__restrict__ mt_vid, int6
             if (dist_out) dist_out[v] = nm;
         }
     }
-    if (lane == 0 && changed) atomicAdd(counter, (unsigned long long)changed);
+    if (lane == 0 && changed) atomicAdd(count_shard(counter), (unsigned long long)changed);
 }
 
 // Training-sample log: for every big vertex, (inputs from the previous

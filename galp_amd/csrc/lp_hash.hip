@@ -906,13 +906,20 @@ k_hub_final(const E *__restrict__ off, const int32_t *__restrict__ nbr, const in
     block_count_add<4>(changed, counter, sred);
 }
 
-__global__ void k_iter_end(unsigned long long *counter, int32_t *stop, long long *iter_counts,
-                           int32_t *iters_done, int it, double thr) {
+// One wave: sums the shards of the change counter, clears them, records the
+// iteration and applies the stop rule.
+__global__ void __launch_bounds__(kCountShards)
+k_iter_end(unsigned long long *counter, int32_t *stop, long long *iter_counts, int32_t *iters_done, int it,
+           double thr) {
+    static_assert(kCountShards == kWave, "one lane per shard");
     if (*stop) return;
-    const unsigned long long c = *counter;
+    unsigned long long c = counter[threadIdx.x * kCountStride];
+    counter[threadIdx.x * kCountStride] = 0ull;
+#pragma unroll
+    for (int s = kWave / 2; s > 0; s >>= 1) c += __shfl_xor(c, s);
+    if (threadIdx.x) return;
     iter_counts[it] = (long long)c;
     *iters_done = it + 1;
-    *counter = 0ull;
     if ((double)c <= thr) *stop = 1;
 }
 
@@ -1166,7 +1173,7 @@ int launch_hash_iteration_incore(galp_graph *g) {
 }
 
 int launch_iter_end(galp_graph *g) {
-    k_iter_end<<<1, 1, 0, g->stream>>>(g->d_counter, g->d_stop, g->d_iter_counts, g->d_iters_done,
+    k_iter_end<<<1, kCountShards, 0, g->stream>>>(g->d_counter, g->d_stop, g->d_iter_counts, g->d_iters_done,
                                        g->iter % kMaxIters, (double)g->n * 1e-5);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(g->ctx, GALP_EHIP, std::string("iter_end launch: ") + hipGetErrorString(e));
