@@ -378,6 +378,7 @@ static int upload_impl(galp_graph *g, const galp_csr_view *c) {
         GALP_HIP(ctx, hipMemcpy(g->d_perm, perm.data(), 4 * (size_t)n, hipMemcpyHostToDevice));
         GALP_HIP(ctx, hipMemcpy(g->d_iperm, iperm.data(), 4 * (size_t)n, hipMemcpyHostToDevice));
     }
+    GALP_TRY(dev_fill_u32(g, (uint32_t *)g->d_stop, 1, 0u));   // the row check's flag, until the first init
     if (g->reorder && !ooc) {
         int64_t *d_off_old = nullptr;
         int32_t *d_nbr_old = nullptr;
@@ -390,7 +391,7 @@ static int upload_impl(galp_graph *g, const galp_csr_view *c) {
         }
         hipError_t e1 = hipMemcpy(d_off_old, off.data(), 8 * (size_t)(n + 1), hipMemcpyHostToDevice);
         hipError_t e2 = m ? hipMemcpy(d_nbr_old, c->neighbors, 4 * (size_t)m, hipMemcpyHostToDevice) : hipSuccess;
-        rc = (e1 == hipSuccess && e2 == hipSuccess) ? dev_permute_rows(g, d_off_old, d_nbr_old, g->d_nbr)
+        rc = (e1 == hipSuccess && e2 == hipSuccess) ? dev_permute_rows(g, d_off_old, d_nbr_old, g->d_nbr, g->d_stop)
                                                     : fail(ctx, GALP_EHIP, "upload of the original CSR failed");
         hipError_t e3 = hipStreamSynchronize(g->stream);
         (void)hipFree(d_off_old);
@@ -399,7 +400,10 @@ static int upload_impl(galp_graph *g, const galp_csr_view *c) {
         if (rc != GALP_OK) return rc;
         if (e3 != hipSuccess) return fail(ctx, GALP_EHIP, std::string("permute: ") + hipGetErrorString(e3));
     } else if (!g->reorder) {
-        if (m && !ooc) GALP_HIP(ctx, hipMemcpy(g->d_nbr, c->neighbors, 4 * (size_t)m, hipMemcpyHostToDevice));
+        if (m && !ooc) {
+            GALP_HIP(ctx, hipMemcpy(g->d_nbr, c->neighbors, 4 * (size_t)m, hipMemcpyHostToDevice));
+            GALP_TRY(dev_check_rows(g, g->d_stop));
+        }
         if (!vlist.empty()) {
             GALP_TRY(dev_alloc(g, &g->d_vlist, (int64_t)vlist.size()));
             GALP_HIP(ctx, hipMemcpy(g->d_vlist, vlist.data(), 4 * vlist.size(), hipMemcpyHostToDevice));
@@ -444,7 +448,10 @@ static int upload_impl(galp_graph *g, const galp_csr_view *c) {
         GALP_TRY(ooc_setup(g, c, offi, perm, iperm, vlist, hub_vertices, hub_tile0, hub_item0));
     }
     if (g->opts.method == GALP_METHOD_SORT) GALP_TRY(sort_setup(g));
+    if (!ooc)
+        GALP_HIP(ctx, hipMemcpyAsync(g->h_pinned, g->d_stop, 4, hipMemcpyDeviceToHost, g->stream));
     GALP_HIP(ctx, hipStreamSynchronize(g->stream));
+    if (!ooc) g->rows_ascend = g->h_pinned[0] == 0;
     if (g->opts.dispatch == GALP_DISPATCH_LEARNED) GALP_TRY(learn_setup(g));
     g->preprocess_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     return GALP_OK;
@@ -495,7 +502,12 @@ int side_join(galp_graph *g, int k) {
 }
 
 static int launch_iteration(galp_graph *g) {
-    if (g->batch) GALP_TRY(launch_batch_lists(g));   // drops the graphs that stopped
+    // from labels[i] = i, no row holding a neighbour twice: the closed form
+    // (out of core only where the rows' last neighbours are on the device)
+    const bool first = g->iter == 0 && g->identity && g->rows_ascend && (!g->ooc || g->ooc->d_last);
+    // drops the graphs that stopped; in the first iteration too, whose end
+    // overwrites the rebuild flag that batch_reset set
+    if (g->batch) GALP_TRY(launch_batch_lists(g));
     switch (g->opts.method) {
     case GALP_METHOD_HASH:
         if (g->opts.dispatch == GALP_DISPATCH_LEARNED) {
@@ -503,12 +515,14 @@ static int launch_iteration(galp_graph *g) {
                 return fail(g->ctx, GALP_ESTATE, "learned dispatch needs a network: call galp_graph_set_mlp");
         }
         // out of core, the learned front runs per batch
-        if (g->ooc) GALP_TRY(launch_ooc_iteration(g));
+        if (first) GALP_TRY(launch_first_iteration(g));
+        else if (g->ooc) GALP_TRY(launch_ooc_iteration(g));
         else GALP_TRY(launch_hash_iteration_incore(g));
         if (g->learn) GALP_TRY(learn_after_iteration(g));
         break;
     case GALP_METHOD_SORT:
-        if (g->ooc) GALP_TRY(launch_ooc_iteration(g));
+        if (first) GALP_TRY(launch_first_iteration(g));
+        else if (g->ooc) GALP_TRY(launch_ooc_iteration(g));
         else GALP_TRY(launch_sort_iteration(g, full_view(g)));
         break;
     default:
@@ -707,6 +721,7 @@ GALP_API int galp_lp_init(galp_graph *g) {
     GALP_HIP(g->ctx, hipStreamSynchronize(g->stream));
     g->cur = 0;
     g->iter = 0;
+    g->identity = true;
     g->initialized = true;
     return GALP_OK;
 }
@@ -733,6 +748,7 @@ GALP_API int galp_lp_set_labels(galp_graph *g, const int32_t *host_labels) {
     GALP_HIP(g->ctx, hipStreamSynchronize(g->stream));
     g->cur = 0;
     g->iter = 0;
+    g->identity = false;
     g->initialized = true;
     return GALP_OK;
 }

@@ -356,6 +356,10 @@ GALP_API int galp_graph_set_batch(galp_graph *g, int64_t ngraphs, const int64_t 
                 return rc;
             }
         }
+        if (const int rc = dev_fill_u32(g, (uint32_t *)B->d_alen, 2 * (NUM_BUCKETS + 1), 0u); rc != GALP_OK) {
+            batch_free(g);
+            return rc;
+        }
         int64_t members = 0;
         for (int b = 0; b < B_HUB; ++b) members += g->bucket[b].nv;
         g->device_bytes += 4 * members + 8 * (NUM_BUCKETS + 1);

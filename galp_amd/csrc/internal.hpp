@@ -220,6 +220,7 @@ struct OocState {
     hipStream_t copy_stream = nullptr;
     hipEvent_t ev_copied[2] = {nullptr, nullptr}, ev_free[2] = {nullptr, nullptr};
     bool used[2] = {false, false};
+    int32_t *d_last = nullptr;           // each row's last neighbour (-1: empty), for the first iteration; may be null
 };
 }  // namespace galp
 
@@ -257,6 +258,11 @@ struct galp_graph {
     int64_t n = 0, m = 0;
     bool off64 = false;
     bool reorder = false;
+    // every row's neighbour ids (input numbering) strictly ascend, so no row
+    // holds a neighbour twice: from labels[i] = i every label then counts
+    // once and the first iteration has a closed form (launch_first_iteration)
+    bool rows_ascend = false;
+    bool identity = false;          // the current labels are labels[i] = i
     hipStream_t stream = nullptr;
     // Side streams for the independent parts of an in-core iteration (the
     // lane-group classes; the LDS classes), forked from and joined back to
@@ -467,8 +473,12 @@ int learn_after_iteration(galp_graph *g);
 int dev_init_labels(galp_graph *g);
 int dev_clear_stop(galp_graph *g);
 int dev_fill_u32(galp_graph *g, uint32_t *p, int64_t n, uint32_t val);
+// Both set *bad (a device word) when a row's input ids do not strictly ascend.
 int dev_permute_rows(galp_graph *g, const int64_t *d_off_old, const int32_t *d_nbr_old,
-                     int32_t *d_nbr_new);
+                     int32_t *d_nbr_new, int32_t *bad);
+int dev_check_rows(galp_graph *g, int32_t *bad);
+// The first iteration from labels[i] = i of a graph whose rows strictly ascend.
+int launch_first_iteration(galp_graph *g);
 int dev_map_labels(galp_graph *g, const int32_t *lab, int32_t *out);
 int dev_unmap_labels(galp_graph *g, const int32_t *in, int32_t *lab);
 

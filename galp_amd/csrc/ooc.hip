@@ -20,6 +20,7 @@
 //             reuse after the kernels that read it.
 
 #include <algorithm>
+#include <atomic>
 #include <cstring>
 #include <vector>
 
@@ -66,6 +67,7 @@ void ooc_free(galp_graph *g) {
         if (O->ev_free[k]) (void)hipEventDestroy(O->ev_free[k]);
     }
     if (O->copy_stream) (void)hipStreamDestroy(O->copy_stream);
+    if (O->d_last) (void)hipFree(O->d_last);
     if (O->h_nbr) (void)hipHostFree(O->h_nbr);
     delete O;
     g->ooc = nullptr;
@@ -85,6 +87,10 @@ int ooc_setup(galp_graph *g, const galp_csr_view *c, const std::vector<int64_t> 
         return fail(g->ctx, GALP_ENOMEM, "pinned host buffer for the neighbour array");
     }
     const int32_t *src = c->neighbors;
+    // each row's last neighbour (internal numbering), and whether every row's
+    // input ids strictly ascend: the first iteration then needs no batch
+    std::vector<int32_t> last((size_t)n, -1);
+    std::atomic<bool> ascend{true};
     if (g->reorder) {
         const bool o64 = c->offsets_are_64 != 0;
         parallel_for(0, n, [&](int64_t k) {
@@ -92,13 +98,26 @@ int ooc_setup(galp_graph *g, const galp_csr_view *c, const std::vector<int64_t> 
             const int64_t b = o64 ? ((const int64_t *)c->offsets)[v] : ((const int32_t *)c->offsets)[v];
             const int64_t d = offi[(size_t)k + 1] - offi[(size_t)k];
             int32_t *dst = O->h_nbr + offi[(size_t)k];
-            for (int64_t j = 0; j < d; ++j) dst[j] = perm[(size_t)src[b + j]];
+            bool up = true;
+            for (int64_t j = 0; j < d; ++j) {
+                dst[j] = perm[(size_t)src[b + j]];
+                up &= j == 0 || src[b + j - 1] < src[b + j];
+            }
+            if (d) last[(size_t)k] = dst[d - 1];
+            if (!up) ascend.store(false, std::memory_order_relaxed);
         });
     } else {
         const int64_t chunk = 1 << 22;
         parallel_for(0, (m + chunk - 1) / chunk, [&](int64_t k) {
             const int64_t lo = k * chunk, hi = std::min(m, lo + chunk);
             std::memcpy(O->h_nbr + lo, src + lo, 4 * (size_t)(hi - lo));
+        });
+        parallel_for(0, n, [&](int64_t v) {
+            const int64_t b = offi[(size_t)v], e = offi[(size_t)v + 1];
+            bool up = true;
+            for (int64_t j = b + 1; j < e; ++j) up &= src[j - 1] < src[j];
+            if (e > b) last[(size_t)v] = src[e - 1];
+            if (!up) ascend.store(false, std::memory_order_relaxed);
         });
     }
     // batches and their share of every class and of the hub lists
@@ -157,6 +176,15 @@ int ooc_setup(galp_graph *g, const galp_csr_view *c, const std::vector<int64_t> 
     if (g->opts.policy == GALP_POLICY_OOC_ASYNC &&
         hipStreamCreateWithFlags(&O->copy_stream, hipStreamNonBlocking) != hipSuccess)
         return fail(g->ctx, GALP_EHIP, "out-of-core copy stream");
+    // kept only where the memory budget has room for it: without it the first
+    // iteration streams like the others
+    const std::string err = g->ctx->err;
+    if (ascend.load() && dev_alloc(g, &O->d_last, n) == GALP_OK) {
+        if (n && hipMemcpy(O->d_last, last.data(), 4 * (size_t)n, hipMemcpyHostToDevice) != hipSuccess)
+            return fail(g->ctx, GALP_EHIP, "out-of-core last neighbours");
+        g->rows_ascend = true;
+    }
+    g->ctx->err = err;   // doing without is no failure
     return GALP_OK;
 }
 
