@@ -75,6 +75,12 @@ void prof_begin_dev(galp_graph *g, const char *name, const int64_t *dev_bytes, P
     if (g->prof.on) pl->dev_bytes = dev_bytes;
 }
 
+void prof_begin_class(galp_graph *g, const char *name, int b, double alg_bytes, PendingLaunch *pl) {
+    if (g->prof.on && front_now(g) && g->front->d_bytes)
+        prof_begin_dev(g, name, g->front->d_bytes + (int64_t)(g->iter % kMaxIters) * NUM_BUCKETS + b, pl);
+    else prof_begin(g, name, alg_bytes, pl);
+}
+
 void prof_end(galp_graph *g, PendingLaunch *pl) {
     if (!g->prof.on) return;
     if (pl->e1) (void)hipEventRecord(pl->e1, g->stream);
@@ -125,6 +131,7 @@ static void dev_free_all(galp_graph *g) {
     sort_free(g);
     ooc_free(g);
     batch_free(g);
+    front_free(g);
     if (g->gexec) (void)hipGraphExecDestroy(g->gexec);
     g->gexec = nullptr;
     void *ptrs[] = {g->d_off, g->d_nbr, g->d_lab[0], g->d_lab[1], g->d_perm, g->d_iperm, g->d_vlist,
@@ -378,7 +385,20 @@ static int upload_impl(galp_graph *g, const galp_csr_view *c) {
         GALP_HIP(ctx, hipMemcpy(g->d_perm, perm.data(), 4 * (size_t)n, hipMemcpyHostToDevice));
         GALP_HIP(ctx, hipMemcpy(g->d_iperm, iperm.data(), 4 * (size_t)n, hipMemcpyHostToDevice));
     }
+    // Whether every row's ids strictly ascend (the closed form of the first
+    // iteration) and, then, whether the graph is symmetric (the lists of
+    // frontier.hip), on the rows in their input numbering.
     GALP_TRY(dev_fill_u32(g, (uint32_t *)g->d_stop, 1, 0u));   // the row check's flag, until the first init
+    const bool lists = !ooc && m >= kFrontMinEdges &&
+                       (g->opts.method == GALP_METHOD_HASH ? g->opts.variant == 1
+                                                           : g->opts.policy == GALP_POLICY_INCORE);
+    bool symmetric = false;
+    auto check_rows = [&](const void *d_off, bool off64, const int32_t *d_nbr) {
+        GALP_HIP(ctx, hipMemcpyAsync(g->h_pinned, g->d_stop, 4, hipMemcpyDeviceToHost, g->stream));
+        GALP_HIP(ctx, hipStreamSynchronize(g->stream));
+        g->rows_ascend = g->h_pinned[0] == 0;
+        return lists && g->rows_ascend ? dev_check_symmetric(g, d_off, off64, d_nbr, &symmetric) : GALP_OK;
+    };
     if (g->reorder && !ooc) {
         int64_t *d_off_old = nullptr;
         int32_t *d_nbr_old = nullptr;
@@ -393,6 +413,7 @@ static int upload_impl(galp_graph *g, const galp_csr_view *c) {
         hipError_t e2 = m ? hipMemcpy(d_nbr_old, c->neighbors, 4 * (size_t)m, hipMemcpyHostToDevice) : hipSuccess;
         rc = (e1 == hipSuccess && e2 == hipSuccess) ? dev_permute_rows(g, d_off_old, d_nbr_old, g->d_nbr, g->d_stop)
                                                     : fail(ctx, GALP_EHIP, "upload of the original CSR failed");
+        if (rc == GALP_OK) rc = check_rows(d_off_old, true, d_nbr_old);
         hipError_t e3 = hipStreamSynchronize(g->stream);
         (void)hipFree(d_off_old);
         (void)hipFree(d_nbr_old);
@@ -404,6 +425,7 @@ static int upload_impl(galp_graph *g, const galp_csr_view *c) {
             GALP_HIP(ctx, hipMemcpy(g->d_nbr, c->neighbors, 4 * (size_t)m, hipMemcpyHostToDevice));
             GALP_TRY(dev_check_rows(g, g->d_stop));
         }
+        if (!ooc) GALP_TRY(check_rows(g->d_off, g->off64, g->d_nbr));
         if (!vlist.empty()) {
             GALP_TRY(dev_alloc(g, &g->d_vlist, (int64_t)vlist.size()));
             GALP_HIP(ctx, hipMemcpy(g->d_vlist, vlist.data(), 4 * vlist.size(), hipMemcpyHostToDevice));
@@ -448,11 +470,12 @@ static int upload_impl(galp_graph *g, const galp_csr_view *c) {
         GALP_TRY(ooc_setup(g, c, offi, perm, iperm, vlist, hub_vertices, hub_tile0, hub_item0));
     }
     if (g->opts.method == GALP_METHOD_SORT) GALP_TRY(sort_setup(g));
-    if (!ooc)
-        GALP_HIP(ctx, hipMemcpyAsync(g->h_pinned, g->d_stop, 4, hipMemcpyDeviceToHost, g->stream));
     GALP_HIP(ctx, hipStreamSynchronize(g->stream));
-    if (!ooc) g->rows_ascend = g->h_pinned[0] == 0;
     if (g->opts.dispatch == GALP_DISPATCH_LEARNED) GALP_TRY(learn_setup(g));
+    if (symmetric) {
+        GALP_TRY(front_setup(g));
+        GALP_HIP(ctx, hipStreamSynchronize(g->stream));
+    }
     g->preprocess_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     return GALP_OK;
 }
@@ -508,6 +531,7 @@ static int launch_iteration(galp_graph *g) {
     // drops the graphs that stopped; in the first iteration too, whose end
     // overwrites the rebuild flag that batch_reset set
     if (g->batch) GALP_TRY(launch_batch_lists(g));
+    if (!first && front_now(g)) GALP_TRY(launch_front(g));
     switch (g->opts.method) {
     case GALP_METHOD_HASH:
         if (g->opts.dispatch == GALP_DISPATCH_LEARNED) {

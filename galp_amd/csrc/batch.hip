@@ -165,7 +165,7 @@ __global__ void __launch_bounds__(1024)
 k_batch_stop(unsigned long long *__restrict__ gcount, const int64_t *__restrict__ gn, int32_t *__restrict__ gstop,
              int32_t *__restrict__ giters, int64_t ngraphs, unsigned long long *__restrict__ counter,
              int32_t *__restrict__ stop, long long *__restrict__ iter_counts, int32_t *__restrict__ iters_done,
-             int it, int64_t *__restrict__ rebuild) {
+             int it, int64_t *__restrict__ rebuild, int64_t *__restrict__ front) {
     __shared__ unsigned long long stotal;
     __shared__ int32_t sactive, sstopped;
     if (*stop) return;
@@ -176,6 +176,7 @@ k_batch_stop(unsigned long long *__restrict__ gcount, const int64_t *__restrict_
     }
     // the class kernels' whole-graph count is not used in batched runs
     if (threadIdx.x < kCountShards) counter[threadIdx.x * kCountStride] = 0ull;
+    if (front && threadIdx.x < kFrontCtl) front[threadIdx.x] = 0;   // the frontier's control words
     __syncthreads();
     unsigned long long tot = 0;
     int active = 0, stopped = 0;
@@ -264,7 +265,7 @@ int launch_batch_end(galp_graph *g) {
     k_batch_epilogue<<<grid, 256, 0, g->stream>>>(prev, next, B->d_gid, B->d_gstop, B->d_gcount, g->n, g->d_stop);
     k_batch_stop<<<1, 1024, 0, g->stream>>>(B->d_gcount, B->d_gn, B->d_gstop, B->d_giters, B->ngraphs, g->d_counter,
                                             g->d_stop, g->d_iter_counts, g->d_iters_done, g->iter % kMaxIters,
-                                            B->lists ? B->d_alen + NUM_BUCKETS : nullptr);
+                                            B->lists ? B->d_alen + NUM_BUCKETS : nullptr, front_ctl(g));
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? GALP_OK : fail(g->ctx, GALP_EHIP, std::string("batch epilogue: ") + hipGetErrorString(e));
 }

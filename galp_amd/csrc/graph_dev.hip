@@ -33,8 +33,9 @@ __global__ void k_fill_u32(uint32_t *p, int64_t n, uint32_t val) {
 // One thread per shard of the change counter.
 __global__ void __launch_bounds__(kCountShards)
 k_reset_control(unsigned long long *counter, int32_t *stop, int32_t *iters_done,
-                                int32_t *err, int reset_done) {
+                                int32_t *err, int reset_done, int64_t *front) {
     counter[threadIdx.x * kCountStride] = 0ull;
+    if (front && threadIdx.x < kFrontCtl) front[threadIdx.x] = 0;
     if (threadIdx.x) return;
     *stop = 0;
     if (reset_done) {
@@ -152,14 +153,14 @@ static int grid1d(int64_t n, int threads) {
 
 int dev_init_labels(galp_graph *g) {
     if (g->n) k_iota2<<<grid1d(g->n, 256), 256, 0, g->stream>>>(g->d_lab[0], g->d_lab[1], g->n);
-    k_reset_control<<<1, kCountShards, 0, g->stream>>>(g->d_counter, g->d_stop, g->d_iters_done, g->d_err, 1);
+    k_reset_control<<<1, kCountShards, 0, g->stream>>>(g->d_counter, g->d_stop, g->d_iters_done, g->d_err, 1, front_ctl(g));
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(g->ctx, GALP_EHIP, std::string("init kernels: ") + hipGetErrorString(e));
     return GALP_OK;
 }
 
 int dev_clear_stop(galp_graph *g) {
-    k_reset_control<<<1, kCountShards, 0, g->stream>>>(g->d_counter, g->d_stop, g->d_iters_done, g->d_err, 0);
+    k_reset_control<<<1, kCountShards, 0, g->stream>>>(g->d_counter, g->d_stop, g->d_iters_done, g->d_err, 0, front_ctl(g));
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(g->ctx, GALP_EHIP, std::string("reset kernel: ") + hipGetErrorString(e));
     return GALP_OK;

@@ -225,6 +225,50 @@ struct OocState {
 }  // namespace galp
 
 namespace galp {
+// Iterations over the rows that can still change (frontier.hip): marks and
+// per-class lists of the vertices with a neighbour that changed, and the
+// control words of one iteration, cleared by its bookkeeping kernel.
+constexpr int kFrontEdges = NUM_BUCKETS;          // [0, NUM_BUCKETS): list lengths (B_HUB: their tiles)
+constexpr int kFrontPush = 2 * NUM_BUCKETS;       // edges of the lists per class, then: edges of changed vertices
+constexpr int kFrontReady = kFrontPush + 1;       // 1: the lists are built
+constexpr int kFrontCtl = 32;
+static_assert(kFrontReady < kFrontCtl && kFrontCtl <= 64, "one wave clears the control words");
+// Lists are tried when the changed vertices' rows hold at most m /
+// kFrontPushDiv edges, on graphs of at least kFrontMinEdges edges: on smaller
+// ones the three launches of an iteration (12 us) and the set-up (the
+// symmetry check, the memory) cost what the lists save (RMAT-18, 7.6 M
+// edges: 1741 us without, 1786 with; LFR-300K uploaded and run once, 6 M
+// edges: 5.7 ms without, 6.3 with; RMAT-20, 31 M: 5.6 and 3.8 ms).
+constexpr int64_t kFrontPushDiv = 8;
+constexpr int64_t kFrontMinEdges = (int64_t)1 << 23;
+struct FrontState {
+    uint32_t *d_mem = nullptr;      // holds all but d_bytes
+    uint32_t *d_mark = nullptr;     // one byte per vertex
+    int32_t *d_lists = nullptr;     // class b's list at bucket[b].v0
+    int32_t *d_hub_sel = nullptr;   // hub processed this iteration
+    int32_t *d_tiles = nullptr;     // tiles of those hubs
+    int64_t *d_ctl = nullptr;       // kFrontCtl words
+    int64_t *d_bytes = nullptr;     // profiling: algorithmic bytes per iteration and class
+};
+// What a class kernel reads of it: the control words (null: always the whole
+// class), its list (the hub kernels: a flag per hub) and the list's length.
+struct FrontList {
+    const int64_t *ctl;
+    int64_t max_edges;
+    const int32_t *list;
+    const int64_t *len;
+};
+// The lists are walked when they were built and hold few enough edges.
+__device__ __forceinline__ bool front_lists_on(const FrontList &f) {
+    if (!f.ctl || !f.ctl[kFrontReady]) return false;
+    int64_t edges = 0;
+#pragma unroll
+    for (int b = 0; b < NUM_BUCKETS; ++b) edges += f.ctl[kFrontEdges + b];
+    return edges <= f.max_edges;
+}
+}  // namespace galp
+
+namespace galp {
 // Batched runs (batch.hip): graph id per vertex (internal numbering), per
 // graph vertex count, change counter, stop flag and iterations done.
 struct BatchState {
@@ -320,6 +364,7 @@ struct galp_graph {
     galp::SortState *sort = nullptr;
     galp::OocState *ooc = nullptr;
     galp::BatchState *batch = nullptr;
+    galp::FrontState *front = nullptr;
     int8_t tune[galp::NUM_BUCKETS] = {};   // kernel configuration per degree class (autotuner)
     int8_t streams = 0;   // in-core class kernels: 0 by size, 1 one stream, 3 three (the autotuner's choice)
     // learned dispatch in core: bit i set = iteration i routes by the network,
@@ -445,6 +490,24 @@ inline void invalidate_captured(galp_graph *g) {
     g->gexec_niter = -1;
 }
 
+// Iterations over the rows that can still change (frontier.hip).
+int front_setup(galp_graph *g);
+void front_free(galp_graph *g);
+bool front_now(const galp_graph *g);   // the iteration being launched may use the lists
+int launch_front(galp_graph *g);
+int dev_check_symmetric(galp_graph *g, const void *off, bool off64, const int32_t *nbr, bool *symmetric);
+inline FrontList front_list(const galp_graph *g, int b) {
+    if (!front_now(g)) return FrontList{nullptr, 0, nullptr, nullptr};
+    const FrontState *F = g->front;
+    return FrontList{F->d_ctl, g->m / 4 * 3, F->d_lists + g->bucket[b].v0, F->d_ctl + b};
+}
+inline FrontList front_hubs(const galp_graph *g) {   // list: a flag per hub; len: their tiles
+    FrontList f = front_list(g, B_HUB);
+    if (f.ctl) f.list = g->front->d_hub_sel;
+    return f;
+}
+inline int64_t *front_ctl(const galp_graph *g) { return g->front ? g->front->d_ctl : nullptr; }
+
 // Batched runs (batch.hip).
 void batch_free(galp_graph *g);
 int batch_reset(galp_graph *g);
@@ -488,5 +551,8 @@ void prof_end(galp_graph *g, PendingLaunch *pl);
 // As prof_begin, with the launch's algorithmic bytes read from the device
 // when the timings are collected.
 void prof_begin_dev(galp_graph *g, const char *name, const int64_t *dev_bytes, PendingLaunch *pl);
+// A class kernel's launch: alg_bytes when it walks its whole class, else what
+// the lists hold, read from the device.
+void prof_begin_class(galp_graph *g, const char *name, int b, double alg_bytes, PendingLaunch *pl);
 
 }  // namespace galp

@@ -139,13 +139,14 @@ k_dispatch(const E *__restrict__ off, const int32_t *__restrict__ vlist, int64_t
            int32_t *__restrict__ cw_v, int64_t *__restrict__ cw_e0, int32_t *__restrict__ cw_len,
            int32_t *__restrict__ cw_pslot, const int64_t *__restrict__ cw_base, int32_t *const *__restrict__ plist,
            int32_t *__restrict__ hub_hd, int64_t *__restrict__ ctr, int64_t *__restrict__ cand_bytes,
-           const int32_t *__restrict__ stop) {
+           const int32_t *__restrict__ stop, FrontList front) {
     __shared__ uint8_t scode[kDispChunk];
     __shared__ int32_t sv[kDispChunk];
     __shared__ int64_t sb[kDispChunk], sd[kDispChunk];
     __shared__ unsigned long long scount[kSlots];
     __shared__ unsigned long long sbytes;
     if (*stop) return;
+    if (front_lists_on(front)) return;   // the class kernels walk the frontier's lists
     if (threadIdx.x < kSlots) scount[threadIdx.x] = 0;
     if (threadIdx.x == 0) sbytes = 0;
     __syncthreads();
@@ -1019,7 +1020,7 @@ static void launch_dispatch(galp_graph *g, LearnState *L, int32_t *const *dpl, c
         L->d_dist[L->dcur], L->cand_thresh, g->nhubs, L->d_mt_of, L->d_mt_cand, L->d_hub_sel, L->d_cw_v,
         L->d_cw_e0, L->d_cw_len, L->d_cw_pslot, L->d_cw_base, dpl, L->d_hub_hd, L->d_plist_n,
         L->d_cand_bytes + g->iter % kMaxIters,
-        g->d_stop);
+        g->d_stop, front_list(g, B_HUB));
 }
 
 // The dispatch and the candidate path over big vertices [v0, v0 + nv) (an

@@ -311,7 +311,7 @@ k_hash_lds(const E *__restrict__ off, const int32_t *__restrict__ nbr,
            const int32_t *__restrict__ vlist, int64_t v0, int64_t nv, const int64_t *__restrict__ nv_dev,
            const int32_t *__restrict__ vlistB, const int64_t *__restrict__ nvB_dev,
            unsigned long long *__restrict__ counter, const int32_t *__restrict__ stop,
-           int32_t *__restrict__ err, int32_t *__restrict__ distinct) {
+           int32_t *__restrict__ err, int32_t *__restrict__ distinct, FrontList front) {
     static_assert((1 << CAPBITS) >= 2 * T * EPT, "load factor must stay <= 1/2");
     constexpr int CAP = 1 << CAPBITS;
     __shared__ uint32_t skey[CAP];
@@ -320,7 +320,13 @@ k_hash_lds(const E *__restrict__ off, const int32_t *__restrict__ nbr,
     __shared__ unsigned long long sred64[T / kWave];
     if (*stop) return;
     if (nv_dev) nv = *nv_dev;   // lists built on the device this iteration
-    const int64_t nvB = nvB_dev ? *nvB_dev : 0;
+    int64_t nvB = nvB_dev ? *nvB_dev : 0;
+    if (front_lists_on(front)) {   // only the rows that can still change
+        vlist = front.list;
+        v0 = 0;
+        nv = *front.len;
+        nvB = 0;
+    }
     if ((int64_t)blockIdx.x >= nv && (int64_t)blockIdx.x >= nvB) return;
     for (int s = threadIdx.x; s < CAP; s += T) {
         skey[s] = kEmpty;
@@ -384,10 +390,12 @@ struct HubTilePolicy {
     const int32_t *hub_sel;   // null: every hub; else only hubs with a non-zero flag
     int *sscan;               // T / kWave ints of LDS for the block scan
     const int32_t *hub_hd;    // null: every hub; else only hubs whose flag equals HD
+    const int32_t *tlist;     // null: tiles [.., ntiles); else the first ntiles entries of a tile list
 
     __device__ Item item(int64_t t) const {
         Item it{false, 0, 0, 0, 1, 0, t};
         if (t < ntiles) {
+            if (tlist) it.t = t = tlist[t];
             const int h = tile_hub[t];
             const int64_t v = hub_vid[h];
             const int64_t rb = (int64_t)off[v], re = (int64_t)off[v + 1];
@@ -487,7 +495,8 @@ k_hub_tile(const E *__restrict__ off, const int32_t *__restrict__ nbr, const int
            uint32_t *__restrict__ out_key, uint32_t *__restrict__ out_ent,
            int32_t *__restrict__ tile_idx, const int32_t *__restrict__ stop, int32_t *__restrict__ err,
            const int32_t *__restrict__ hub_sel, const int64_t *__restrict__ nsel,
-           const int32_t *__restrict__ hub_hd, const int64_t *__restrict__ nhd) {
+           const int32_t *__restrict__ hub_hd, const int64_t *__restrict__ nhd, FrontList front,
+           const int32_t *__restrict__ front_tiles) {
     constexpr int CAP = 1 << kHubTileCapBits;
     constexpr int EPT = kHubTile / T;
     // keys | counts | positions; the partition histogram (P + 1 entries)
@@ -496,7 +505,17 @@ k_hub_tile(const E *__restrict__ off, const int32_t *__restrict__ nbr, const int
     __shared__ uint32_t tab[3 * CAP];
     __shared__ int sscan[T / kWave];
     if (*stop) return;
-    if (nsel) {   // learned dispatch: nsel hubs on this path, nhd of them high-distinct
+    if (front_lists_on(front)) {   // only the hubs that can still change, all in the first launch
+        if (HD) return;
+        hub_sel = nullptr;
+        hub_hd = nullptr;
+        tbase = 0;
+        ntiles = *front.len;
+        if ((int64_t)blockIdx.x >= ntiles) return;
+    } else {
+        front_tiles = nullptr;
+    }
+    if (!front_tiles && nsel) {   // learned dispatch: nsel hubs on this path, nhd of them high-distinct
         const int64_t ns = *nsel, nh = nhd ? *nhd : 0;
         if ((hub_hd ? (HD ? nh : ns - nh) : ns) == 0) return;   // none for this launch
     }
@@ -509,7 +528,7 @@ k_hub_tile(const E *__restrict__ off, const int32_t *__restrict__ nbr, const int
     HubTilePolicy<T, EPT, E, HD> pol{off,      tile_hub, hub_tile0,     hub_vid,  hub_nparts, tile_idx_off,
                                      ntiles,   tab,      tab + CAP,     tab + 2 * CAP,        tab + CAP,
                                      out_key,  out_ent,  tile_idx,      err,      hub_sel,    sscan,
-                                     hub_hd};
+                                     hub_hd,   front_tiles};
     pipelined<T, EPT>(pol, nbr, prev, tbase + (int64_t)blockIdx.x, (int64_t)gridDim.x, (int)threadIdx.x);
 }
 
@@ -531,9 +550,14 @@ k_hub_merge_small(const HubItem *__restrict__ items, int64_t ibase, int64_t nite
                   const int32_t *__restrict__ tile_idx, const uint32_t *__restrict__ out_key,
                   const uint32_t *__restrict__ out_ent, unsigned long long *__restrict__ hub_best,
                   const int32_t *__restrict__ hub_sel, uint32_t *__restrict__ hub_distinct,
-                  const int64_t *__restrict__ nsel, int32_t *__restrict__ big, const int32_t *__restrict__ stop) {
+                  const int64_t *__restrict__ nsel, int32_t *__restrict__ big, const int32_t *__restrict__ stop,
+                  FrontList front) {
     constexpr int NW = kHmSmallT / kWave;
     __shared__ int32_t slo[NW][kWave], sstart[NW][kWave];
+    if (front_lists_on(front)) {
+        hub_sel = front.list;
+        nsel = front.len;
+    }
     if (*stop || (nsel && *nsel == 0)) return;
     const int lane = lane_id(), w = (int)(threadIdx.x / kWave);
     const int64_t iend = ibase + nitems, stride = (int64_t)gridDim.x * NW;
@@ -669,7 +693,7 @@ k_hub_merge(const HubItem *__restrict__ items, int64_t ibase, int64_t nitems, co
             const int32_t *__restrict__ tile_idx, const uint32_t *__restrict__ out_key,
             const uint32_t *__restrict__ out_ent, unsigned long long *__restrict__ hub_best,
             const int32_t *__restrict__ stop, int32_t *__restrict__ err, uint32_t *__restrict__ hub_distinct,
-            const int64_t *__restrict__ nsel) {
+            const int64_t *__restrict__ nsel, FrontList front) {
     constexpr int CAP = 1 << kHubMergeCapBits;
     constexpr int EPT = 4;   // entries per thread and pass
     __shared__ uint32_t skey[CAP];
@@ -683,6 +707,7 @@ k_hub_merge(const HubItem *__restrict__ items, int64_t ibase, int64_t nitems, co
     __shared__ unsigned long long sred64[T / kWave];
     __shared__ int32_t sfull;   // a label found the table full in this round
     __shared__ uint32_t sbig[T / 32];   // flags of the current chunk of items
+    if (front_lists_on(front)) nsel = front.len;   // the wave merge has cleared the other hubs' flags
     if (*stop || (nsel && *nsel == 0)) return;
     for (int s = threadIdx.x; s < CAP; s += T) {
         skey[s] = kEmpty;
@@ -885,8 +910,12 @@ k_hub_final(const E *__restrict__ off, const int32_t *__restrict__ nbr, const in
             int64_t nhubs, unsigned long long *__restrict__ hub_best, const int32_t *__restrict__ hub_sel,
             uint32_t *__restrict__ hub_distinct, int32_t *__restrict__ distinct, const int32_t *__restrict__ prev,
             int32_t *__restrict__ next, unsigned long long *__restrict__ counter,
-            const int32_t *__restrict__ stop, const int64_t *__restrict__ nsel) {
+            const int32_t *__restrict__ stop, const int64_t *__restrict__ nsel, FrontList front) {
     __shared__ uint32_t sred[256 / kWave];
+    if (front_lists_on(front)) {
+        hub_sel = front.list;
+        nsel = front.len;
+    }
     if (*stop || (nsel && *nsel == 0)) return;
     uint32_t changed = 0;
     for (int64_t h = (int64_t)blockIdx.x * 256 + threadIdx.x; h < nhubs; h += (int64_t)gridDim.x * 256) {
@@ -906,13 +935,15 @@ k_hub_final(const E *__restrict__ off, const int32_t *__restrict__ nbr, const in
     block_count_add<4>(changed, counter, sred);
 }
 
-// One wave: sums the shards of the change counter, clears them, records the
-// iteration and applies the stop rule.
+// One wave: sums the shards of the change counter, clears them and the
+// frontier's control words (front may be null), records the iteration and
+// applies the stop rule.
 __global__ void __launch_bounds__(kCountShards)
 k_iter_end(unsigned long long *counter, int32_t *stop, long long *iter_counts, int32_t *iters_done, int it,
-           double thr) {
+           double thr, int64_t *front) {
     static_assert(kCountShards == kWave, "one lane per shard");
     if (*stop) return;
+    if (front && threadIdx.x < kFrontCtl) front[threadIdx.x] = 0;
     unsigned long long c = counter[threadIdx.x * kCountStride];
     counter[threadIdx.x * kCountStride] = 0ull;
 #pragma unroll
@@ -944,7 +975,8 @@ static void launch_group(galp_graph *g, const IterView &w, int bid, const int32_
     const BucketRange &r = w.cls[bid];
     if (!r.nv) return;
     PendingLaunch pl;
-    prof_begin(g, kBucketName[bid], class_bytes<E>(r), &pl);
+    prof_begin_class(g, kBucketName[bid], bid, class_bytes<E>(r), &pl);
+    const FrontList fl = front_list(g, bid);
     const int64_t per_block = 256 / G;
     const int64_t blocks = (r.nv + per_block - 1) / per_block;
     // learned dispatch: the sweep-only resolver in iterations where most big
@@ -955,15 +987,15 @@ static void launch_group(galp_graph *g, const IterView &w, int bid, const int32_
     if (batch_lists(g))   // the running graphs' vertices of the class
         k_group<G, HashGroupResolve, HashGroupSweep, true, E><<<grid_for(g, blocks, blocks_per_cu), 256, 0, g->stream>>>(
             (const E *)w.off, w.nbr, prev, next, g->batch->d_alist[bid], 0, r.nv, g->batch->d_alen + bid,
-            g->d_counter, g->d_stop, hd, hd_total);
+            g->d_counter, g->d_stop, hd, hd_total, fl);
     else if (g->d_vlist)
         k_group<G, HashGroupResolve, HashGroupSweep, true, E><<<grid_for(g, blocks, blocks_per_cu), 256, 0, g->stream>>>(
             (const E *)w.off, w.nbr, prev, next, g->d_vlist, r.v0, r.nv, nullptr, g->d_counter, g->d_stop, hd,
-            hd_total);
+            hd_total, fl);
     else
         k_group<G, HashGroupResolve, HashGroupSweep, false, E><<<grid_for(g, blocks, blocks_per_cu), 256, 0,
                                                                  g->stream>>>(
-            (const E *)w.off, w.nbr, prev, next, nullptr, r.v0, r.nv, nullptr, g->d_counter, g->d_stop, hd, hd_total);
+            (const E *)w.off, w.nbr, prev, next, nullptr, r.v0, r.nv, nullptr, g->d_counter, g->d_stop, hd, hd_total, fl);
     prof_end(g, &pl);
 }
 
@@ -973,21 +1005,22 @@ static void launch_lds(galp_graph *g, const IterView &w, int bid, const int32_t 
     const BucketRange &r = w.cls[bid];
     if (!r.nv) return;
     PendingLaunch pl;
-    prof_begin(g, kBucketName[bid], class_bytes<E>(r), &pl);
+    prof_begin_class(g, kBucketName[bid], bid, class_bytes<E>(r), &pl);
+    const FrontList fl = front_list(g, bid);
     int32_t *dist = distinct_out(g);
     if (batch_lists(g))   // the running graphs' vertices of the class
         k_hash_lds<T, EPT, CAPBITS, E, 3><<<grid_for(g, r.nv, blocks_per_cu), T, 0, g->stream>>>(
             (const E *)w.off, w.nbr, prev, next, g->batch->d_alist[bid], 0, r.nv, g->batch->d_alen + bid, nullptr,
-            nullptr, g->d_counter, g->d_stop, g->d_err, dist);
+            nullptr, g->d_counter, g->d_stop, g->d_err, dist, fl);
     else if (learned_now(g))   // this iteration's two lists for the class
         k_hash_lds<T, EPT, CAPBITS, E, 3><<<grid_for(g, r.nv, blocks_per_cu), T, 0, g->stream>>>(
             (const E *)w.off, w.nbr, prev, next, g->learn->plist[bid], 0, r.nv, g->learn->d_plist_n + bid,
             g->learn->plist[NUM_BUCKETS + bid], g->learn->d_plist_n + kCtrHd + bid, g->d_counter, g->d_stop,
-            g->d_err, dist);
+            g->d_err, dist, fl);
     else
         k_hash_lds<T, EPT, CAPBITS, E, 3><<<grid_for(g, r.nv, blocks_per_cu), T, 0, g->stream>>>(
             (const E *)w.off, w.nbr, prev, next, g->d_vlist, r.v0, r.nv, nullptr, nullptr, nullptr, g->d_counter,
-            g->d_stop, g->d_err, dist);
+            g->d_stop, g->d_err, dist, fl);
     prof_end(g, &pl);
 }
 
@@ -1006,31 +1039,33 @@ static void launch_hubs(galp_graph *g, const IterView &w, const int32_t *prev, i
     const int64_t *nsel = sel ? g->learn->d_plist_n + kCtrPlainHubs : nullptr;
     const int64_t *nhd = sel ? g->learn->d_plist_n + kCtrHd + B_HUB : nullptr;
     PendingLaunch pl;
-    prof_begin(g, "hub_tile", 8.0 * hub_edges, &pl);
+    const FrontList fl = front_hubs(g);
+    const int32_t *ftiles = fl.ctl ? g->front->d_tiles : nullptr;
+    prof_begin_class(g, "hub_tile", B_HUB, 8.0 * hub_edges, &pl);
     // tiles [t0, t1): the pipeline starts at t0 + blockIdx.x, stops at t1
     k_hub_tile<TT, E, false><<<grid_for(g, nt, 3), TT, 0, g->stream>>>(
         (const E *)w.off, w.nbr, prev, g->d_tile_hub, g->d_hub_tile0, g->d_hub_vid, g->d_hub_nparts,
         g->d_tile_idx_off, w.t0, w.t1, g->d_out_key, g->d_out_ent, g->d_tile_idx, g->d_stop,
-        g->d_err, sel, nsel, sel ? g->learn->d_hub_hd : nullptr, nhd);
+        g->d_err, sel, nsel, sel ? g->learn->d_hub_hd : nullptr, nhd, fl, ftiles);
     if (sel)   // learned dispatch: the hubs predicted high-distinct
         k_hub_tile<TT, E, true><<<grid_for(g, nt, 3), TT, 0, g->stream>>>(
             (const E *)w.off, w.nbr, prev, g->d_tile_hub, g->d_hub_tile0, g->d_hub_vid, g->d_hub_nparts,
             g->d_tile_idx_off, w.t0, w.t1, g->d_out_key, g->d_out_ent, g->d_tile_idx, g->d_stop,
-            g->d_err, sel, nsel, g->learn->d_hub_hd, nhd);
+            g->d_err, sel, nsel, g->learn->d_hub_hd, nhd, fl, ftiles);
     prof_end(g, &pl);
     prof_begin(g, "hub_merge", 0.0, &pl);
     k_hub_merge_small<<<grid_for(g, (ni + kHmSmallT / kWave - 1) / (kHmSmallT / kWave), 8), kHmSmallT, 0,
                         g->stream>>>(g->d_item_meta, w.i0, ni, g->d_tile_idx, g->d_out_key, g->d_out_ent,
-                                     g->d_hub_best, sel, hdist, nsel, g->d_merge_big, g->d_stop);
+                                     g->d_hub_best, sel, hdist, nsel, g->d_merge_big, g->d_stop, fl);
     k_hub_merge<TM, LIST><<<grid_for(g, ni, TM == 256 || !LIST ? 3 : 2), TM, 0, g->stream>>>(
         g->d_item_meta, w.i0, ni, g->d_merge_big, g->d_tile_idx, g->d_out_key, g->d_out_ent, g->d_hub_best,
-        g->d_stop, g->d_err, hdist, nsel);
+        g->d_stop, g->d_err, hdist, nsel, fl);
     prof_end(g, &pl);
     prof_begin(g, "hub_final", (double)sizeof(E) * 2.0 * (double)nh + 16.0 * (double)nh, &pl);
     k_hub_final<E><<<grid_for(g, (nh + 255) / 256, 4), 256, 0, g->stream>>>(
         (const E *)w.off, w.nbr, g->d_hub_vid + w.h0, nh, g->d_hub_best + w.h0, sel ? sel + w.h0 : nullptr,
         hdist ? hdist + w.h0 : nullptr, distinct_out(g), prev, next, g->d_counter,
-        g->d_stop, nsel);
+        g->d_stop, nsel, fl);
     prof_end(g, &pl);
 }
 
@@ -1174,7 +1209,7 @@ int launch_hash_iteration_incore(galp_graph *g) {
 
 int launch_iter_end(galp_graph *g) {
     k_iter_end<<<1, kCountShards, 0, g->stream>>>(g->d_counter, g->d_stop, g->d_iter_counts, g->d_iters_done,
-                                       g->iter % kMaxIters, (double)g->n * 1e-5);
+                                       g->iter % kMaxIters, (double)g->n * 1e-5, front_ctl(g));
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(g->ctx, GALP_EHIP, std::string("iter_end launch: ") + hipGetErrorString(e));
     return GALP_OK;

@@ -80,6 +80,17 @@ struct SortGroupResolve {
     }
 };
 
+// The rows a kernel walks: its whole class, or the frontier's list of those
+// that can still change.
+__device__ __forceinline__ void take_front(const FrontList &front, const int32_t *__restrict__ &vlist, int64_t &v0,
+                                           int64_t &nv) {
+    if (front_lists_on(front)) {
+        vlist = front.list;
+        v0 = 0;
+        nv = *front.len;
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Rows of the smaller classes (65..1024): one block of T threads per vertex,
 // a bitonic network in LDS (fewer, cheaper steps than radix passes at these
@@ -187,11 +198,13 @@ template <int T, int EPT, typename E>
 __global__ void __launch_bounds__(T)
 k_sort_bitonic(const E *__restrict__ off, const int32_t *__restrict__ nbr, const int32_t *__restrict__ prev,
            int32_t *__restrict__ next, const int32_t *__restrict__ vlist, int64_t v0, int64_t nv,
-           unsigned long long *__restrict__ counter, const int32_t *__restrict__ stop, int32_t *__restrict__ err) {
+           unsigned long long *__restrict__ counter, const int32_t *__restrict__ stop, int32_t *__restrict__ err,
+           FrontList front) {
     __shared__ unsigned long long skey[T * EPT];
     __shared__ unsigned long long sred64[T / kWave];
     __shared__ uint32_t sred[T / kWave];
     if (*stop) return;
+    take_front(front, vlist, v0, nv);
     LdsBitonicPolicy<T, EPT, E> pol{off, prev, next, vlist, v0, nv, skey, sred64, err, 0u};
     pipelined<T, EPT>(pol, nbr, prev, (int64_t)blockIdx.x, (int64_t)gridDim.x, (int)threadIdx.x);
     __syncthreads();
@@ -391,7 +404,8 @@ template <int NW, int EPT, typename E>
 __global__ void __launch_bounds__(NW * kWave)
 k_sort_reg(const E *__restrict__ off, const int32_t *__restrict__ nbr, const int32_t *__restrict__ prev,
            int32_t *__restrict__ next, const int32_t *__restrict__ vlist, int64_t v0, int64_t nv,
-           unsigned long long *__restrict__ counter, const int32_t *__restrict__ stop, int32_t *__restrict__ err) {
+           unsigned long long *__restrict__ counter, const int32_t *__restrict__ stop, int32_t *__restrict__ err,
+           FrontList front) {
     constexpr int T = NW * kWave;
     __shared__ unsigned long long sx[NW > 1 ? T * EPT : 1];
     __shared__ uint32_t sedge[2 * T];
@@ -399,6 +413,7 @@ k_sort_reg(const E *__restrict__ off, const int32_t *__restrict__ nbr, const int
     __shared__ unsigned long long sred64[NW];
     __shared__ uint32_t sred[NW];
     if (*stop) return;
+    take_front(front, vlist, v0, nv);
     RegBitonicPolicy<NW, EPT, E> pol{off, prev, next, vlist, v0, nv, sx, sedge, sw, sred64, err, 0u};
     pipelined<T, EPT>(pol, nbr, prev, (int64_t)blockIdx.x, (int64_t)gridDim.x, (int)threadIdx.x);
     if constexpr (NW > 1) __syncthreads();
@@ -629,7 +644,7 @@ __global__ void __launch_bounds__(T)
 k_sort_lds(const E *__restrict__ off, const int32_t *__restrict__ nbr, const int32_t *__restrict__ prev,
            int32_t *__restrict__ next, const int32_t *__restrict__ vlist, int64_t v0, int64_t nv,
            unsigned long long *__restrict__ counter, const int32_t *__restrict__ stop, int32_t *__restrict__ err,
-           int passes) {
+           int passes, FrontList front) {
     static_assert(T * EPT <= 65536, "positions are 16-bit");
     static_assert((T * EPT / (T / kWave)) % kWave == 0, "whole chunks per wave");
     __shared__ uint32_t skey[2 * T * EPT];
@@ -638,6 +653,7 @@ k_sort_lds(const E *__restrict__ off, const int32_t *__restrict__ nbr, const int
     __shared__ unsigned long long sred64[T / kWave];
     __shared__ uint32_t sred[T / kWave];
     if (*stop) return;
+    take_front(front, vlist, v0, nv);
     LdsSortPolicy<T, EPT, E> pol{off, prev, next, vlist, v0, nv, skey, spos, whist, sred64, err, passes, 0u};
     pipelined<T, EPT>(pol, nbr, prev, (int64_t)blockIdx.x, (int64_t)gridDim.x, (int)threadIdx.x);
     __syncthreads();
@@ -728,14 +744,20 @@ k_hs_tile_wave(const E *__restrict__ off, const int32_t *__restrict__ nbr, const
                const int32_t *__restrict__ hub_vid, const int32_t *__restrict__ hub_nparts,
                const int64_t *__restrict__ tile_idx_off, int64_t tbase, int64_t ntiles,
                uint32_t *__restrict__ out_key, uint32_t *__restrict__ out_ent, int32_t *__restrict__ tile_idx,
-               const int32_t *__restrict__ stop) {
+               const int32_t *__restrict__ stop, FrontList front, const int32_t *__restrict__ front_tiles) {
     constexpr int EPT = kHsWaveEPT;
     constexpr int NW = kHsWaveT / kWave;
     static_assert(kHubMaxParts <= (1 << 12) && kHubTile == (1 << 11), "key layout: 12 + 31 + 11 bits");
     if (*stop) return;
+    const bool lists = front_lists_on(front);   // only the tiles of the hubs that can still change
+    if (lists) {
+        tbase = 0;
+        ntiles = *front.len;
+    }
     const int lane = lane_id();
     const int64_t wid = (int64_t)blockIdx.x * NW + threadIdx.x / kWave;
-    for (int64_t t = tbase + wid; t < ntiles; t += (int64_t)gridDim.x * NW) {
+    for (int64_t i = tbase + wid; i < ntiles; i += (int64_t)gridDim.x * NW) {
+        const int64_t t = lists ? front_tiles[i] : i;
         const int h = tile_hub[t];
         const int64_t v = hub_vid[h];
         const int64_t rb = (int64_t)off[v], re = (int64_t)off[v + 1];
@@ -964,15 +986,21 @@ k_hs_merge_small(const int32_t *__restrict__ item_hub, const int32_t *__restrict
                  const int64_t *__restrict__ tile_idx_off, const int32_t *__restrict__ tile_idx,
                  const uint32_t *__restrict__ out_key, const uint32_t *__restrict__ out_ent,
                  unsigned long long *__restrict__ hub_best, int32_t *__restrict__ big,
-                 const int32_t *__restrict__ stop) {
+                 const int32_t *__restrict__ stop, FrontList front) {
     constexpr int NW = kHsSmallT / kWave;
     __shared__ HsWaveLds sw[NW];
     if (*stop) return;
+    const bool lists = front_lists_on(front);
+    if (lists && *front.len == 0) return;
     const int lane = lane_id();
     HsWaveLds &w = sw[threadIdx.x / kWave];
     const int64_t wid = (int64_t)blockIdx.x * NW + threadIdx.x / kWave;
     for (int64_t it = ibase + wid; it < ibase + nitems; it += (int64_t)gridDim.x * NW) {
         const int h = item_hub[it];
+        if (lists && !front.list[h]) {   // uniform per wave; the block merge skips it too
+            if (lane == 0) big[it] = 0;
+            continue;
+        }
         const int p = item_part[it];
         const int64_t t0 = hub_tile0[h], nt = hub_ntiles[h];
         int total = 0;
@@ -1038,7 +1066,7 @@ k_hs_merge(const int32_t *__restrict__ item_hub, const int32_t *__restrict__ ite
            const int64_t *__restrict__ tile_idx_off, const int32_t *__restrict__ tile_idx,
            const uint32_t *__restrict__ out_key, const uint32_t *__restrict__ out_ent,
            unsigned long long *__restrict__ hub_best, const int32_t *__restrict__ stop, int32_t *__restrict__ err,
-           int passes) {
+           int passes, FrontList front) {
     constexpr int N = kHsMergeCap;
     __shared__ uint32_t skey[2 * N];
     __shared__ uint16_t spos[2 * N];
@@ -1049,7 +1077,7 @@ k_hs_merge(const int32_t *__restrict__ item_hub, const int32_t *__restrict__ ite
     __shared__ int stotal, snruns;
     __shared__ unsigned long long sred64[T / kWave];
     __shared__ uint32_t sbig[T / 32];   // flags of the current chunk of items
-    if (*stop) return;
+    if (*stop || (front_lists_on(front) && *front.len == 0)) return;
     const int tid = (int)threadIdx.x;
     // the flagged items of each chunk of T of the block's items, gathered
     // into an LDS bit mask (one flag load per thread instead of a dependent
@@ -1163,13 +1191,16 @@ template <typename E>
 __global__ void __launch_bounds__(256)
 k_hs_final(const E *__restrict__ off, const int32_t *__restrict__ nbr, const int32_t *__restrict__ hub_vid,
            int64_t nhubs, unsigned long long *__restrict__ hub_best, const int32_t *__restrict__ prev,
-           int32_t *__restrict__ next, unsigned long long *__restrict__ counter, const int32_t *__restrict__ stop) {
+           int32_t *__restrict__ next, unsigned long long *__restrict__ counter, const int32_t *__restrict__ stop,
+           FrontList front) {
     __shared__ uint32_t sred[4];
     if (*stop) return;
+    const bool lists = front_lists_on(front);
+    if (lists && *front.len == 0) return;
     uint32_t changed = 0;
     for (int64_t base = (int64_t)blockIdx.x * 256; base < nhubs; base += (int64_t)gridDim.x * 256) {
         const int64_t h = base + threadIdx.x;
-        if (h < nhubs) {
+        if (h < nhubs && (!lists || front.list[h])) {
             const int64_t v = hub_vid[h];
             const unsigned long long b = hub_best[h];
             hub_best[h] = 0ull;
@@ -1232,17 +1263,20 @@ static void sort_group(galp_graph *g, const IterView &w, int bid, const int32_t 
     const BucketRange &r = w.cls[bid];
     if (!r.nv) return;
     PendingLaunch pl;
-    prof_begin(g, kBucketName[bid], class_bytes<E>(r), &pl);
+    prof_begin_class(g, kBucketName[bid], bid, class_bytes<E>(r), &pl);
+    const FrontList fl = front_list(g, bid);
     const int64_t per_block = 256 / G;
     const int64_t blocks = (r.nv + per_block - 1) / per_block;
     if (g->d_vlist)
         k_group<G, SortGroupResolve, SortGroupResolve, true, E><<<grid_for(g, blocks, blocks_per_cu), 256, 0,
                                                                   g->stream>>>(
-            (const E *)w.off, w.nbr, prev, next, g->d_vlist, r.v0, r.nv, nullptr, g->d_counter, g->d_stop, nullptr, 0);
+            (const E *)w.off, w.nbr, prev, next, g->d_vlist, r.v0, r.nv, nullptr, g->d_counter, g->d_stop, nullptr, 0,
+            fl);
     else
         k_group<G, SortGroupResolve, SortGroupResolve, false, E><<<grid_for(g, blocks, blocks_per_cu), 256, 0,
                                                                    g->stream>>>(
-            (const E *)w.off, w.nbr, prev, next, nullptr, r.v0, r.nv, nullptr, g->d_counter, g->d_stop, nullptr, 0);
+            (const E *)w.off, w.nbr, prev, next, nullptr, r.v0, r.nv, nullptr, g->d_counter, g->d_stop, nullptr, 0,
+            fl);
     prof_end(g, &pl);
 }
 
@@ -1253,14 +1287,15 @@ static void sort_lds(galp_graph *g, const IterView &w, int bid, const int32_t *p
     const BucketRange &r = w.cls[bid];
     if (!r.nv) return;
     PendingLaunch pl;
-    prof_begin(g, kBucketName[bid], class_bytes<E>(r), &pl);
+    prof_begin_class(g, kBucketName[bid], bid, class_bytes<E>(r), &pl);
+    const FrontList fl = front_list(g, bid);
     if constexpr (RADIX)
         k_sort_lds<T, EPT, E><<<grid_for(g, r.nv, blocks_per_cu), T, 0, g->stream>>>(
             (const E *)w.off, w.nbr, prev, next, g->d_vlist, r.v0, r.nv, g->d_counter, g->d_stop, g->d_err,
-            g->sort->passes);
+            g->sort->passes, fl);
     else
         k_sort_bitonic<T, EPT, E><<<grid_for(g, r.nv, blocks_per_cu), T, 0, g->stream>>>(
-            (const E *)w.off, w.nbr, prev, next, g->d_vlist, r.v0, r.nv, g->d_counter, g->d_stop, g->d_err);
+            (const E *)w.off, w.nbr, prev, next, g->d_vlist, r.v0, r.nv, g->d_counter, g->d_stop, g->d_err, fl);
     prof_end(g, &pl);
 }
 
@@ -1270,9 +1305,10 @@ static void sort_reg(galp_graph *g, const IterView &w, int bid, const int32_t *p
     const BucketRange &r = w.cls[bid];
     if (!r.nv) return;
     PendingLaunch pl;
-    prof_begin(g, kBucketName[bid], class_bytes<E>(r), &pl);
+    prof_begin_class(g, kBucketName[bid], bid, class_bytes<E>(r), &pl);
+    const FrontList fl = front_list(g, bid);
     k_sort_reg<NW, EPT, E><<<grid_for(g, r.nv, blocks_per_cu), NW * kWave, 0, g->stream>>>(
-        (const E *)w.off, w.nbr, prev, next, g->d_vlist, r.v0, r.nv, g->d_counter, g->d_stop, g->d_err);
+        (const E *)w.off, w.nbr, prev, next, g->d_vlist, r.v0, r.nv, g->d_counter, g->d_stop, g->d_err, fl);
     prof_end(g, &pl);
 }
 
@@ -1286,21 +1322,22 @@ static int sort_hubs(galp_graph *g, const IterView &w, const int32_t *prev, int3
     double hub_edges = 0.0;
     if (w.h0 == 0 && w.h1 == g->nhubs) hub_edges = (double)g->bucket[B_HUB].edges;
     PendingLaunch pl;
-    prof_begin(g, "hub_sort", 8.0 * hub_edges, &pl);
+    const FrontList fl = front_hubs(g);
+    prof_begin_class(g, "hub_sort", B_HUB, 8.0 * hub_edges, &pl);
     k_hs_tile_wave<E><<<grid_for(g, (nt + kHsWaveT / kWave - 1) / (kHsWaveT / kWave), tile_per_cu), kHsWaveT, 0,
                         g->stream>>>((const E *)w.off, w.nbr, prev, g->d_tile_hub, g->d_hub_tile0, g->d_hub_vid,
                                      g->d_hub_nparts, g->d_tile_idx_off, w.t0, w.t1, g->d_out_key, g->d_out_ent,
-                                     g->d_tile_idx, g->d_stop);
+                                     g->d_tile_idx, g->d_stop, fl, fl.ctl ? g->front->d_tiles : nullptr);
     const SortState *S = g->sort;
     k_hs_merge_small<<<grid_for(g, (ni + kHsSmallT / kWave - 1) / (kHsSmallT / kWave), 3), kHsSmallT, 0,
                        g->stream>>>(g->d_item_hub, g->d_item_part, w.i0, ni, g->d_hub_tile0, g->d_hub_ntiles,
                                     g->d_tile_idx_off, g->d_tile_idx, g->d_out_key, g->d_out_ent, g->d_hub_best,
-                                    g->d_merge_big, g->d_stop);
+                                    g->d_merge_big, g->d_stop, fl);
     k_hs_merge<kHsMergeT><<<grid_for(g, ni, merge_per_cu), kHsMergeT, 0, g->stream>>>(
         g->d_item_hub, g->d_item_part, w.i0, ni, g->d_merge_big, g->d_hub_tile0, g->d_hub_ntiles, g->d_tile_idx_off,
-        g->d_tile_idx, g->d_out_key, g->d_out_ent, g->d_hub_best, g->d_stop, g->d_err, S->passes);
+        g->d_tile_idx, g->d_out_key, g->d_out_ent, g->d_hub_best, g->d_stop, g->d_err, S->passes, fl);
     k_hs_final<E><<<grid_for(g, (nh + 255) / 256, 4), 256, 0, g->stream>>>(
-        (const E *)w.off, w.nbr, g->d_hub_vid + w.h0, nh, g->d_hub_best + w.h0, prev, next, g->d_counter, g->d_stop);
+        (const E *)w.off, w.nbr, g->d_hub_vid + w.h0, nh, g->d_hub_best + w.h0, prev, next, g->d_counter, g->d_stop, fl);
     prof_end(g, &pl);
     return GALP_OK;
 }

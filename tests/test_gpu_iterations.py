@@ -1,7 +1,8 @@
 """Iterations that do not run the class kernels over every row: the closed
-form of the first iteration (rows without repeated neighbours).  Every
-iteration is compared with the oracle; labels and counts are whole numbers,
-so they are equal or wrong."""
+form of the first iteration (rows without repeated neighbours) and the later
+iterations over the rows with a changed neighbour (symmetric graphs of at
+least 2^23 edges).  Every iteration is compared with the oracle; labels and
+counts are whole numbers, so they are equal or wrong."""
 import numpy as np
 import pytest
 
@@ -75,3 +76,115 @@ def test_first_iteration_logs_distinct_counts(ctx):
     assert len(y) == big.sum() and np.all(x[:, 3] == -1.0)
     got = np.sort(np.rint(np.exp2(y.astype(np.float64)) - 1).astype(np.int64))
     assert np.array_equal(got, np.sort(np.diff(off)[big]))
+
+
+@pytest.fixture(scope="module")
+def settling():
+    """A symmetric graph of at least 2^23 edges that settles within a dozen
+    iterations, with rows of every class: communities of 400 vertices, and
+    vertices of degree 1..9000 joined to whole communities' members, in two
+    copies that share no edge."""
+    rng = np.random.default_rng(5)
+    n, comm = 190000, 400
+    u = np.repeat(np.arange(n), 12)
+    v = u // comm * comm + rng.integers(0, comm, size=len(u))
+    keep = u % comm >= 8   # eight vertices of each community draw nothing: short rows
+    u, v = u[keep], v[keep]
+    v = np.where(v % comm < 8, v + 8, v)
+    pairs = [np.stack([u, v], 1), rng.integers(0, n, size=(20000, 2))]
+    for k, d in enumerate([66, 130, 260, 520, 1030, 2050, 4096, 4097, 9000, 6000]):
+        others = rng.choice(n, size=d, replace=False)
+        pairs.append(np.stack([np.full(d, 7 + 397 * k), others], 1))
+    e = np.concatenate(pairs)
+    e = e[e[:, 0] != e[:, 1]]
+    key = np.unique(np.concatenate([e[:, 0] * n + e[:, 1], e[:, 1] * n + e[:, 0]]))
+    off = np.searchsorted(key // n, np.arange(n + 1)).astype(np.int64)
+    nbr = (key % n).astype(np.int32)
+    off = np.concatenate([off, off[1:] + off[-1], [2 * off[-1]]])   # and one vertex without edges
+    nbr = np.concatenate([nbr, nbr + np.int32(n)])
+    assert len(nbr) >= 1 << 23
+    refs, prev = [], np.arange(2 * n + 1, dtype=np.int32)
+    for _ in range(12):
+        prev, cnt = oracle.lp_iterate(off, nbr, prev)
+        refs.append((prev, cnt))
+    return off, nbr, refs
+
+
+VARIANTS = [dict(), dict(reorder=0), dict(method=_abi.METHOD_SORT), dict(method=_abi.METHOD_SORT, reorder=0),
+            dict(offsets64=1), dict(profile=1)]
+
+
+@pytest.mark.parametrize("opts", VARIANTS, ids=["hash", "hash-noreorder", "sort", "sort-noreorder", "off64", "profile"])
+def test_changed_rows_only(ctx, settling, opts):
+    off, nbr, refs = settling
+    print(f"[lists] {opts} m={len(nbr)}", flush=True)
+    with _abi.Graph(ctx, off, nbr, **opts) as g:
+        g.init()
+        for it, (ref, cnt) in enumerate(refs):
+            st = g.step()
+            assert st["updated"] == cnt, it + 1
+            assert np.array_equal(g.labels(), ref), it + 1
+        if opts.get("profile"):   # the class kernels' bytes show that the lists were walked
+            prof = {k["name"]: k for k in g.profile()}
+            assert prof["front"]["launches"] >= 9
+            full = sum(g.info()["bucket_edges"]) * 8.0 * (len(refs) - 1)
+            assert 0 < sum(k["alg_bytes"] for nm, k in prof.items() if nm != "first") < 0.8 * full
+        # any other state: the lists start over
+        lab = refs[-1][0].copy()
+        lab[::9773] = np.arange(len(lab))[::9773]
+        g.set_labels(lab)
+        for it in range(3):
+            lab, cnt = oracle.lp_iterate(off, nbr, lab)
+            assert g.step()["updated"] == cnt, it
+            assert np.array_equal(g.labels(), lab), it
+
+
+@pytest.mark.parametrize("capture", [0, 1])
+def test_changed_rows_only_device_loop(ctx, settling, capture):
+    off, nbr, refs = settling
+    stop = next((i for i, (_, c) in enumerate(refs) if c <= (len(off) - 1) * 1e-5), len(refs) - 1)
+    with _abi.Graph(ctx, off, nbr, graph_capture=capture) as g, _abi.Graph(ctx, off, nbr) as other:
+        for rep in range(3):
+            labels, res = g.run(len(refs))
+            assert res["iterations"] == stop + 1, rep
+            assert np.array_equal(labels, refs[stop][0]), rep
+            other.run(3)   # eager work between the replays
+
+
+def test_one_way_edges_take_every_row(ctx, settling):
+    """Without the reverse of one edge the lists would miss a row."""
+    off, nbr, _ = settling
+    e = int(off[100])
+    off2 = off.copy()
+    off2[101:] -= 1
+    nbr2 = np.delete(nbr, e)
+    with _abi.Graph(ctx, off2, nbr2, profile=1) as g:
+        g.init()
+        check_steps(g, off2, nbr2, 8)
+        assert "front" not in {k["name"] for k in g.profile()}
+
+
+@pytest.mark.parametrize("net", ["all-cand", "rand"])
+def test_changed_rows_only_learned(ctx, settling, net):
+    off, nbr, refs = settling
+    params = np.zeros(_abi.mlp_num_params(8), np.float32) if net == "all-cand" else _abi.mlp_init(8, 3)
+    with _abi.Graph(ctx, off, nbr, dispatch=_abi.DISPATCH_LEARNED) as g:
+        g.set_mlp(8, params, 6.0)
+        g.init()
+        for it, (ref, cnt) in enumerate(refs):
+            assert g.step()["updated"] == cnt, it + 1
+            assert np.array_equal(g.labels(), ref), it + 1
+
+
+@pytest.mark.parametrize("method", [_abi.METHOD_HASH, _abi.METHOD_SORT])
+def test_changed_rows_only_batch(ctx, settling, method):
+    """The two copies as two graphs of a batch: each stops by its own rule."""
+    off, nbr, refs = settling
+    n = (len(off) - 2) // 2
+    final, per, counts = oracle.lp_run(off[:n + 1], nbr[:off[n]], niter=12)
+    with _abi.Graph(ctx, off, nbr, method=method, reorder=0) as g:
+        g.set_batch([0, n, 2 * n + 1])
+        labels, _ = g.run(12)
+        iters = g.batch_iterations()
+    assert iters[0] == len(counts)
+    assert np.array_equal(labels[:n], final) and np.array_equal(labels[n:2 * n] - n, final)
