@@ -13,14 +13,18 @@ namespace galp {
 // winner is the label of lane `last`.
 // One wave holds 64/G vertices per round; rounds are software-pipelined:
 // while round t is resolved, the labels of round t+1 and the neighbour ids
-// of round t+2 are loading, and the offsets of round t+3.
+// of round t+2 are loading, the offsets of round t+3 and, from a vertex list,
+// the ids of round t+4 (an id loaded with the offsets that need it is the
+// youngest load in flight, and waiting for it drains all the others).  This
+// block is number bi of the nb that share the class.
 template <int G, class Resolve, bool VLIST, typename E>
 __device__ __forceinline__ uint32_t group_rounds(const E *__restrict__ off, const int32_t *__restrict__ nbr,
                                                  const int32_t *__restrict__ prev, int32_t *__restrict__ next,
-                                                 const int32_t *__restrict__ vlist, int64_t v0, int64_t nv) {
+                                                 const int32_t *__restrict__ vlist, int64_t v0, int64_t nv,
+                                                 int64_t bi, int64_t nb) {
     const int p = lane_id() & (G - 1);
     constexpr int64_t per_block = 256 / G;
-    const int64_t stride = (int64_t)gridDim.x * per_block;
+    const int64_t stride = nb * per_block;
     // Raw offsets stay in the pipeline registers until the next stage uses
     // them (any arithmetic on a just-loaded value would wait for it), and
     // every load is issued by every lane from a clamped address, so no load
@@ -30,12 +34,12 @@ __device__ __forceinline__ uint32_t group_rounds(const E *__restrict__ off, cons
         E ob, oe;     // off[v], off[v+1], raw
         bool ok;      // i < nv
     };
-    auto state = [&](int64_t i) {
+    auto ident = [&](int64_t i) -> int32_t { return VLIST ? vlist[v0 + (i < nv ? i : 0)] : 0; };
+    auto state = [&](int64_t i, int32_t id) {   // id: ident(i)
         St s;
         s.ok = i < nv;
-        const int64_t ic = s.ok ? i : 0;
-        if constexpr (VLIST) s.v = (int64_t)vlist[v0 + ic];
-        else s.v = v0 + ic;
+        if constexpr (VLIST) s.v = (int64_t)id;
+        else s.v = v0 + (s.ok ? i : 0);
         s.ob = off[s.v];
         s.oe = off[s.v + 1];
         return s;
@@ -55,12 +59,14 @@ __device__ __forceinline__ uint32_t group_rounds(const E *__restrict__ off, cons
             changed += (L != old);
         }
     };
-    int64_t base = (int64_t)blockIdx.x * per_block;   // uniform round index
+    int64_t base = bi * per_block;                    // uniform round index
     int64_t i = base + threadIdx.x / G;               // this lane's vertex index
     // Four state slots rotate through the stages; the loop is unrolled by
     // the rotation period so no register holding an in-flight load is ever
     // copied (a copy would wait for it).
-    St sa = state(i), sb = state(i + stride), sc = state(i + 2 * stride), sd;
+    const int32_t ia = ident(i), ib = ident(i + stride), ic = ident(i + 2 * stride);
+    int32_t id = ident(i + 3 * stride);
+    St sa = state(i, ia), sb = state(i + stride, ib), sc = state(i + 2 * stride, ic), sd;
     int32_t u = ldn(sa);
     int32_t LA = gat(u, sa), oA = prev[sa.v], LB, oB;
     u = ldn(sb);
@@ -68,7 +74,8 @@ __device__ __forceinline__ uint32_t group_rounds(const E *__restrict__ off, cons
     LN = gat(u, S1);                                     \
     ON = prev[S1.v];                                     \
     u = ldn(S2);                                         \
-    S3 = state(i + 3 * stride);                          \
+    S3 = state(i + 3 * stride, id);                      \
+    id = ident(i + 4 * stride);                          \
     resolve(S0, LC, OC);                                 \
     i += stride;                                         \
     base += stride;                                      \
@@ -101,14 +108,16 @@ k_group(const E *__restrict__ off, const int32_t *__restrict__ nbr,
     if (front_lists_on(front)) {   // uniform
         nv = *front.len;
         if ((int64_t)blockIdx.x * (256 / G) >= nv) return;
-        const uint32_t ch = group_rounds<G, Resolve, true, E>(off, nbr, prev, next, front.list, 0, nv);
+        const uint32_t ch = group_rounds<G, Resolve, true, E>(off, nbr, prev, next, front.list, 0, nv,
+                                                                   (int64_t)blockIdx.x, (int64_t)gridDim.x);
         block_count_add<4>(ch, counter, scratch);
         return;
     }
     if (nv_dev) nv = *nv_dev;
     const bool alt = hd_count && 2 * (*hd_count) > hd_total;   // uniform
-    const uint32_t changed = alt ? group_rounds<G, Alt, VLIST, E>(off, nbr, prev, next, vlist, v0, nv)
-                                 : group_rounds<G, Resolve, VLIST, E>(off, nbr, prev, next, vlist, v0, nv);
+    const int64_t bi = blockIdx.x, nb = gridDim.x;
+    const uint32_t changed = alt ? group_rounds<G, Alt, VLIST, E>(off, nbr, prev, next, vlist, v0, nv, bi, nb)
+                                 : group_rounds<G, Resolve, VLIST, E>(off, nbr, prev, next, vlist, v0, nv, bi, nb);
     block_count_add<4>(changed, counter, scratch);
 }
 

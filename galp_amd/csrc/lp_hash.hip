@@ -48,11 +48,15 @@ const char *const kBucketName[NUM_BUCKETS] = {"g4",   "g8",   "g16",  "g32",  "g
 //          label's count (popcount) and last position (highest set bit), so
 //          the labels of a converged neighbourhood are settled in a round
 //          each, whatever the order;
-//   sweep: lanes still unresolved (a group with more than PEEL distinct
-//          labels) count the lanes of their group holding their label; the
-//          max over those lanes of (count << 8 | lane) is the max over their
-//          labels of (count << 8 | last), since a label's highest lane is its
-//          last position.
+//          Rounds stop after one that settles less than a quarter of the
+//          wave's open lanes: the labels are diverse, and the sweep costs
+//          the same however many lanes it finds;
+//   sweep: lanes still unresolved count the lanes of their group holding
+//          their label (at G = 64 by splitting a lane mask bit by bit,
+//          match_lanes; below by comparing over lane moves); the max over
+//          those lanes of (count << 8 | lane) is the max over their labels of
+//          (count << 8 | last), since a label's highest lane is its last
+//          position.
 // A peeled label takes all of its lanes with it, so the sweep's counts
 // among unresolved lanes are full counts.  The result is the same for every
 // lane of the group.
@@ -85,15 +89,14 @@ __device__ __forceinline__ uint32_t group_best(int32_t L) {
         }
         best = any ? max(best, (cnt << 8) | last) : best;
         active = active && !eq;
+        if (4 * __popcll(b) < __popcll(ball)) break;   // few repeats: the sweep resolves the rest at once
     }
-    if (__ballot(active)) {
-        const int32_t La = active ? L : -1;
+    if (const unsigned long long left = __ballot(active)) {
         uint32_t cnt = 0;
         if constexpr (G == kWave) {
-#pragma unroll
-            for (int j = 0; j < kWave; ++j) cnt += (uint32_t)(__builtin_amdgcn_readlane(La, j) == La);
+            cnt = (uint32_t)__popcll(match_lanes(L, left));
         } else {
-            cnt = group_count_eq<G>(La);
+            cnt = group_count_eq<G>(active ? L : -1);
         }
         best = max(best, group_max<G>(active ? ((cnt << 8) | (uint32_t)(lane & (G - 1))) : 0u));
     }

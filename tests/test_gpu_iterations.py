@@ -78,6 +78,26 @@ def test_first_iteration_logs_distinct_counts(ctx):
     assert np.array_equal(got, np.sort(np.diff(off)[big]))
 
 
+@pytest.mark.parametrize("distinct", [1, 2, 3, 17, 63, 5000])
+def test_lane_group_rows(ctx, distinct):
+    """Rows of 1..64 edges over labels of `distinct` values, the lowest and
+    the highest vertex id among them: every mix of settled and diverse rows."""
+    rng = np.random.default_rng(distinct)
+    n = 6007
+    rows = [rng.integers(0, n, size=v % 65).tolist() for v in range(n)]
+    off, nbr = csr(rows)
+    values = np.unique(np.concatenate([[0, n - 1], rng.integers(0, n, size=distinct)]))[:max(distinct, 1)]
+    lab = values[rng.integers(0, len(values), size=n)].astype(np.int32)
+    lab[:n // 2:3] = values[0]   # some rows mostly one label
+    for opts in (dict(), dict(reorder=0), dict(method=_abi.METHOD_SORT)):
+        print(f"[groups] distinct={distinct} {opts}", flush=True)
+        with _abi.Graph(ctx, off, nbr, **opts) as g:
+            g.set_labels(lab)
+            ref, cnt = oracle.lp_iterate(off, nbr, lab)
+            assert g.step()["updated"] == cnt
+            assert np.array_equal(g.labels(), ref)
+
+
 @pytest.fixture(scope="module")
 def settling():
     """A symmetric graph of at least 2^23 edges that settles within a dozen
