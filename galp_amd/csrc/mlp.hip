@@ -275,6 +275,287 @@ k_mlp_train(float *__restrict__ params, const float *__restrict__ x, const float
     }
 }
 
+// The same training run for H = 32 on the matrix units, bit for bit: an fp32
+// MFMA adds its products to the accumulator in order of k, each by a fused
+// multiply-add, which is what the sums of k_mlp_train compile to.  That
+// kernel waits on LDS (two reads per multiply-add in the sums over samples:
+// 82 us a minibatch of 512); here a minibatch takes MFMA_US us.
+// A chunk of 256 samples has two phases:
+//  forward and backward (waves 0..3, one per SIMD, 64 samples each as two
+//  32-sample tiles whose chains interleave): the layers are computed
+//  transposed, Z^T = W * H^T, with samples across the lanes, 32x32x2 MFMAs.
+//  An accumulator then holds, for a lane's sample, the units 8p + 4 half + q
+//  (half: lane / 32), and the next layer's operand wants units 2s | 2s + 1 in
+//  the lanes' halves: v_permlane32_swap of neighbouring registers gives it,
+//  so activations go from layer to layer in registers.  The output unit's
+//  sum runs over the units in order with both tiles' samples in one register
+//  (64 lanes), by plain multiply-adds;
+//  gradients: activations and deltas lie in LDS, transposed (unit-major), the
+//  samples of each 16 permuted so that one 16-byte read feeds a lane's four
+//  16x16x4 MFMAs.  dW2 is four 16x16 tiles (waves 0..3); dW1 and db1 are
+//  columns 0..3 and 4 of two tiles, the fourth operand row being ones (waves
+//  6, 7); dW3, db2 and db3 are sums by lane (wave 4).  The accumulators stay
+//  in registers over the chunks of a minibatch.
+// Padding samples hold zero deltas and activations, which add nothing.
+constexpr int kTmChunk = 256;
+constexpr int kTmPitch = kTmChunk + 8;   // 4 rows apart: the other 32 banks
+constexpr int kTmW2Pitch = 33;
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// a = (a.low half, b.low half), b = (a.high half, b.high half)
+__device__ __forceinline__ void swap_halves(float &a, float &b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
+
+// The next layer's operands from a 32x32 accumulator (units of the lanes'
+// samples): op[s] holds unit 2s in the low lanes, 2s + 1 in the high ones.
+__device__ __forceinline__ void units_to_operands(const float (&h)[16], float (&op)[16]) {
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+        float a = h[4 * p], b = h[4 * p + 1], c = h[4 * p + 2], d = h[4 * p + 3];
+        swap_halves(a, b);
+        swap_halves(c, d);
+        op[4 * p] = a;
+        op[4 * p + 1] = c;
+        op[4 * p + 2] = b;
+        op[4 * p + 3] = d;
+    }
+}
+
+__global__ void __launch_bounds__(kTrainThreads)
+k_mlp_train_mfma(float *__restrict__ params, const float *__restrict__ x, const float *__restrict__ y, int64_t n,
+                 int epochs, int B, float lr, float b1, float b2, float eps) {
+    constexpr int H = 32;
+    constexpr int P = mlp_num_params(H);
+    constexpr int Q = (P + kTrainThreads - 1) / kTrainThreads;   // parameters per thread
+    constexpr int kW2 = 5 * H, kB2 = kW2 + H * H;                // offsets in the parameter vector
+    // parameters in LDS: W1, b1 as they lie, W2 in rows of 33, then b2, W3, b3
+    constexpr int kLW2 = 5 * H, kLB2 = kLW2 + H * kTmW2Pitch, kLW3 = kLB2 + H, kLB3 = kLW3 + H;
+    __shared__ __align__(16) float sh1[H * kTmPitch], sh2[H * kTmPitch], sd1[H * kTmPitch], sd2[H * kTmPitch];
+    __shared__ __align__(16) float sx[6 * kTmPitch];   // the four inputs, ones, zeros
+    __shared__ __align__(16) float sg[kTmPitch];
+    __shared__ float sp[kLB3 + 1];
+    __shared__ float sgrad[P];
+    const int t = threadIdx.x, lane = lane_id();
+    const int w = __builtin_amdgcn_readfirstlane(t / kWave);
+    const int col = lane & 31, half = lane >> 5;
+    auto lds_of = [](int q) {
+        if (q < kW2) return q;
+        if (q < kB2) return kLW2 + (q - kW2) / H * kTmW2Pitch + (q - kW2) % H;
+        return q - kB2 + kLB2;
+    };
+    auto place = [](int i) { return (i & ~15) | ((i & 3) << 2) | ((i >> 2) & 3); };   // sample i of a chunk
+    float pm[Q], pv[Q], pw[Q];
+#pragma unroll
+    for (int r = 0; r < Q; ++r) {
+        const int q = t + r * kTrainThreads;
+        pm[r] = 0.f;
+        pv[r] = 0.f;
+        pw[r] = q < P ? params[q] : 0.f;
+        if (q < P) sp[lds_of(q)] = pw[r];
+    }
+    for (int i = t; i < kTmPitch; i += kTrainThreads) {
+        sx[4 * kTmPitch + i] = 1.f;
+        sx[5 * kTmPitch + i] = 0.f;
+    }
+    __syncthreads();
+    const float scale = 1.0f / (float)B;
+    float pow1 = 1.f, pow2 = 1.f;   // b1^step, b2^step
+    // this lane's samples of a chunk: one per tile for the layers, one for the output
+    float4 xn[2];
+    float yn = 0.f;
+    auto load = [&](int64_t off, int c0) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int i = w * 64 + u * 32 + col;
+            xn[u] = c0 + i < B ? ((const float4 *)x)[off + c0 + i] : float4{0.f, 0.f, 0.f, 0.f};
+        }
+        const int i = w * 64 + lane;
+        yn = c0 + i < B ? y[off + c0 + i] : 0.f;
+    };
+    if (w < 4 && epochs > 0 && B <= n) load(0, 0);
+    for (int e = 0; e < epochs; ++e) {
+        for (int64_t off = 0; off + B <= n; off += B) {
+            f32x4 acc = {0.f, 0.f, 0.f, 0.f};   // this wave's gradient tile
+            float acc_v = 0.f, acc_b3 = 0.f;    // wave 4: dW3 or db2 of this lane, db3
+            for (int c0 = 0; c0 < B; c0 += kTmChunk) {
+                const int cs = min(kTmChunk, B - c0);
+                const int blocks = (cs + 15) / 16;
+                if (w < 4 && w * 64 < 16 * blocks) {
+                    const int base = w * 64;
+                    float z1[2][16], h1[2][16], z2[2][16], h2[2][16];
+                    bool ok[2];
+                    int at[2];
+                    f32x16 c[2];
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        ok[u] = base + 32 * u + col < cs;
+                        at[u] = place(base + 32 * u + col);
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) c[u][r] = sp[4 * H + 8 * (r >> 2) + 4 * half + (r & 3)];
+                    }
+                    {
+                        const float a0 = sp[4 * col + half], a1 = sp[4 * col + 2 + half];
+#pragma unroll
+                        for (int u = 0; u < 2; ++u)
+                            c[u] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, half ? xn[u].y : xn[u].x, c[u], 0, 0, 0);
+#pragma unroll
+                        for (int u = 0; u < 2; ++u)
+                            c[u] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, half ? xn[u].w : xn[u].z, c[u], 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        // the inputs, for dW1: each half of the lanes stores two of the four
+                        sx[(2 * half) * kTmPitch + at[u]] = half ? xn[u].z : xn[u].x;
+                        sx[(2 * half + 1) * kTmPitch + at[u]] = half ? xn[u].w : xn[u].y;
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) {
+                            z1[u][r] = c[u][r];
+                            h1[u][r] = z1[u][r] > 0.f ? z1[u][r] : 0.f;
+                            sh1[(8 * (r >> 2) + 4 * half + (r & 3)) * kTmPitch + at[u]] = ok[u] ? h1[u][r] : 0.f;
+                            c[u][r] = sp[kLB2 + 8 * (r >> 2) + 4 * half + (r & 3)];
+                        }
+                    }
+                    float op[2][16];
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) units_to_operands(h1[u], op[u]);
+#pragma unroll
+                    for (int s = 0; s < 16; ++s) {
+                        const float a = sp[kLW2 + col * kTmW2Pitch + 2 * s + half];
+#pragma unroll
+                        for (int u = 0; u < 2; ++u)
+                            c[u] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, op[u][s], c[u], 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) {
+                            z2[u][r] = c[u][r];
+                            h2[u][r] = z2[u][r] > 0.f ? z2[u][r] : 0.f;
+                            sh2[(8 * (r >> 2) + 4 * half + (r & 3)) * kTmPitch + at[u]] = ok[u] ? h2[u][r] : 0.f;
+                        }
+                        units_to_operands(h2[u], op[u]);
+                    }
+                    float out = sp[kLB3];   // lanes 0..31: tile 0's samples, 32..63: tile 1's
+#pragma unroll
+                    for (int s = 0; s < 16; ++s) {
+                        float a = op[0][s], b = op[1][s];
+                        swap_halves(a, b);   // unit 2s, unit 2s + 1 of this lane's sample
+                        out += sp[kLW3 + 2 * s] * a;
+                        out += sp[kLW3 + 2 * s + 1] * b;
+                    }
+                    float g0 = base + lane < cs ? (out - yn) * scale : 0.f;
+                    sg[place(base + lane)] = g0;
+                    float g1 = g0;
+                    swap_halves(g0, g1);   // tile 0's and tile 1's deltas in both halves
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        float d2[16];
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) {
+                            const int row = 8 * (r >> 2) + 4 * half + (r & 3);
+                            d2[r] = z2[u][r] > 0.f ? (u ? g1 : g0) * sp[kLW3 + row] : 0.f;
+                            sd2[row * kTmPitch + at[u]] = d2[r];
+                            c[u][r] = 0.f;
+                        }
+                        units_to_operands(d2, op[u]);
+                    }
+#pragma unroll
+                    for (int s = 0; s < 16; ++s) {
+                        const float a = sp[kLW2 + (2 * s + half) * kTmW2Pitch + col];
+#pragma unroll
+                        for (int u = 0; u < 2; ++u)
+                            c[u] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, op[u][s], c[u], 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int u = 0; u < 2; ++u)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r)
+                            sd1[(8 * (r >> 2) + 4 * half + (r & 3)) * kTmPitch + at[u]] =
+                                z1[u][r] > 0.f ? c[u][r] : 0.f;
+                }
+                if (w < 4) {   // the next chunk's samples load behind the gradients
+                    int cn = c0 + kTmChunk;
+                    int64_t on = off;
+                    if (cn >= B) {
+                        cn = 0;
+                        on = off + 2 * (int64_t)B <= n ? off + B : 0;
+                    }
+                    load(on, cn);
+                }
+                __syncthreads();
+                if (w < 4 || w >= 6) {
+                    const int m = lane & 15, k4 = 4 * (lane >> 4);
+                    const float *pa = w < 4 ? sd2 + ((w >> 1) * 16 + m) * kTmPitch : sd1 + ((w - 6) * 16 + m) * kTmPitch;
+                    const float *pb = w < 4 ? sh1 + ((w & 1) * 16 + m) * kTmPitch : sx + min(m, 5) * kTmPitch;
+#pragma unroll 2
+                    for (int b = 0; b < blocks; ++b) {
+                        const f32x4 a = *(const f32x4 *)(pa + b * 16 + k4), v = *(const f32x4 *)(pb + b * 16 + k4);
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q], v[q], acc, 0, 0, 0);
+                    }
+                } else if (w == 4) {
+                    const float *pv2 = (half ? sd2 : sh2) + col * kTmPitch;
+                    for (int b = 0; b < blocks; ++b) {
+                        f32x4 v[4], g[4];
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            v[q] = *(const f32x4 *)(pv2 + b * 16 + 4 * q);
+                            g[q] = *(const f32x4 *)(sg + b * 16 + 4 * q);
+                        }
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) {   // sample i lies in word i / 4 of its quarter
+                            const float gi = g[i & 3][i >> 2], vi = v[i & 3][i >> 2];
+                            acc_v = __builtin_fmaf(half ? 1.f : gi, vi, acc_v);
+                            acc_b3 += gi;
+                        }
+                    }
+                }
+                __syncthreads();   // the chunk's rows are rewritten next
+            }
+            if (w < 4) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    sgrad[kW2 + ((w >> 1) * 16 + 4 * (lane >> 4) + r) * H + (w & 1) * 16 + (lane & 15)] = acc[r];
+            } else if (w >= 6) {
+                const int m = lane & 15;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int j = (w - 6) * 16 + 4 * (lane >> 4) + r;
+                    if (m < 4) sgrad[4 * j + m] = acc[r];
+                    else if (m == 4) sgrad[4 * H + j] = acc[r];
+                }
+            } else if (w == 4) {
+                sgrad[(half ? kB2 : kB2 + H) + col] = acc_v;
+                if (lane == 0) sgrad[P - 1] = acc_b3;
+            }
+            __syncthreads();
+            pow1 *= b1;
+            pow2 *= b2;
+            const float c1 = 1.f - pow1, c2 = 1.f - pow2;
+#pragma unroll
+            for (int r = 0; r < Q; ++r) {
+                const int q = t + r * kTrainThreads;
+                const float g = q < P ? sgrad[q] : 0.f;
+                pm[r] = b1 * pm[r] + (1.f - b1) * g;
+                pv[r] = b2 * pv[r] + (1.f - b2) * g * g;
+                pw[r] -= lr * (pm[r] / c1) / (sqrtf(pv[r] / c2) + eps);
+                if (q < P) sp[lds_of(q)] = pw[r];
+            }
+            __syncthreads();
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < Q; ++r) {
+        const int q = t + r * kTrainThreads;
+        if (q < P) params[q] = pw[r];
+    }
+}
+
 template <int H>
 static int mlp_grad_launch(hipStream_t st, const float *dp, const float *dx, const float *dy, int64_t n,
                            float *dpgrad, float *dploss, float *dgrad, float *dloss) {
@@ -304,7 +585,7 @@ static int mlp_train_dev(hipStream_t st, int H, float *dp, const float *dx, cons
     switch (H) {
     case 8: k_mlp_train<8><<<1, kTrainThreads, 0, st>>>(dp, dx, dy, n, epochs, B, lr, b1, b2, eps); break;
     case 16: k_mlp_train<16><<<1, kTrainThreads, 0, st>>>(dp, dx, dy, n, epochs, B, lr, b1, b2, eps); break;
-    case 32: k_mlp_train<32><<<1, kTrainThreads, 0, st>>>(dp, dx, dy, n, epochs, B, lr, b1, b2, eps); break;
+    case 32: k_mlp_train_mfma<<<1, kTrainThreads, 0, st>>>(dp, dx, dy, n, epochs, B, lr, b1, b2, eps); break;
     default: return GALP_EINVAL;
     }
     return hipGetLastError() == hipSuccess ? GALP_OK : GALP_EHIP;
