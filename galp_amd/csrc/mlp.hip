@@ -279,17 +279,17 @@ k_mlp_train(float *__restrict__ params, const float *__restrict__ x, const float
 // MFMA adds its products to the accumulator in order of k, each by a fused
 // multiply-add, which is what the sums of k_mlp_train compile to.  That
 // kernel waits on LDS (two reads per multiply-add in the sums over samples:
-// 82 us a minibatch of 512); here a minibatch takes MFMA_US us.
+// 82 us a minibatch of 512); here a minibatch takes 15 us, of which the
+// busiest SIMD's MFMAs are 7.
 // A chunk of 256 samples has two phases:
-//  forward and backward (waves 0..3, one per SIMD, 64 samples each as two
-//  32-sample tiles whose chains interleave): the layers are computed
+//  forward and backward (32 samples a wave, two waves per SIMD so that one's
+//  vector and LDS work runs behind the other's MFMAs): the layers are computed
 //  transposed, Z^T = W * H^T, with samples across the lanes, 32x32x2 MFMAs.
 //  An accumulator then holds, for a lane's sample, the units 8p + 4 half + q
 //  (half: lane / 32), and the next layer's operand wants units 2s | 2s + 1 in
 //  the lanes' halves: v_permlane32_swap of neighbouring registers gives it,
 //  so activations go from layer to layer in registers.  The output unit's
-//  sum runs over the units in order with both tiles' samples in one register
-//  (64 lanes), by plain multiply-adds;
+//  sum runs over the units in order by plain multiply-adds in both halves;
 //  gradients: activations and deltas lie in LDS, transposed (unit-major), the
 //  samples of each 16 permuted so that one 16-byte read feeds a lane's four
 //  16x16x4 MFMAs.  dW2 is four 16x16 tiles (waves 0..3); dW1 and db1 are
@@ -365,120 +365,94 @@ k_mlp_train_mfma(float *__restrict__ params, const float *__restrict__ x, const 
     __syncthreads();
     const float scale = 1.0f / (float)B;
     float pow1 = 1.f, pow2 = 1.f;   // b1^step, b2^step
-    // this lane's samples of a chunk: one per tile for the layers, one for the output
-    float4 xn[2];
+    // waves w and w + 4 share a SIMD: the first takes the matrix unit when both
+    // want it, so that the other's vector work falls beside it
+    if (w < 4) __builtin_amdgcn_s_setprio(1);
+    // this lane's sample of a chunk (both halves of the wave hold the same 32)
+    float4 xn{0.f, 0.f, 0.f, 0.f};
     float yn = 0.f;
+    const int mine = w * 32 + col, at = place(mine);
     auto load = [&](int64_t off, int c0) {
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int i = w * 64 + u * 32 + col;
-            xn[u] = c0 + i < B ? ((const float4 *)x)[off + c0 + i] : float4{0.f, 0.f, 0.f, 0.f};
-        }
-        const int i = w * 64 + lane;
-        yn = c0 + i < B ? y[off + c0 + i] : 0.f;
+        const bool in = c0 + mine < B;
+        const int64_t i = off + (in ? c0 + mine : 0);
+        xn = ((const float4 *)x)[i];
+        yn = y[i];
+        if (!in) xn = float4{0.f, 0.f, 0.f, 0.f};
     };
-    if (w < 4 && epochs > 0 && B <= n) load(0, 0);
+    if (epochs > 0 && B <= n) load(0, 0);
     for (int e = 0; e < epochs; ++e) {
         for (int64_t off = 0; off + B <= n; off += B) {
             f32x4 acc = {0.f, 0.f, 0.f, 0.f};   // this wave's gradient tile
             float acc_v = 0.f, acc_b3 = 0.f;    // wave 4: dW3 or db2 of this lane, db3
+            // this minibatch's parameters in the layouts of the MFMAs
+            float rb1[16], rb2[16], rw3[16], rw2[16], rw2t[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int row = 8 * (r >> 2) + 4 * half + (r & 3);
+                rb1[r] = sp[4 * H + row];
+                rb2[r] = sp[kLB2 + row];
+                rw3[r] = sp[kLW3 + row];
+                rw2[r] = sp[kLW2 + col * kTmW2Pitch + 2 * r + half];
+                rw2t[r] = sp[kLW2 + (2 * r + half) * kTmW2Pitch + col];
+            }
+            const float rw1a = sp[4 * col + half], rw1b = sp[4 * col + 2 + half];
             for (int c0 = 0; c0 < B; c0 += kTmChunk) {
                 const int cs = min(kTmChunk, B - c0);
                 const int blocks = (cs + 15) / 16;
-                if (w < 4 && w * 64 < 16 * blocks) {
-                    const int base = w * 64;
-                    float z1[2][16], h1[2][16], z2[2][16], h2[2][16];
-                    bool ok[2];
-                    int at[2];
-                    f32x16 c[2];
+                if (w * 32 < 16 * blocks) {
+                    const bool ok = mine < cs;
+                    float h1[16], h2[16], op[16];
+                    f32x16 c;
 #pragma unroll
-                    for (int u = 0; u < 2; ++u) {
-                        ok[u] = base + 32 * u + col < cs;
-                        at[u] = place(base + 32 * u + col);
+                    for (int r = 0; r < 16; ++r) c[r] = rb1[r];
+                    c = __builtin_amdgcn_mfma_f32_32x32x2f32(rw1a, half ? xn.y : xn.x, c, 0, 0, 0);
+                    c = __builtin_amdgcn_mfma_f32_32x32x2f32(rw1b, half ? xn.w : xn.z, c, 0, 0, 0);
+                    // the inputs, for dW1: each half of the lanes stores two of the four
+                    sx[(2 * half) * kTmPitch + at] = half ? xn.z : xn.x;
+                    sx[(2 * half + 1) * kTmPitch + at] = half ? xn.w : xn.y;
 #pragma unroll
-                        for (int r = 0; r < 16; ++r) c[u][r] = sp[4 * H + 8 * (r >> 2) + 4 * half + (r & 3)];
+                    for (int r = 0; r < 16; ++r) {
+                        h1[r] = c[r] > 0.f ? c[r] : 0.f;
+                        sh1[(8 * (r >> 2) + 4 * half + (r & 3)) * kTmPitch + at] = ok ? h1[r] : 0.f;
+                        c[r] = rb2[r];
                     }
-                    {
-                        const float a0 = sp[4 * col + half], a1 = sp[4 * col + 2 + half];
+                    units_to_operands(h1, op);
 #pragma unroll
-                        for (int u = 0; u < 2; ++u)
-                            c[u] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, half ? xn[u].y : xn[u].x, c[u], 0, 0, 0);
+                    for (int s = 0; s < 16; ++s)
+                        c = __builtin_amdgcn_mfma_f32_32x32x2f32(rw2[s], op[s], c, 0, 0, 0);
 #pragma unroll
-                        for (int u = 0; u < 2; ++u)
-                            c[u] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, half ? xn[u].w : xn[u].z, c[u], 0, 0, 0);
+                    for (int r = 0; r < 16; ++r) {
+                        h2[r] = c[r] > 0.f ? c[r] : 0.f;
+                        sh2[(8 * (r >> 2) + 4 * half + (r & 3)) * kTmPitch + at] = ok ? h2[r] : 0.f;
                     }
-#pragma unroll
-                    for (int u = 0; u < 2; ++u) {
-                        // the inputs, for dW1: each half of the lanes stores two of the four
-                        sx[(2 * half) * kTmPitch + at[u]] = half ? xn[u].z : xn[u].x;
-                        sx[(2 * half + 1) * kTmPitch + at[u]] = half ? xn[u].w : xn[u].y;
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) {
-                            z1[u][r] = c[u][r];
-                            h1[u][r] = z1[u][r] > 0.f ? z1[u][r] : 0.f;
-                            sh1[(8 * (r >> 2) + 4 * half + (r & 3)) * kTmPitch + at[u]] = ok[u] ? h1[u][r] : 0.f;
-                            c[u][r] = sp[kLB2 + 8 * (r >> 2) + 4 * half + (r & 3)];
-                        }
-                    }
-                    float op[2][16];
-#pragma unroll
-                    for (int u = 0; u < 2; ++u) units_to_operands(h1[u], op[u]);
+                    units_to_operands(h2, op);
+                    float out = sp[kLB3];
 #pragma unroll
                     for (int s = 0; s < 16; ++s) {
-                        const float a = sp[kLW2 + col * kTmW2Pitch + 2 * s + half];
-#pragma unroll
-                        for (int u = 0; u < 2; ++u)
-                            c[u] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, op[u][s], c[u], 0, 0, 0);
-                    }
-#pragma unroll
-                    for (int u = 0; u < 2; ++u) {
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) {
-                            z2[u][r] = c[u][r];
-                            h2[u][r] = z2[u][r] > 0.f ? z2[u][r] : 0.f;
-                            sh2[(8 * (r >> 2) + 4 * half + (r & 3)) * kTmPitch + at[u]] = ok[u] ? h2[u][r] : 0.f;
-                        }
-                        units_to_operands(h2[u], op[u]);
-                    }
-                    float out = sp[kLB3];   // lanes 0..31: tile 0's samples, 32..63: tile 1's
-#pragma unroll
-                    for (int s = 0; s < 16; ++s) {
-                        float a = op[0][s], b = op[1][s];
-                        swap_halves(a, b);   // unit 2s, unit 2s + 1 of this lane's sample
+                        float a = op[s], b = op[s];
+                        swap_halves(a, b);   // units 2s and 2s + 1 in both halves
                         out += sp[kLW3 + 2 * s] * a;
                         out += sp[kLW3 + 2 * s + 1] * b;
                     }
-                    float g0 = base + lane < cs ? (out - yn) * scale : 0.f;
-                    sg[place(base + lane)] = g0;
-                    float g1 = g0;
-                    swap_halves(g0, g1);   // tile 0's and tile 1's deltas in both halves
+                    const float g = ok ? (out - yn) * scale : 0.f;
+                    sg[at] = g;
+                    float d2[16];
 #pragma unroll
-                    for (int u = 0; u < 2; ++u) {
-                        float d2[16];
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) {
-                            const int row = 8 * (r >> 2) + 4 * half + (r & 3);
-                            d2[r] = z2[u][r] > 0.f ? (u ? g1 : g0) * sp[kLW3 + row] : 0.f;
-                            sd2[row * kTmPitch + at[u]] = d2[r];
-                            c[u][r] = 0.f;
-                        }
-                        units_to_operands(d2, op[u]);
+                    for (int r = 0; r < 16; ++r) {
+                        const int row = 8 * (r >> 2) + 4 * half + (r & 3);
+                        d2[r] = h2[r] > 0.f ? g * rw3[r] : 0.f;
+                        sd2[row * kTmPitch + at] = d2[r];
+                        c[r] = 0.f;
                     }
+                    units_to_operands(d2, op);
 #pragma unroll
-                    for (int s = 0; s < 16; ++s) {
-                        const float a = sp[kLW2 + (2 * s + half) * kTmW2Pitch + col];
+                    for (int s = 0; s < 16; ++s)
+                        c = __builtin_amdgcn_mfma_f32_32x32x2f32(rw2t[s], op[s], c, 0, 0, 0);
 #pragma unroll
-                        for (int u = 0; u < 2; ++u)
-                            c[u] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, op[u][s], c[u], 0, 0, 0);
-                    }
-#pragma unroll
-                    for (int u = 0; u < 2; ++u)
-#pragma unroll
-                        for (int r = 0; r < 16; ++r)
-                            sd1[(8 * (r >> 2) + 4 * half + (r & 3)) * kTmPitch + at[u]] =
-                                z1[u][r] > 0.f ? c[u][r] : 0.f;
+                    for (int r = 0; r < 16; ++r)
+                        sd1[(8 * (r >> 2) + 4 * half + (r & 3)) * kTmPitch + at] = h1[r] > 0.f ? c[r] : 0.f;
                 }
-                if (w < 4) {   // the next chunk's samples load behind the gradients
+                {   // the next chunk's samples load behind the gradients
                     int cn = c0 + kTmChunk;
                     int64_t on = off;
                     if (cn >= B) {
@@ -488,30 +462,46 @@ k_mlp_train_mfma(float *__restrict__ params, const float *__restrict__ x, const 
                     load(on, cn);
                 }
                 __syncthreads();
+                // gradients, each block's operands read one block ahead
                 if (w < 4 || w >= 6) {
                     const int m = lane & 15, k4 = 4 * (lane >> 4);
-                    const float *pa = w < 4 ? sd2 + ((w >> 1) * 16 + m) * kTmPitch : sd1 + ((w - 6) * 16 + m) * kTmPitch;
-                    const float *pb = w < 4 ? sh1 + ((w & 1) * 16 + m) * kTmPitch : sx + min(m, 5) * kTmPitch;
-#pragma unroll 2
+                    const float *pa = (w < 4 ? sd2 + ((w >> 1) * 16 + m) * kTmPitch : sd1 + ((w - 6) * 16 + m) * kTmPitch) + k4;
+                    const float *pb = (w < 4 ? sh1 + ((w & 1) * 16 + m) * kTmPitch : sx + min(m, 5) * kTmPitch) + k4;
+                    f32x4 a = *(const f32x4 *)pa, v = *(const f32x4 *)pb;
                     for (int b = 0; b < blocks; ++b) {
-                        const f32x4 a = *(const f32x4 *)(pa + b * 16 + k4), v = *(const f32x4 *)(pb + b * 16 + k4);
+                        const int nx = b + 1 < blocks ? (b + 1) * 16 : 0;
+                        const f32x4 an = *(const f32x4 *)(pa + nx), vn = *(const f32x4 *)(pb + nx);
 #pragma unroll
                         for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q], v[q], acc, 0, 0, 0);
+                        a = an;
+                        v = vn;
                     }
                 } else if (w == 4) {
                     const float *pv2 = (half ? sd2 : sh2) + col * kTmPitch;
+                    f32x4 v[4], g[4];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        v[q] = *(const f32x4 *)(pv2 + 4 * q);
+                        g[q] = *(const f32x4 *)(sg + 4 * q);
+                    }
                     for (int b = 0; b < blocks; ++b) {
-                        f32x4 v[4], g[4];
+                        const int nx = b + 1 < blocks ? (b + 1) * 16 : 0;
+                        f32x4 vn[4], gn[4];
 #pragma unroll
                         for (int q = 0; q < 4; ++q) {
-                            v[q] = *(const f32x4 *)(pv2 + b * 16 + 4 * q);
-                            g[q] = *(const f32x4 *)(sg + b * 16 + 4 * q);
+                            vn[q] = *(const f32x4 *)(pv2 + nx + 4 * q);
+                            gn[q] = *(const f32x4 *)(sg + nx + 4 * q);
                         }
 #pragma unroll
                         for (int i = 0; i < 16; ++i) {   // sample i lies in word i / 4 of its quarter
                             const float gi = g[i & 3][i >> 2], vi = v[i & 3][i >> 2];
                             acc_v = __builtin_fmaf(half ? 1.f : gi, vi, acc_v);
                             acc_b3 += gi;
+                        }
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            v[q] = vn[q];
+                            g[q] = gn[q];
                         }
                     }
                 }
