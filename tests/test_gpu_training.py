@@ -59,7 +59,7 @@ def test_train_matches_host(ctx, n, batch, epochs):
     p0 = _abi.mlp_init(H, n)
     got, _ = _abi.mlp_train(ctx, H, p0, x, y, epochs=epochs, batch=batch, lr=1e-3, seed=3)
     want = train_host(p0, x, y, epochs, batch, 1e-3, 3)
-    # at most 6 Adam steps of at most lr * (1 + small) each: a sign of a
+    # Adam steps of at most lr * (1 + small) each: a sign of a
     # near-zero gradient may differ in single precision, which moves a
     # parameter by up to 2 lr a step; anything but a few such parameters is
     # within float32's accumulation error of a step
