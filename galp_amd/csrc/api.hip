@@ -494,6 +494,11 @@ IterView full_view(const galp_graph *g) {
     return w;
 }
 
+bool fused_rows(const galp_graph *g) {
+    return !g->ooc && !g->prof.on && !g->class_kernels && g->m < kFusedMaxEdges &&
+           (g->opts.method == GALP_METHOD_HASH ? g->opts.variant == 1 : g->opts.policy == GALP_POLICY_INCORE);
+}
+
 bool concurrent_allowed(const galp_graph *g) {
     return !g->ooc && !g->prof.on && g->side[0] && g->side[1] && g->opts.variant != 0 &&
            g->opts.policy != GALP_POLICY_LI;

@@ -136,6 +136,7 @@ GALP_API int galp_graph_set_tuning(galp_graph *g, const int32_t *options) {
     for (int b = 0; b < NUM_BUCKETS; ++b)
         if (options[b] < 0 || options[b] >= kTuneOptions) return fail(g->ctx, GALP_EINVAL, "tuning option out of range");
     for (int b = 0; b < NUM_BUCKETS; ++b) g->tune[b] = (int8_t)options[b];
+    g->class_kernels = true;
     invalidate_captured(g);
     return GALP_OK;
 }

@@ -366,6 +366,7 @@ struct galp_graph {
     galp::BatchState *batch = nullptr;
     galp::FrontState *front = nullptr;
     int8_t tune[galp::NUM_BUCKETS] = {};   // kernel configuration per degree class (autotuner)
+    bool class_kernels = false;   // options set by hand: a kernel per class at every size
     int8_t streams = 0;   // in-core class kernels: 0 by size, 1 one stream, 3 three (the autotuner's choice)
     // learned dispatch in core: bit i set = iteration i routes by the network,
     // clear = by the degree classes alone (the judge's choice, autotune.hip);
@@ -427,6 +428,11 @@ int launch_iter_end(galp_graph *g);
 // the largest graph counts, not the batch.
 constexpr int64_t kConcurrentMinEdges = (int64_t)1 << 24;
 constexpr int64_t kConcurrentMaxVertices = (int64_t)1 << 25;
+// All row classes below B4K in one launch (rows_fused.hpp): in core, up to
+// kFusedMaxEdges edges, the default variants, unless single kernels are timed
+// or were chosen by hand (galp_graph_set_tuning).
+constexpr int64_t kFusedMaxEdges = (int64_t)1 << 25;
+bool fused_rows(const galp_graph *g);
 bool concurrent_allowed(const galp_graph *g);
 bool concurrent_classes(const galp_graph *g);
 // Launches made between side_begin(g, k) and side_end(g, k, s) go to side

@@ -28,6 +28,7 @@
 #include "internal.hpp"
 #include "pipeline.hpp"
 #include "group_kernel.hpp"
+#include "rows_fused.hpp"
 
 namespace galp {
 
@@ -171,7 +172,9 @@ __device__ __forceinline__ uint32_t lds_try_insert(uint32_t *skey, uint32_t L, b
 // insert one by one.  Returns the lane's slot; *own marks lanes that wrote
 // the slot (they reset it afterwards), *creator the one lane per table that
 // claimed it; *maxc tracks the largest count seen.
-template <int BITS, int PEEL, bool LAST>
+// ADAPT: a round is only committed when its label fills a quarter of the open
+// lanes; otherwise the labels are diverse and all lanes insert at once.
+template <int BITS, int PEEL, bool LAST, bool ADAPT = false>
 __device__ __forceinline__ uint32_t lds_insert_chunk(uint32_t *skey, uint32_t *scnt, uint32_t *slast,
                                                      int32_t L, uint32_t pos, bool *own,
                                                      bool *creator, uint32_t *maxc, int32_t *err) {
@@ -188,6 +191,7 @@ __device__ __forceinline__ uint32_t lds_insert_chunk(uint32_t *skey, uint32_t *s
         const int32_t Lk = __builtin_amdgcn_readlane(L, leader);
         const bool eq = active && (L == Lk);
         const unsigned long long m = __ballot(eq);
+        if (ADAPT && 4 * __popcll(m) < __popcll(ball)) break;   // uniform
         const uint32_t lastpos = LAST ? (uint32_t)__builtin_amdgcn_readlane((int)pos, 63 - __clzll((long long)m)) : 0u;
         uint32_t sl = 0;
         if (lane == leader) {
@@ -221,7 +225,19 @@ __device__ __forceinline__ uint32_t lds_insert_chunk(uint32_t *skey, uint32_t *s
 // Pass 2 keeps the largest position whose label has count C: that
 // position's label is argmax (count, last).  Each lane then resets the slots
 // it used, leaving the table empty for the next vertex.
-template <int T, int EPT, int CAPBITS, typename E, int PEEL>
+// A team is the T threads sharing a row: a block, or (T = 64) one wave of
+// any block, which then needs no barrier.
+template <int T>
+__device__ __forceinline__ void team_sync() {
+    if constexpr (T == kWave) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    } else {
+        __syncthreads();
+    }
+}
+
+template <int T, int EPT, int CAPBITS, typename E, int PEEL, bool ADAPT = false>
 struct LdsVertexPolicy {
     struct Item {
         bool valid;
@@ -239,6 +255,7 @@ struct LdsVertexPolicy {
     unsigned long long *sred64;
     int32_t *err;
     int32_t *distinct;   // if set: distinct labels per vertex (learned dispatch feature)
+    int tid;             // within the team
     uint32_t changed;
 
     __device__ Item item(int64_t i) const {
@@ -250,7 +267,7 @@ struct LdsVertexPolicy {
             it.old = prev[it.v];
             it.valid = true;
             if (it.len > T * EPT) {   // never planned into this class
-                if (threadIdx.x == 0) atomicOr(err, 8);
+                if (tid == 0) atomicOr(err, 8);
                 it.len = 0;
             }
         }
@@ -263,19 +280,19 @@ struct LdsVertexPolicy {
         uint32_t slot[EPT];
         bool own[EPT], creator[EPT];
         uint32_t maxc = 0;
-        __syncthreads();
+        team_sync<T>();
 #pragma unroll
         for (int k = 0; k < EPT; ++k) {
-            const int pos = k * T + (int)threadIdx.x;
-            slot[k] = lds_insert_chunk<CAPBITS, PEEL, false>(skey, scnt, nullptr, pos < it.len ? lab[k] : -1,
+            const int pos = k * T + tid;
+            slot[k] = lds_insert_chunk<CAPBITS, PEEL, false, ADAPT>(skey, scnt, nullptr, pos < it.len ? lab[k] : -1,
                                                           (uint32_t)pos, &own[k], &creator[k], &maxc, err);
         }
-        __syncthreads();
+        team_sync<T>();
         maxc = block_max<T / kWave>(maxc, sred);
         unsigned long long best = 0;
 #pragma unroll
         for (int k = 0; k < EPT; ++k) {
-            const int pos = k * T + (int)threadIdx.x;
+            const int pos = k * T + tid;
             if (pos < it.len && scnt[slot[k]] == maxc)
                 best = ((unsigned long long)(pos + 1) << 32) | (uint32_t)lab[k];
         }
@@ -293,7 +310,7 @@ struct LdsVertexPolicy {
                 scnt[slot[k]] = 0;
             }
         }
-        if (threadIdx.x == 0) {
+        if (tid == 0) {
             const int32_t w = (int32_t)(uint32_t)best;
             next[it.v] = w;
             changed += (w != it.old);
@@ -338,19 +355,99 @@ k_hash_lds(const E *__restrict__ off, const int32_t *__restrict__ nbr,
     uint32_t changed = 0;
     if ((int64_t)blockIdx.x < nv) {   // uniform per block
         LdsVertexPolicy<T, EPT, CAPBITS, E, PEEL_A> pol{off, prev, next, vlist, v0, nv, skey, scnt, sred, sred64,
-                                                        err, distinct, 0u};
+                                                        err, distinct, (int)threadIdx.x, 0u};
         pipelined<T, EPT>(pol, nbr, prev, (int64_t)blockIdx.x, (int64_t)gridDim.x, (int)threadIdx.x);
         changed += pol.changed;
     }
     if ((int64_t)blockIdx.x < nvB) {
         __syncthreads();
         LdsVertexPolicy<T, EPT, CAPBITS, E, 0> pol{off, prev, next, vlistB, 0, nvB, skey, scnt, sred, sred64, err,
-                                                   distinct, 0u};
+                                                   distinct, (int)threadIdx.x, 0u};
         pipelined<T, EPT>(pol, nbr, prev, (int64_t)blockIdx.x, (int64_t)gridDim.x, (int)threadIdx.x);
         changed += pol.changed;
     }
     __syncthreads();
     block_count_add<T / kWave>(changed, counter, sred);
+}
+
+// ---------------------------------------------------------------------------
+// All classes up to degree 2048 in one launch (rows_fused.hpp): the lane
+// groups, 65..512 with a wave and its own table per row (four per block),
+// 513..2048 with a block per row.  The resolver and the table kernels adapt to
+// diverse labels by themselves (peel rounds stop), so learned dispatch's two
+// lists of a class run the same code one after the other.
+constexpr int kHashRows = B_B2K + 1;
+template <int T, int EPT, int CAPBITS, typename E>
+__device__ __forceinline__ uint32_t fused_tables(const RowsWork &w, const E *off, const int32_t *nbr,
+                                                 const int32_t *prev, int32_t *next, uint32_t *tab, uint32_t *sred,
+                                                 unsigned long long *sred64, int32_t *err, int32_t *distinct) {
+    constexpr int TEAMS = kRowsThreads / T;   // 4 waves or the block
+    constexpr int CAP = 1 << CAPBITS;
+    const int team = TEAMS == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / T);
+    const int tid = TEAMS == 1 ? (int)threadIdx.x : lane_id();
+    uint32_t *skey = tab + team * 2 * CAP, *scnt = skey + CAP;
+    for (int s = tid; s < CAP; s += T) {
+        skey[s] = kEmpty;
+        scnt[s] = 0;
+    }
+    const int64_t first = w.bi * TEAMS + team, stride = w.nb * TEAMS;
+    uint32_t changed = 0;
+    for (int pass = 0; pass < 2; ++pass) {
+        const int32_t *vlist = pass ? w.r.vlistB : w.r.vlist;
+        if (pass && !vlist) break;
+        const int64_t nv = pass ? *w.r.nvB_dev : w.r.nv;
+        if (first >= nv) continue;
+        team_sync<T>();
+        LdsVertexPolicy<T, EPT, CAPBITS, E, 3, true> pol{off, prev, next, vlist, pass ? 0 : w.r.v0, nv, skey, scnt,
+                                                         sred, sred64, err, distinct, tid, 0u};
+        pipelined<T, EPT>(pol, nbr, prev, first, stride, tid);
+        changed += pol.changed;
+    }
+    return changed;
+}
+
+template <int G, typename E>
+__device__ __forceinline__ uint32_t fused_group(const RowsWork &w, const E *off, const int32_t *nbr,
+                                                const int32_t *prev, int32_t *next) {
+    if (w.bi * (kRowsThreads / G) >= w.r.nv) return 0;
+    if (w.r.vlist)
+        return group_rounds<G, HashGroupResolve, true, E>(off, nbr, prev, next, w.r.vlist, w.r.v0, w.r.nv, w.bi, w.nb);
+    return group_rounds<G, HashGroupResolve, false, E>(off, nbr, prev, next, nullptr, w.r.v0, w.r.nv, w.bi, w.nb);
+}
+
+template <typename E>
+__global__ void __launch_bounds__(kRowsThreads) __attribute__((amdgpu_waves_per_eu(kRowsPerCu)))
+k_hash_rows(RowsArgs<kHashRows> args, const E *__restrict__ off, const int32_t *__restrict__ nbr,
+            const int32_t *__restrict__ prev, int32_t *__restrict__ next, unsigned long long *__restrict__ counter,
+            const int32_t *__restrict__ stop, int32_t *__restrict__ err, int32_t *__restrict__ distinct) {
+    __shared__ uint32_t tab[2 << 12];   // keys and counts: 4 x 1024 slots or 4096
+    __shared__ uint32_t sred[kRowsWaves];
+    __shared__ unsigned long long sred64[kRowsWaves];
+    if (*stop) return;
+    const RowsWork w = rows_work(args);
+    if (w.cls < 0) return;
+    uint32_t changed = 0;
+    switch (w.cls) {   // uniform
+    case B_G4: changed = fused_group<4, E>(w, off, nbr, prev, next); break;
+    case B_G8: changed = fused_group<8, E>(w, off, nbr, prev, next); break;
+    case B_G16: changed = fused_group<16, E>(w, off, nbr, prev, next); break;
+    case B_G32: changed = fused_group<32, E>(w, off, nbr, prev, next); break;
+    case B_G64: changed = fused_group<64, E>(w, off, nbr, prev, next); break;
+    case B_W128:
+        changed = fused_tables<64, 2, 8, E>(w, off, nbr, prev, next, tab, sred, sred64, err, distinct);
+        break;
+    case B_W256:
+        changed = fused_tables<64, 4, 9, E>(w, off, nbr, prev, next, tab, sred, sred64, err, distinct);
+        break;
+    case B_W512:
+        changed = fused_tables<64, 8, 10, E>(w, off, nbr, prev, next, tab, sred, sred64, err, distinct);
+        break;
+    case B_B1K:
+        changed = fused_tables<256, 4, 11, E>(w, off, nbr, prev, next, tab, sred, sred64, err, distinct);
+        break;
+    default: changed = fused_tables<256, 8, 12, E>(w, off, nbr, prev, next, tab, sred, sred64, err, distinct);
+    }
+    block_count_add<kRowsWaves>(changed, counter, sred);
 }
 
 // ---------------------------------------------------------------------------
@@ -1131,6 +1228,36 @@ static void launch_class(galp_graph *g, const IterView &w, int b, const int32_t 
     }
 }
 
+// Classes G4..B2K of a view in one launch.
+template <typename E>
+static void launch_rows(galp_graph *g, const IterView &w, const int32_t *prev, int32_t *next) {
+    static const int kPerBlock[kHashRows] = {64, 32, 16, 8, 4, 4, 4, 4, 1, 1};
+    RowsArgs<kHashRows> a{};
+    a.front = front_list(g, B_G4);
+    const bool learned = learned_now(g);
+    for (int b = 0; b < kHashRows; ++b) {
+        const BucketRange &r = w.cls[b];
+        const FrontList fl = front_list(g, b);
+        RowsClass &c = a.c[b];
+        c = RowsClass{g->d_vlist, r.v0, r.nv, nullptr, nullptr, nullptr, fl.list, fl.len, 1.f, kPerBlock[b]};
+        if (batch_lists(g)) {
+            c.vlist = g->batch->d_alist[b];
+            c.v0 = 0;
+            c.nv_dev = g->batch->d_alen + b;
+        } else if (learned && b >= B_W128) {   // this iteration's two lists for the class
+            c.vlist = g->learn->plist[b];
+            c.v0 = 0;
+            c.nv_dev = g->learn->d_plist_n + b;
+            c.vlistB = g->learn->plist[NUM_BUCKETS + b];
+            c.nvB_dev = g->learn->d_plist_n + kCtrHd + b;
+        }
+    }
+    const int grid = rows_plan(g, w, a, B_W128);
+    if (!grid) return;
+    k_hash_rows<E><<<grid, kRowsThreads, 0, g->stream>>>(a, (const E *)w.off, w.nbr, prev, next, g->d_counter,
+                                                         g->d_stop, g->d_err, distinct_out(g));
+}
+
 int launch_hash_class(galp_graph *g, int b) {
     const IterView w = full_view(g);
     const int32_t *prev = g->d_lab[g->cur];
@@ -1146,6 +1273,13 @@ static int hash_iteration(galp_graph *g, const IterView &w) {
     const int32_t *prev = g->d_lab[g->cur];
     int32_t *next = g->d_lab[g->cur ^ 1];
     launch_class<E>(g, w, B_HUB, prev, next);   // largest work first
+    if (fused_rows(g)) {
+        launch_class<E>(g, w, B_B4K, prev, next);
+        launch_rows<E>(g, w, prev, next);
+        const hipError_t ef = hipGetLastError();
+        return ef == hipSuccess ? GALP_OK
+                                : fail(g->ctx, GALP_EHIP, std::string("hash kernel launch: ") + hipGetErrorString(ef));
+    }
     if (g->opts.variant == 0) {
         // -l 0: no degree classes below the hubs -- every row through the
         // block-per-vertex table kernel, as the reference's naive variant
@@ -1178,7 +1312,7 @@ template <typename E>
 static int hash_iteration_incore(galp_graph *g) {
     const IterView w = full_view(g);
     const bool learned = learned_now(g);
-    if (!concurrent_classes(g)) {
+    if (fused_rows(g) || !concurrent_classes(g)) {
         if (learned) {
             const int rc = launch_learned_front(g, true);
             if (rc != GALP_OK) return rc;
