@@ -8,6 +8,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace galp {
 
 constexpr int kWave = 64;
@@ -126,32 +128,55 @@ __device__ __forceinline__ uint32_t group_count_eq(int32_t x) {
     return c;
 }
 
+// Wave-wide reduction of 32-bit words for an operation with identity 0 (max
+// of unsigned, or); uniform result.  Row shifts and row broadcasts fold into
+// the operation's own instruction, one per step, where a butterfly needs a
+// move or two besides.
+template <class Op>
+__device__ __forceinline__ uint32_t wave_reduce_u32(uint32_t x, Op op) {
+    auto step = [&](auto ctrl, auto rows) {
+        x = op(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int32_t)x, decltype(ctrl)::value, decltype(rows)::value,
+                                                        0xF, false));
+    };
+    using all = std::integral_constant<int, 0xF>;
+    step(std::integral_constant<int, 0x111>{}, all{});   // row_shr 1, 2, 4, 8: a row's lane 15 holds its total
+    step(std::integral_constant<int, 0x112>{}, all{});
+    step(std::integral_constant<int, 0x114>{}, all{});
+    step(std::integral_constant<int, 0x118>{}, all{});
+    step(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xA>{});   // row_bcast 15 into rows 1, 3
+    step(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xC>{});   // row_bcast 31 into rows 2, 3
+    return (uint32_t)__builtin_amdgcn_readlane((int32_t)x, kWave - 1);
+}
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t x) {
+    return wave_reduce_u32(x, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
+}
+
 // Lanes of `among` (a wave mask that holds this lane) whose x equals this
 // lane's; meaningless in other lanes.  The mask is split by one ballot per
-// bit in which the lanes of `among` differ, four vector instructions a bit:
-// about 80 for 20-bit labels, where comparing against every lane's value in
-// turn takes 192.  With it (and unproductive peel rounds cut short) the
-// 33..64 class, which issue of these instructions bounds while labels are
-// diverse, took a 512-graph batch's run from 14.8 to 11.2 ms.
+// bit, four vector instructions a bit and hardly a scalar one, skipping the
+// groups of four bits in which the lanes of `among` agree: about 80 for
+// 20-bit labels, where comparing against every lane's value in turn takes
+// 192.  With it (and unproductive peel rounds cut short) the 33..64 class,
+// which issue of these instructions bounds while labels are diverse, took a
+// 512-graph batch's run from 14.8 to 11.2 ms.
 __device__ __forceinline__ unsigned long long match_lanes(int32_t x, unsigned long long among) {
     const int32_t first = __builtin_amdgcn_readlane(x, __ffsll((long long)among) - 1);
     const bool in = (among >> lane_id()) & 1ull;
-    int32_t d = in ? x ^ first : 0;
-    d |= lane_xor<1>(d);
-    d |= lane_xor<2>(d);
-    d |= lane_xor<4>(d);
-    d |= lane_xor<8>(d);
-    // one lane of each 16-lane row stands for the row
-    uint32_t vary = (uint32_t)(__builtin_amdgcn_readlane(d, 0) | __builtin_amdgcn_readlane(d, 16) |
-                               __builtin_amdgcn_readlane(d, 32) | __builtin_amdgcn_readlane(d, 48));
+    const uint32_t vary =
+        wave_reduce_u32(in ? (uint32_t)(x ^ first) : 0u, [](uint32_t a, uint32_t b) { return a | b; });
     uint32_t lo = (uint32_t)among, hi = (uint32_t)(among >> 32);
-    while (vary) {   // uniform
-        const int bit = __ffs((int)vary) - 1;
-        vary &= vary - 1u;
-        const int32_t m = (int32_t)((uint32_t)x << (31 - bit)) >> 31;   // the bit in every position
-        const unsigned long long b = __ballot(m != 0);
-        lo &= ~((uint32_t)b ^ (uint32_t)m);
-        hi &= ~((uint32_t)(b >> 32) ^ (uint32_t)m);
+#pragma unroll
+    for (int nib = 0; nib < 8; ++nib) {
+        if (!((vary >> (4 * nib)) & 15u)) continue;   // uniform
+#pragma unroll
+        for (int bit = 4 * nib; bit < 4 * nib + 4; ++bit) {
+            uint32_t m = (uint32_t)__builtin_amdgcn_sbfe(x, bit, 1);   // the bit in every position
+            asm("" : "+v"(m));   // else the compare is rebuilt from a shift of x, one instruction more
+            const unsigned long long b = __builtin_amdgcn_ballot_w64(m != 0u);
+            constexpr int kAndNotXor = 0x90;   // lo & ~(b ^ m)
+            lo = __builtin_amdgcn_bitop3_b32(lo, (uint32_t)b, m, kAndNotXor);
+            hi = __builtin_amdgcn_bitop3_b32(hi, (uint32_t)(b >> 32), m, kAndNotXor);
+        }
     }
     return ((unsigned long long)hi << 32) | lo;
 }

@@ -1,6 +1,8 @@
 // group_kernel.hpp -- the degree <= 64 driver shared by both LP methods.
 #pragma once
 
+#include <type_traits>
+
 #include "device_common.hpp"
 #include "internal.hpp"
 
@@ -18,7 +20,7 @@ namespace galp {
 // youngest load in flight, and waiting for it drains all the others).  This
 // block is number bi of the nb that share the class.
 template <int G, class Resolve, bool VLIST, typename E>
-__device__ __forceinline__ uint32_t group_rounds(const E *__restrict__ off, const int32_t *__restrict__ nbr,
+__device__ __forceinline__ uint32_t group_rounds_lanes(const E *__restrict__ off, const int32_t *__restrict__ nbr,
                                                  const int32_t *__restrict__ prev, int32_t *__restrict__ next,
                                                  const int32_t *__restrict__ vlist, int64_t v0, int64_t nv,
                                                  int64_t bi, int64_t nb) {
@@ -48,7 +50,7 @@ __device__ __forceinline__ uint32_t group_rounds(const E *__restrict__ off, cons
     auto ldn = [&](const St &s) -> int32_t {
         return __builtin_nontemporal_load(&nbr[has(s) ? (int64_t)s.ob + p : 0]);
     };
-    auto gat = [&](int32_t u, const St &s) -> int32_t { return prev[has(s) ? u : 0]; };
+    auto gat = [&](int32_t u, const St &s) -> int32_t { return prev[has(s) ? (uint32_t)u : 0u]; };
     uint32_t changed = 0;
     // the winner lane (best's low byte) holds the new label and writes it
     auto resolve = [&](const St &s, int32_t Lraw, int32_t old) {
@@ -88,6 +90,87 @@ __device__ __forceinline__ uint32_t group_rounds(const E *__restrict__ off, cons
     }
 #undef GALP_GROUP_STAGE
     return changed;
+}
+
+// Degree 33..64, a wave per row: the same pipeline with the row's offsets, old
+// label and list id loaded through the scalar cache into scalar registers,
+// since they are the same in all lanes.  A round issues three vector memory
+// instructions (ids, gather, label) for six, and holds 25 vector registers for
+// 52, which the fused kernel's mix of classes gains from: LFR-1M learned 2124
+// -> 1973 us.  (The 512-graph batch, bound by the resolver's issue, is
+// unchanged, and two rows a wave, for G = 32, lost as much again to selects.)
+template <class Resolve, bool VLIST, typename E>
+__device__ __forceinline__ uint32_t wave_rounds(const E *__restrict__ off, const int32_t *__restrict__ nbr,
+                                                const int32_t *__restrict__ prev, int32_t *__restrict__ next,
+                                                const int32_t *__restrict__ vlist, int64_t v0, int64_t nv,
+                                                int64_t bi, int64_t nb) {
+    constexpr int NW = 256 / kWave;
+    const int lane = lane_id();
+    const int64_t stride = nb * NW;
+    int64_t i = bi * NW + __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);   // uniform
+    struct St {
+        int64_t v;
+        E ob, oe;      // off[v], off[v + 1]
+        int32_t old;   // prev[v]
+        int32_t len;   // set by ldn; 0 past the end
+    };
+    auto ident = [&](int64_t i) -> int32_t { return VLIST ? vlist[v0 + (i < nv ? i : 0)] : 0; };
+    auto state = [&](int64_t i, int32_t id) {
+        St t;
+        t.v = VLIST ? (int64_t)id : v0 + (i < nv ? i : 0);
+        t.ob = off[t.v];
+        t.oe = off[t.v + 1];
+        t.old = prev[t.v];
+        t.len = 0;
+        return t;
+    };
+    auto ldn = [&](St &t, int64_t i) -> int32_t {
+        t.len = i < nv ? (int32_t)(t.oe - t.ob) : 0;
+        using U = typename std::conditional<sizeof(E) == 4, uint32_t, uint64_t>::type;
+        return __builtin_nontemporal_load(&nbr[lane < t.len ? (U)t.ob + (U)lane : (U)0]);
+    };
+    auto gat = [&](int32_t u, const St &t) -> int32_t { return prev[lane < t.len ? (uint32_t)u : 0u]; };
+    uint32_t changed = 0;
+    // the winner lane (best's low byte) holds the new label and writes it
+    auto resolve = [&](const St &t, int32_t Lraw) {
+        const int32_t L = lane < t.len ? Lraw : -1;
+        const uint32_t best = Resolve::template best<kWave>(L);
+        if (lane == (int)(best & 0xffu) && t.len > 0) {
+            next[t.v] = L;
+            changed += (L != t.old);
+        }
+    };
+    const int32_t ia = ident(i), ib = ident(i + stride), ic = ident(i + 2 * stride);
+    int32_t id = ident(i + 3 * stride);
+    St sa = state(i, ia), sb = state(i + stride, ib), sc = state(i + 2 * stride, ic), sd;
+    int32_t u = ldn(sa, i);
+    int32_t LA = gat(u, sa), LB;
+    u = ldn(sb, i + stride);
+#define GALP_GROUP_STAGE(S0, S1, S2, S3, LC, LN) \
+    LN = gat(u, S1);                             \
+    u = ldn(S2, i + 2 * stride);                 \
+    S3 = state(i + 3 * stride, id);              \
+    id = ident(i + 4 * stride);                  \
+    resolve(S0, LC);                             \
+    i += stride;                                 \
+    if (i >= nv) break;
+    while (i < nv) {
+        GALP_GROUP_STAGE(sa, sb, sc, sd, LA, LB)
+        GALP_GROUP_STAGE(sb, sc, sd, sa, LB, LA)
+        GALP_GROUP_STAGE(sc, sd, sa, sb, LA, LB)
+        GALP_GROUP_STAGE(sd, sa, sb, sc, LB, LA)
+    }
+#undef GALP_GROUP_STAGE
+    return changed;
+}
+
+template <int G, class Resolve, bool VLIST, typename E>
+__device__ __forceinline__ uint32_t group_rounds(const E *__restrict__ off, const int32_t *__restrict__ nbr,
+                                                 const int32_t *__restrict__ prev, int32_t *__restrict__ next,
+                                                 const int32_t *__restrict__ vlist, int64_t v0, int64_t nv,
+                                                 int64_t bi, int64_t nb) {
+    if constexpr (G == kWave) return wave_rounds<Resolve, VLIST, E>(off, nbr, prev, next, vlist, v0, nv, bi, nb);
+    else return group_rounds_lanes<G, Resolve, VLIST, E>(off, nbr, prev, next, vlist, v0, nv, bi, nb);
 }
 
 // Alt: the resolver of iterations where most rows are high-distinct (the

@@ -99,7 +99,9 @@ __device__ __forceinline__ uint32_t group_best(int32_t L) {
         } else {
             cnt = group_count_eq<G>(active ? L : -1);
         }
-        best = max(best, group_max<G>(active ? ((cnt << 8) | (uint32_t)(lane & (G - 1))) : 0u));
+        const uint32_t mine = active ? ((cnt << 8) | (uint32_t)(lane & (G - 1))) : 0u;
+        if constexpr (G == kWave) best = max(best, wave_max_u32(mine));
+        else best = max(best, group_max<G>(mine));
     }
     return best;
 }

@@ -42,7 +42,7 @@ __device__ __forceinline__ void pipelined(Policy &pol, const int32_t *__restrict
         for (int k = 0; k < EPT; ++k) {
             const int pos = k * T + tid;
             const bool ok = it.valid && pos < it.len;
-            lab[k] = prev[ok ? u[k] : 0];
+            lab[k] = prev[ok ? (uint32_t)u[k] : 0u];   // ids are not negative: no sign extension
         }
     };
     Item s0 = pol.item(i), s1 = pol.item(i + stride), s2 = pol.item(i + 2 * stride);
