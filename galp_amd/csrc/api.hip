@@ -138,10 +138,12 @@ static void dev_free_all(galp_graph *g) {
                     g->d_out, g->d_hub_vid, g->d_hub_nparts, g->d_item_hub, g->d_item_part, g->d_item_meta,
                     g->d_hub_best, g->d_merge_big, g->d_hub_tile0, g->d_hub_ntiles, g->d_tile_hub,
                     g->d_tile_idx_off,
-                    g->d_tile_idx, g->d_out_key, g->d_out_ent, g->d_counter, g->d_stop, g->d_iters_done, g->d_iter_counts, g->d_err};
+                    g->d_tile_idx, g->d_out_key, g->d_out_ent, g->d_counter, g->d_stop, g->d_iter_counts};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     if (g->h_pinned) (void)hipHostFree(g->h_pinned);
+    for (hipEvent_t e : g->ev)
+        if (e) (void)hipEventDestroy(e);
     for (auto e : g->prof.pool) (void)hipEventDestroy(e);
     for (auto &pl : g->prof.pending) {
         if (pl.e0) (void)hipEventDestroy(pl.e0);
@@ -369,9 +371,11 @@ static int upload_impl(galp_graph *g, const galp_csr_view *c) {
     GALP_TRY(dev_alloc(g, &g->d_lab[0], n));
     GALP_TRY(dev_alloc(g, &g->d_lab[1], n));
     GALP_TRY(dev_alloc(g, &g->d_counter, kCountShards * kCountStride));
-    GALP_TRY(dev_alloc(g, &g->d_stop, 1));
-    GALP_TRY(dev_alloc(g, &g->d_iters_done, 1));
-    GALP_TRY(dev_alloc(g, &g->d_err, 1));
+    GALP_TRY(dev_alloc(g, &g->d_stop, kCtlWords));
+    g->d_iters_done = g->d_stop + 1;
+    g->d_err = g->d_stop + 2;
+    GALP_HIP(ctx, hipEventCreate(&g->ev[0]));
+    GALP_HIP(ctx, hipEventCreate(&g->ev[1]));
     GALP_TRY(dev_alloc(g, &g->d_iter_counts, kMaxIters));
     GALP_HIP(ctx, hipHostMalloc((void **)&g->h_pinned, 64, hipHostMallocDefault));
 
@@ -601,12 +605,30 @@ static int run_captured(galp_graph *g, int niter) {
     return GALP_OK;
 }
 
+// Queues the readback of the control words into h_pinned; after a
+// synchronisation, the error a kernel set becomes the call's.
+static int read_ctl(galp_graph *g) {
+    GALP_HIP(g->ctx, hipMemcpyAsync(g->h_pinned, g->d_stop, 4 * kCtlWords, hipMemcpyDeviceToHost, g->stream));
+    return GALP_OK;
+}
+
 static int check_err(galp_graph *g) {
-    GALP_HIP(g->ctx, hipMemcpyAsync(g->h_pinned + 8, g->d_err, 4, hipMemcpyDeviceToHost, g->stream));
-    GALP_HIP(g->ctx, hipStreamSynchronize(g->stream));
-    if (g->h_pinned[8] != 0)
+    if (g->h_pinned[2] != 0)
         return fail(g->ctx, GALP_EHIP, "kernel reported an internal table overflow (code " +
-                                           std::to_string(g->h_pinned[8]) + ")");
+                                           std::to_string(g->h_pinned[2]) + ")");
+    return GALP_OK;
+}
+
+// labels[i] = i on the graph's stream, without waiting.
+static int queue_init(galp_graph *g) {
+    GALP_TRY(dev_init_labels(g));
+    GALP_TRY(learn_reset_iteration(g));
+    GALP_TRY(batch_reset(g));
+    g->cur = 0;
+    g->iter = 0;
+    g->identity = true;
+    g->initialized = true;
+    g->stop_set = false;
     return GALP_OK;
 }
 
@@ -744,14 +766,8 @@ GALP_API int galp_graph_query(galp_graph *g, galp_graph_info *out) {
 
 GALP_API int galp_lp_init(galp_graph *g) {
     if (!g) return GALP_EINVAL;
-    GALP_TRY(dev_init_labels(g));
-    GALP_TRY(learn_reset_iteration(g));
-    GALP_TRY(batch_reset(g));
+    GALP_TRY(queue_init(g));
     GALP_HIP(g->ctx, hipStreamSynchronize(g->stream));
-    g->cur = 0;
-    g->iter = 0;
-    g->identity = true;
-    g->initialized = true;
     return GALP_OK;
 }
 
@@ -779,41 +795,38 @@ GALP_API int galp_lp_set_labels(galp_graph *g, const int32_t *host_labels) {
     g->iter = 0;
     g->identity = false;
     g->initialized = true;
+    g->stop_set = false;
     return GALP_OK;
 }
 
 GALP_API int galp_lp_step(galp_graph *g, galp_step_stats *st) {
     if (!g) return GALP_EINVAL;
     if (!g->initialized) return fail(g->ctx, GALP_ESTATE, "galp_lp_step before galp_lp_init");
-    hipEvent_t e0, e1;
-    GALP_HIP(g->ctx, hipEventCreate(&e0));
-    GALP_HIP(g->ctx, hipEventCreate(&e1));
-    int rc = dev_clear_stop(g);
+    int rc = g->stop_set ? dev_clear_stop(g) : GALP_OK;
+    g->stop_set = true;   // until this iteration is known not to have set it
     if (rc == GALP_OK) {
-        (void)hipEventRecord(e0, g->stream);
+        (void)hipEventRecord(g->ev[0], g->stream);
         rc = launch_iteration(g);
-        (void)hipEventRecord(e1, g->stream);
+        (void)hipEventRecord(g->ev[1], g->stream);
     }
-    const int idx = g->iter % kMaxIters;
     if (rc == GALP_OK) {
-        hipError_t e = hipMemcpyAsync(g->h_pinned, g->d_iter_counts + idx, 8, hipMemcpyDeviceToHost, g->stream);
         g->h_pinned[9] = 0;
-        if (e == hipSuccess && learned_now(g))
+        hipError_t e = hipSuccess;
+        if (learned_now(g))
             e = hipMemcpyAsync(g->h_pinned + 9, g->learn->d_plist_n + kCtrOverflow, 4, hipMemcpyDeviceToHost,
                                g->stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(g->h_pinned + 2, g->d_stop, 4, hipMemcpyDeviceToHost, g->stream);
+        if (e == hipSuccess) rc = read_ctl(g);
         if (e == hipSuccess) e = hipStreamSynchronize(g->stream);
         if (e != hipSuccess) rc = fail(g->ctx, GALP_EHIP, std::string("step readback: ") + hipGetErrorString(e));
     }
     float ms = 0.f;
-    if (rc == GALP_OK) (void)hipEventElapsedTime(&ms, e0, e1);
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
+    if (rc == GALP_OK) (void)hipEventElapsedTime(&ms, g->ev[0], g->ev[1]);
     if (rc == GALP_OK) rc = check_err(g);
     prof_collect(g);
     if (rc != GALP_OK) return rc;
     long long cnt;
-    std::memcpy(&cnt, g->h_pinned, 8);
+    std::memcpy(&cnt, g->h_pinned + kCtlCount, 8);
+    g->stop_set = g->h_pinned[0] != 0;
     g->cur ^= 1;
     g->iter += 1;
     if (st) {
@@ -821,7 +834,7 @@ GALP_API int galp_lp_step(galp_graph *g, galp_step_stats *st) {
         st->overflowed = g->h_pinned[9];
         st->device_ms = ms;
         st->iteration = g->iter;
-        st->stopped = g->h_pinned[2] != 0;
+        st->stopped = g->stop_set;
     }
     return GALP_OK;
 }
@@ -845,10 +858,11 @@ GALP_API int galp_lp_run(galp_graph *g, int32_t niter, int32_t verbose, int32_t 
     if (!g) return GALP_EINVAL;
     if (niter < 0 || niter > kMaxIters) return fail(g->ctx, GALP_EINVAL, "niter must be in [0, 4096]");
     using clk = std::chrono::steady_clock;
-    GALP_TRY(galp_lp_init(g));
+    GALP_TRY(queue_init(g));
     auto t1 = clk::now();
     double dev_ms = 0.0;
     int done = 0;
+    bool have_labels = false;
     if (verbose) {
         for (int i = 0; i < niter; ++i) {
             auto ti = clk::now();
@@ -862,11 +876,9 @@ GALP_API int galp_lp_run(galp_graph *g, int32_t niter, int32_t verbose, int32_t 
         }
         std::fflush(stdout);
     } else {
-        hipEvent_t e0, e1;
-        GALP_HIP(g->ctx, hipEventCreate(&e0));
-        GALP_HIP(g->ctx, hipEventCreate(&e1));
-        int rc = dev_clear_stop(g);
-        (void)hipEventRecord(e0, g->stream);
+        int rc = GALP_OK;
+        g->stop_set = true;
+        (void)hipEventRecord(g->ev[0], g->stream);
         const int cur0 = g->cur;
         if (g->opts.graph_capture && !g->ooc && !g->prof.on && niter > 0) {
             rc = run_captured(g, niter);
@@ -877,26 +889,31 @@ GALP_API int galp_lp_run(galp_graph *g, int32_t niter, int32_t verbose, int32_t 
                 g->cur ^= 1;
             }
         }
-        (void)hipEventRecord(e1, g->stream);
+        (void)hipEventRecord(g->ev[1], g->stream);
+        if (rc == GALP_OK) rc = read_ctl(g);
         if (rc == GALP_OK) {
-            hipError_t e = hipMemcpyAsync(g->h_pinned + 4, g->d_iters_done, 4, hipMemcpyDeviceToHost, g->stream);
+            hipError_t e = hipSuccess;
+            if (labels_out && g->reorder && g->n) {   // queued behind the run: one wait for both
+                rc = dev_map_labels_done(g, cur0, g->d_out);
+                if (rc == GALP_OK)
+                    e = hipMemcpyAsync(labels_out, g->d_out, 4 * (size_t)g->n, hipMemcpyDeviceToHost, g->stream);
+                have_labels = true;
+            }
             if (e == hipSuccess) e = hipStreamSynchronize(g->stream);
             if (e != hipSuccess) rc = fail(g->ctx, GALP_EHIP, std::string("run readback: ") + hipGetErrorString(e));
         }
         float ms = 0.f;
-        if (rc == GALP_OK) (void)hipEventElapsedTime(&ms, e0, e1);
-        (void)hipEventDestroy(e0);
-        (void)hipEventDestroy(e1);
+        if (rc == GALP_OK) (void)hipEventElapsedTime(&ms, g->ev[0], g->ev[1]);
         if (rc == GALP_OK) rc = check_err(g);
         prof_collect(g);
         if (rc != GALP_OK) return rc;
-        done = niter ? g->h_pinned[4] : 0;
+        g->stop_set = g->h_pinned[0] != 0;
+        done = niter ? g->h_pinned[1] : 0;
         g->iter = done;
         g->cur = (cur0 + done) & 1;
         dev_ms = ms;
     }
-    if (labels_out) GALP_TRY(galp_lp_get_labels(g, labels_out));
-    GALP_HIP(g->ctx, hipDeviceSynchronize());
+    if (labels_out && !have_labels) GALP_TRY(galp_lp_get_labels(g, labels_out));
     double f1 = std::chrono::duration<double>(clk::now() - t1).count();
     if (res) {
         res->f1_s = f1;

@@ -199,6 +199,7 @@ k_batch_stop(unsigned long long *__restrict__ gcount, const int64_t *__restrict_
     __syncthreads();
     if (threadIdx.x == 0) {
         iter_counts[it] = (long long)stotal;
+        *(long long *)(stop + kCtlCount) = (long long)stotal;
         *iters_done = it + 1;
         if (!sactive) *stop = 1;
         if (rebuild) *rebuild = sstopped;

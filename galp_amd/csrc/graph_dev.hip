@@ -137,6 +137,17 @@ __global__ void k_map_labels(const int32_t *__restrict__ lab, const int32_t *__r
         out[v] = iperm[lab[perm[v]]];
 }
 
+// The same for the buffer a run of *done iterations from lab0 ended in, so the
+// read-out is queued without waiting for the count.
+__global__ void k_map_labels_done(const int32_t *__restrict__ lab0, const int32_t *__restrict__ lab1,
+                                  const int32_t *__restrict__ done, const int32_t *__restrict__ perm,
+                                  const int32_t *__restrict__ iperm, int32_t *__restrict__ out, int64_t n) {
+    const int32_t *lab = (*done & 1) ? lab1 : lab0;
+    for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n;
+         v += (int64_t)gridDim.x * blockDim.x)
+        out[v] = iperm[lab[perm[v]]];
+}
+
 // lab[perm[v]] = perm[in[v]]: original labels into the internal numbering.
 __global__ void k_unmap_labels(const int32_t *__restrict__ in, const int32_t *__restrict__ perm,
                                int32_t *__restrict__ lab, int64_t n) {
@@ -221,6 +232,15 @@ int launch_first_iteration(galp_graph *g) {
 
 int dev_map_labels(galp_graph *g, const int32_t *lab, int32_t *out) {
     if (g->n) k_map_labels<<<grid1d(g->n, 256), 256, 0, g->stream>>>(lab, g->d_perm, g->d_iperm, out, g->n);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail(g->ctx, GALP_EHIP, std::string("map kernel: ") + hipGetErrorString(e));
+    return GALP_OK;
+}
+
+int dev_map_labels_done(galp_graph *g, int cur0, int32_t *out) {
+    if (g->n)
+        k_map_labels_done<<<grid1d(g->n, 256), 256, 0, g->stream>>>(g->d_lab[cur0], g->d_lab[cur0 ^ 1], g->d_iters_done,
+                                                                   g->d_perm, g->d_iperm, out, g->n);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(g->ctx, GALP_EHIP, std::string("map kernel: ") + hipGetErrorString(e));
     return GALP_OK;

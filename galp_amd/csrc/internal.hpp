@@ -349,11 +349,16 @@ struct galp_graph {
 
     // iteration control (device)
     unsigned long long *d_counter = nullptr;
+    // kCtlWords words read back together (read_ctl): the stop flag, the
+    // iterations done, an error set by a kernel that hit an impossible state,
+    // and the last iteration's change count (kCtlCount, 64-bit)
     int32_t *d_stop = nullptr;
-    int32_t *d_iters_done = nullptr;
+    int32_t *d_iters_done = nullptr;     // d_stop + 1
+    int32_t *d_err = nullptr;            // d_stop + 2
     long long *d_iter_counts = nullptr;  // kMaxIters
-    int32_t *d_err = nullptr;            // set by a kernel that hit an impossible state
     int32_t *h_pinned = nullptr;         // pinned staging for small readbacks
+    hipEvent_t ev[2] = {nullptr, nullptr};   // around an iteration or a run
+    bool stop_set = false;               // the stop flag may be set: clear it before the next iteration
     int iter = 0;                        // iterations executed since init
     bool initialized = false;
     double preprocess_ms = 0.0;
@@ -382,6 +387,8 @@ struct galp_graph {
 namespace galp {
 
 constexpr int kMaxIters = 4096;
+constexpr int kCtlWords = 8;   // 32 bytes
+constexpr int kCtlCount = 4;
 
 int fail(galp_ctx *ctx, int code, const std::string &msg);
 
@@ -549,6 +556,7 @@ int dev_check_rows(galp_graph *g, int32_t *bad);
 // The first iteration from labels[i] = i of a graph whose rows strictly ascend.
 int launch_first_iteration(galp_graph *g);
 int dev_map_labels(galp_graph *g, const int32_t *lab, int32_t *out);
+int dev_map_labels_done(galp_graph *g, int cur0, int32_t *out);   // after *d_iters_done iterations from d_lab[cur0]
 int dev_unmap_labels(galp_graph *g, const int32_t *in, int32_t *lab);
 
 // Profiling helpers (api.hip): bracket a launch with events when enabled.

@@ -1052,6 +1052,7 @@ k_iter_end(unsigned long long *counter, int32_t *stop, long long *iter_counts, i
     for (int s = kWave / 2; s > 0; s >>= 1) c += __shfl_xor(c, s);
     if (threadIdx.x) return;
     iter_counts[it] = (long long)c;
+    *(long long *)(stop + kCtlCount) = (long long)c;
     *iters_done = it + 1;
     if ((double)c <= thr) *stop = 1;
 }
