@@ -377,7 +377,10 @@ static int upload_impl(galp_graph *g, const galp_csr_view *c) {
     GALP_HIP(ctx, hipEventCreate(&g->ev[0]));
     GALP_HIP(ctx, hipEventCreate(&g->ev[1]));
     GALP_TRY(dev_alloc(g, &g->d_iter_counts, kMaxIters));
-    GALP_HIP(ctx, hipHostMalloc((void **)&g->h_pinned, 64, hipHostMallocDefault));
+    const int64_t host_labels = g->reorder && n <= kHostLabels ? n : 0;
+    GALP_HIP(ctx, hipHostMalloc((void **)&g->h_pinned, 4 * (size_t)(kPinnedWords + host_labels), hipHostMallocDefault));
+    std::memset(g->h_pinned, 0, 4 * kPinnedWords);
+    if (host_labels) g->h_labels = g->h_pinned + kPinnedWords;
 
     if (g->off64) GALP_TRY(upload_offsets<int64_t>(g, offi));
     else GALP_TRY(upload_offsets<int32_t>(g, offi));
@@ -499,8 +502,9 @@ IterView full_view(const galp_graph *g) {
 }
 
 bool fused_rows(const galp_graph *g) {
-    return !g->ooc && !g->prof.on && !g->class_kernels && g->m < kFusedMaxEdges &&
-           (g->opts.method == GALP_METHOD_HASH ? g->opts.variant == 1 : g->opts.policy == GALP_POLICY_INCORE);
+    if (g->ooc || g->prof.on || g->class_kernels) return false;
+    return g->opts.method == GALP_METHOD_HASH ? g->opts.variant == 1 && g->m < kFusedMaxEdges
+                                              : g->opts.policy == GALP_POLICY_INCORE && g->m < kFusedMaxEdgesSort;
 }
 
 bool concurrent_allowed(const galp_graph *g) {
@@ -539,6 +543,7 @@ static int launch_iteration(galp_graph *g) {
     const bool first = g->iter == 0 && g->identity && g->rows_ascend && (!g->ooc || g->ooc->d_last);
     // drops the graphs that stopped; in the first iteration too, whose end
     // overwrites the rebuild flag that batch_reset set
+    g->ended = false;
     if (g->batch) GALP_TRY(launch_batch_lists(g));
     if (!first && front_now(g)) GALP_TRY(launch_front(g));
     switch (g->opts.method) {
@@ -561,6 +566,7 @@ static int launch_iteration(galp_graph *g) {
     default:
         return fail(g->ctx, GALP_EUNSUPPORTED, "method " + std::to_string(g->opts.method) + " is not built");
     }
+    if (g->ended) return GALP_OK;   // by the iteration's last kernel
     return g->batch ? launch_batch_end(g) : launch_iter_end(g);
 }
 
@@ -605,13 +611,7 @@ static int run_captured(galp_graph *g, int niter) {
     return GALP_OK;
 }
 
-// Queues the readback of the control words into h_pinned; after a
-// synchronisation, the error a kernel set becomes the call's.
-static int read_ctl(galp_graph *g) {
-    GALP_HIP(g->ctx, hipMemcpyAsync(g->h_pinned, g->d_stop, 4 * kCtlWords, hipMemcpyDeviceToHost, g->stream));
-    return GALP_OK;
-}
-
+// After a synchronisation: the error a kernel set becomes the call's.
 static int check_err(galp_graph *g) {
     if (g->h_pinned[2] != 0)
         return fail(g->ctx, GALP_EHIP, "kernel reported an internal table overflow (code " +
@@ -803,6 +803,7 @@ GALP_API int galp_lp_step(galp_graph *g, galp_step_stats *st) {
     if (!g) return GALP_EINVAL;
     if (!g->initialized) return fail(g->ctx, GALP_ESTATE, "galp_lp_step before galp_lp_init");
     int rc = g->stop_set ? dev_clear_stop(g) : GALP_OK;
+    std::memset(g->h_pinned, 0, 4 * kCtlWords);   // idle: every call waits for its work
     g->stop_set = true;   // until this iteration is known not to have set it
     if (rc == GALP_OK) {
         (void)hipEventRecord(g->ev[0], g->stream);
@@ -815,7 +816,6 @@ GALP_API int galp_lp_step(galp_graph *g, galp_step_stats *st) {
         if (learned_now(g))
             e = hipMemcpyAsync(g->h_pinned + 9, g->learn->d_plist_n + kCtrOverflow, 4, hipMemcpyDeviceToHost,
                                g->stream);
-        if (e == hipSuccess) rc = read_ctl(g);
         if (e == hipSuccess) e = hipStreamSynchronize(g->stream);
         if (e != hipSuccess) rc = fail(g->ctx, GALP_EHIP, std::string("step readback: ") + hipGetErrorString(e));
     }
@@ -844,6 +844,12 @@ GALP_API int galp_lp_get_labels(galp_graph *g, int32_t *host_out) {
     if (!g->initialized) return fail(g->ctx, GALP_ESTATE, "labels read before galp_lp_init");
     if (!g->n) return GALP_OK;
     const int32_t *src = g->d_lab[g->cur];
+    if (g->h_labels) {
+        GALP_TRY(dev_map_labels(g, src, g->h_labels));
+        GALP_HIP(g->ctx, hipStreamSynchronize(g->stream));
+        std::memcpy(host_out, g->h_labels, 4 * (size_t)g->n);
+        return GALP_OK;
+    }
     if (g->reorder) {
         GALP_TRY(dev_map_labels(g, src, g->d_out));
         src = g->d_out;
@@ -878,6 +884,7 @@ GALP_API int galp_lp_run(galp_graph *g, int32_t niter, int32_t verbose, int32_t 
     } else {
         int rc = GALP_OK;
         g->stop_set = true;
+        std::memset(g->h_pinned, 0, 4 * kCtlWords);   // idle: every call waits for its work
         (void)hipEventRecord(g->ev[0], g->stream);
         const int cur0 = g->cur;
         if (g->opts.graph_capture && !g->ooc && !g->prof.on && niter > 0) {
@@ -890,12 +897,11 @@ GALP_API int galp_lp_run(galp_graph *g, int32_t niter, int32_t verbose, int32_t 
             }
         }
         (void)hipEventRecord(g->ev[1], g->stream);
-        if (rc == GALP_OK) rc = read_ctl(g);
         if (rc == GALP_OK) {
             hipError_t e = hipSuccess;
             if (labels_out && g->reorder && g->n) {   // queued behind the run: one wait for both
-                rc = dev_map_labels_done(g, cur0, g->d_out);
-                if (rc == GALP_OK)
+                rc = dev_map_labels_done(g, cur0, g->h_labels ? g->h_labels : g->d_out);
+                if (rc == GALP_OK && !g->h_labels)
                     e = hipMemcpyAsync(labels_out, g->d_out, 4 * (size_t)g->n, hipMemcpyDeviceToHost, g->stream);
                 have_labels = true;
             }
@@ -908,6 +914,7 @@ GALP_API int galp_lp_run(galp_graph *g, int32_t niter, int32_t verbose, int32_t 
         prof_collect(g);
         if (rc != GALP_OK) return rc;
         g->stop_set = g->h_pinned[0] != 0;
+        if (have_labels && g->h_labels) std::memcpy(labels_out, g->h_labels, 4 * (size_t)g->n);
         done = niter ? g->h_pinned[1] : 0;
         g->iter = done;
         g->cur = (cur0 + done) & 1;

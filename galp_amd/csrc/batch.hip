@@ -165,7 +165,7 @@ __global__ void __launch_bounds__(1024)
 k_batch_stop(unsigned long long *__restrict__ gcount, const int64_t *__restrict__ gn, int32_t *__restrict__ gstop,
              int32_t *__restrict__ giters, int64_t ngraphs, unsigned long long *__restrict__ counter,
              int32_t *__restrict__ stop, long long *__restrict__ iter_counts, int32_t *__restrict__ iters_done,
-             int it, int64_t *__restrict__ rebuild, int64_t *__restrict__ front) {
+             int it, int64_t *__restrict__ rebuild, int64_t *__restrict__ front, int32_t *host) {
     __shared__ unsigned long long stotal;
     __shared__ int32_t sactive, sstopped;
     if (*stop) return;
@@ -199,9 +199,9 @@ k_batch_stop(unsigned long long *__restrict__ gcount, const int64_t *__restrict_
     __syncthreads();
     if (threadIdx.x == 0) {
         iter_counts[it] = (long long)stotal;
-        *(long long *)(stop + kCtlCount) = (long long)stotal;
         *iters_done = it + 1;
         if (!sactive) *stop = 1;
+        publish_ctl(host, stop, !sactive, it + 1, (long long)stotal);
         if (rebuild) *rebuild = sstopped;
     }
 }
@@ -266,7 +266,7 @@ int launch_batch_end(galp_graph *g) {
     k_batch_epilogue<<<grid, 256, 0, g->stream>>>(prev, next, B->d_gid, B->d_gstop, B->d_gcount, g->n, g->d_stop);
     k_batch_stop<<<1, 1024, 0, g->stream>>>(B->d_gcount, B->d_gn, B->d_gstop, B->d_giters, B->ngraphs, g->d_counter,
                                             g->d_stop, g->d_iter_counts, g->d_iters_done, g->iter % kMaxIters,
-                                            B->lists ? B->d_alen + NUM_BUCKETS : nullptr, front_ctl(g));
+                                            B->lists ? B->d_alen + NUM_BUCKETS : nullptr, front_ctl(g), g->h_pinned);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? GALP_OK : fail(g->ctx, GALP_EHIP, std::string("batch epilogue: ") + hipGetErrorString(e));
 }

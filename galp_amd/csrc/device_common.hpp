@@ -287,6 +287,88 @@ __device__ __forceinline__ void block_count_add(uint32_t mine, unsigned long lon
     }
 }
 
+// The bookkeeping at an iteration's end, done by k_iter_end or by the last
+// block of the iteration's last kernel (on != 0).
+struct IterEnd {
+    int32_t on;
+    int32_t it;                 // slot of the iteration
+    double thr;                 // stop at or below this many changes
+    int32_t *stop;
+    int32_t *iters_done;
+    long long *iter_counts;
+    int64_t *front;             // the frontier's control words, cleared (may be null)
+    int32_t *host;              // the control words' copy in pinned host memory
+};
+constexpr int kEndCount = 4;    // host + kEndCount: the last change count, 64-bit
+constexpr int kEndFront = 32;   // words of front
+
+// The control words as the host reads them after a synchronisation: written
+// by the iteration's end itself, so no copy is queued behind it.
+__device__ __forceinline__ void publish_ctl(int32_t *host, int32_t *stop, int32_t stopped, int32_t done, long long count) {
+    host[0] = stopped;
+    host[1] = done;
+    host[2] = __hip_atomic_load(stop + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // the error word
+    *(long long *)(host + kEndCount) = count;
+}
+
+// One wave: sums the shards of the change counter and clears them, records
+// the iteration and applies the stop rule.
+__device__ __forceinline__ void end_iteration(unsigned long long *counter, const IterEnd &e) {
+    static_assert(kCountShards == kWave && kEndFront <= kWave, "one lane per shard");
+    unsigned long long *shard = counter + lane_id() * kCountStride;
+    unsigned long long c = __hip_atomic_load(shard, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    shard[0] = 0ull;
+    shard[1] = 0ull;   // tickets
+    shard[2] = 0ull;
+    if (e.front && lane_id() < kEndFront) e.front[lane_id()] = 0;
+#pragma unroll
+    for (int s = kWave / 2; s > 0; s >>= 1) c += __shfl_xor(c, s);
+    if (lane_id()) return;
+    e.iter_counts[e.it] = (long long)c;
+    *e.iters_done = e.it + 1;
+    const int32_t stopped = (double)c <= e.thr;
+    if (stopped) *e.stop = 1;
+    publish_ctl(e.host, e.stop, stopped, e.it + 1, (long long)c);
+}
+
+// block_count_add that ends the iteration when e.on: every block of the grid
+// calls it once, and the last one to come does the bookkeeping, which saves
+// the small graphs a launch per iteration (5 us between two short kernels).
+// Only atomics are ordered here, and each is complete when its result is back,
+// so no block fences or flushes a cache: the count goes to the block's shard,
+// then a ticket to the shard's line, and the last block of each shard takes
+// one of the whole grid.
+template <int NW>
+__device__ __forceinline__ void block_count_end(uint32_t mine, unsigned long long *counter, uint32_t *scratch,
+                                                const IterEnd &e) {
+    if (!e.on) {   // uniform
+        block_count_add<NW>(mine, counter, scratch);
+        return;
+    }
+    uint32_t s = wave_sum_u32(mine);
+    const int w = (int)(threadIdx.x / kWave);
+    __syncthreads();
+    if (lane_id() == 0) scratch[w] = s;
+    __syncthreads();
+    if (w) return;
+    int last = 0;
+    if (lane_id() == 0) {
+        unsigned long long t = 0;
+#pragma unroll
+        for (int i = 0; i < NW; ++i) t += scratch[i];
+        unsigned long long *shard = count_shard(counter);
+        unsigned long long done = atomicAdd(shard, t);
+        asm volatile("s_waitcnt vmcnt(0)" : "+v"(done)::"memory");   // counted before the ticket is taken
+        const uint32_t k = blockIdx.x & (kCountShards - 1);
+        const uint32_t blocks = (gridDim.x - k + kCountShards - 1) / kCountShards;   // of this shard
+        if (atomicAdd(shard + 1, 1ull) + 1ull == blocks) {
+            const uint32_t shards = gridDim.x < (uint32_t)kCountShards ? gridDim.x : (uint32_t)kCountShards;
+            last = atomicAdd(counter + 2, 1ull) + 1ull == shards;
+        }
+    }
+    if (__builtin_amdgcn_readfirstlane(last)) end_iteration(counter, e);
+}
+
 // Loads that bypass the per-CU vector L1, for table words other workgroups
 // update with device-scope atomics.
 __device__ __forceinline__ uint32_t load_coherent(const uint32_t *p) {

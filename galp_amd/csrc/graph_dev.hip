@@ -16,7 +16,16 @@
 
 namespace galp {
 
-__global__ void k_iota2(int32_t *a, int32_t *b, int64_t n) {
+// labels[i] = i in both buffers; the first block clears the control words, with
+// them the iteration count and the error word.
+__global__ void k_init_labels(int32_t *a, int32_t *b, int64_t n, unsigned long long *counter, int32_t *stop,
+                              int64_t *front) {
+    if (blockIdx.x == 0) {
+        if (threadIdx.x < kCountShards)
+            for (int k = 0; k < 3; ++k) counter[threadIdx.x * kCountStride + k] = 0ull;
+        if (front && threadIdx.x < kFrontCtl) front[threadIdx.x] = 0;
+        if (threadIdx.x < kCtlWords) stop[threadIdx.x] = 0;
+    }
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
          i += (int64_t)gridDim.x * blockDim.x) {
         a[i] = (int32_t)i;
@@ -30,18 +39,13 @@ __global__ void k_fill_u32(uint32_t *p, int64_t n, uint32_t val) {
         p[i] = val;
 }
 
-// One thread per shard of the change counter.
+// Clears the stop flag and what an unfinished iteration may have left; one
+// thread per shard of the change counter.
 __global__ void __launch_bounds__(kCountShards)
-k_reset_control(unsigned long long *counter, int32_t *stop, int32_t *iters_done,
-                                int32_t *err, int reset_done, int64_t *front) {
-    counter[threadIdx.x * kCountStride] = 0ull;
+k_clear_stop(unsigned long long *counter, int32_t *stop, int64_t *front) {
+    for (int k = 0; k < 3; ++k) counter[threadIdx.x * kCountStride + k] = 0ull;
     if (front && threadIdx.x < kFrontCtl) front[threadIdx.x] = 0;
-    if (threadIdx.x) return;
-    *stop = 0;
-    if (reset_done) {
-        *iters_done = 0;
-        *err = 0;
-    }
+    if (threadIdx.x == 0) *stop = 0;
 }
 
 // One wave per internal row k: copy row iperm[k] of the original CSR,
@@ -96,9 +100,9 @@ template <typename E>
 __global__ void __launch_bounds__(256)
 k_first_iteration(const E *__restrict__ off, const int32_t *__restrict__ nbr, const int32_t *__restrict__ last,
                   int32_t *__restrict__ next, int32_t *__restrict__ dist, int64_t n,
-                  unsigned long long *__restrict__ counter, const int32_t *__restrict__ stop) {
+                  unsigned long long *__restrict__ counter, IterEnd end) {
     __shared__ uint32_t scratch[256 / kWave];
-    if (*stop) return;
+    if (*end.stop) return;
     const int64_t nthreads = (int64_t)gridDim.x * 256;
     uint32_t changed = 0;
     for (int64_t v0 = (int64_t)blockIdx.x * 256 + threadIdx.x; v0 < n; v0 += kFirstUnroll * nthreads) {
@@ -126,7 +130,7 @@ k_first_iteration(const E *__restrict__ off, const int32_t *__restrict__ nbr, co
             }
         }
     }
-    block_count_add<4>(changed, counter, scratch);
+    block_count_end<4>(changed, counter, scratch, end);
 }
 
 // out[v] = iperm[labels[perm[v]]]: internal labels back to original ids.
@@ -163,15 +167,15 @@ static int grid1d(int64_t n, int threads) {
 }
 
 int dev_init_labels(galp_graph *g) {
-    if (g->n) k_iota2<<<grid1d(g->n, 256), 256, 0, g->stream>>>(g->d_lab[0], g->d_lab[1], g->n);
-    k_reset_control<<<1, kCountShards, 0, g->stream>>>(g->d_counter, g->d_stop, g->d_iters_done, g->d_err, 1, front_ctl(g));
+    k_init_labels<<<grid1d(g->n, 256), 256, 0, g->stream>>>(g->d_lab[0], g->d_lab[1], g->n, g->d_counter, g->d_stop,
+                                                            front_ctl(g));
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(g->ctx, GALP_EHIP, std::string("init kernels: ") + hipGetErrorString(e));
     return GALP_OK;
 }
 
 int dev_clear_stop(galp_graph *g) {
-    k_reset_control<<<1, kCountShards, 0, g->stream>>>(g->d_counter, g->d_stop, g->d_iters_done, g->d_err, 0, front_ctl(g));
+    k_clear_stop<<<1, kCountShards, 0, g->stream>>>(g->d_counter, g->d_stop, front_ctl(g));
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(g->ctx, GALP_EHIP, std::string("reset kernel: ") + hipGetErrorString(e));
     return GALP_OK;
@@ -217,13 +221,15 @@ int launch_first_iteration(galp_graph *g) {
     const int grid = (int)std::min<int64_t>((g->n + per_block - 1) / per_block,
                                             (int64_t)g->ctx->prop.multiProcessorCount * 8);
     PendingLaunch pl;
+    g->ended = may_end(g);
+    const IterEnd end = iter_end_args(g, g->ended);
     prof_begin(g, "first", (double)g->n * (8.0 + 2.0 * (g->off64 ? 8 : 4)), &pl);   // offsets, last id, next label
     if (g->off64)
         k_first_iteration<int64_t><<<grid, 256, 0, g->stream>>>((const int64_t *)g->d_off, g->d_nbr, last, next, dist,
-                                                                g->n, g->d_counter, g->d_stop);
+                                                                g->n, g->d_counter, end);
     else
         k_first_iteration<int32_t><<<grid, 256, 0, g->stream>>>((const int32_t *)g->d_off, g->d_nbr, last, next, dist,
-                                                                g->n, g->d_counter, g->d_stop);
+                                                                g->n, g->d_counter, end);
     prof_end(g, &pl);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(g->ctx, GALP_EHIP, std::string("first iteration: ") + hipGetErrorString(e));

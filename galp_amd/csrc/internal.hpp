@@ -7,6 +7,7 @@
 #include <string>
 #include <vector>
 
+#include "device_common.hpp"
 #include "galp.h"
 
 namespace galp {
@@ -349,15 +350,17 @@ struct galp_graph {
 
     // iteration control (device)
     unsigned long long *d_counter = nullptr;
-    // kCtlWords words read back together (read_ctl): the stop flag, the
-    // iterations done, an error set by a kernel that hit an impossible state,
-    // and the last iteration's change count (kCtlCount, 64-bit)
+    // kCtlWords words: the stop flag, the iterations done, an error set by a
+    // kernel that hit an impossible state; every iteration's end writes them
+    // and its change count (kCtlCount, 64-bit) to h_pinned as well
     int32_t *d_stop = nullptr;
     int32_t *d_iters_done = nullptr;     // d_stop + 1
     int32_t *d_err = nullptr;            // d_stop + 2
     long long *d_iter_counts = nullptr;  // kMaxIters
-    int32_t *h_pinned = nullptr;         // pinned staging for small readbacks
+    int32_t *h_pinned = nullptr;         // pinned: kPinnedWords, then h_labels
+    int32_t *h_labels = nullptr;         // labels of a small graph, written by the device (null: copied)
     hipEvent_t ev[2] = {nullptr, nullptr};   // around an iteration or a run
+    bool ended = false;                  // the iteration being launched ends in its last kernel
     bool stop_set = false;               // the stop flag may be set: clear it before the next iteration
     int iter = 0;                        // iterations executed since init
     bool initialized = false;
@@ -389,6 +392,11 @@ namespace galp {
 constexpr int kMaxIters = 4096;
 constexpr int kCtlWords = 8;   // 32 bytes
 constexpr int kCtlCount = 4;
+// The labels of graphs up to kHostLabels vertices go to pinned host memory as
+// they are mapped, and from there to the caller: a copy command behind the run
+// costs more than the kernel writing 256 KB over the host link (5 us).
+constexpr int kPinnedWords = 16;
+constexpr int64_t kHostLabels = (int64_t)1 << 16;
 
 int fail(galp_ctx *ctx, int code, const std::string &msg);
 
@@ -438,8 +446,17 @@ constexpr int64_t kConcurrentMaxVertices = (int64_t)1 << 25;
 // All row classes below B4K in one launch (rows_fused.hpp): in core, up to
 // kFusedMaxEdges edges, the default variants, unless single kernels are timed
 // or were chosen by hand (galp_graph_set_tuning).
+// The sort method's kernel holds 16 keys a lane for its largest class and has
+// half the waves of the class kernels: RMAT-20 (31 M edges) 3.89 ms with a
+// kernel per class, 4.08 fused.
 constexpr int64_t kFusedMaxEdges = (int64_t)1 << 25;
+constexpr int64_t kFusedMaxEdgesSort = (int64_t)1 << 24;
 bool fused_rows(const galp_graph *g);
+// An iteration's last kernel may do its bookkeeping: not in a batch (each
+// graph has its own) nor while samples are logged (the log kernel comes after
+// and reads the stop flag).
+inline bool may_end(const galp_graph *g) { return !g->batch && !(g->learn && g->learn->log_cap); }
+IterEnd iter_end_args(const galp_graph *g, bool on);
 bool concurrent_allowed(const galp_graph *g);
 bool concurrent_classes(const galp_graph *g);
 // Launches made between side_begin(g, k) and side_end(g, k, s) go to side

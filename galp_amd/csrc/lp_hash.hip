@@ -421,15 +421,15 @@ template <typename E>
 __global__ void __launch_bounds__(kRowsThreads) __attribute__((amdgpu_waves_per_eu(kRowsPerCu)))
 k_hash_rows(RowsArgs<kHashRows> args, const E *__restrict__ off, const int32_t *__restrict__ nbr,
             const int32_t *__restrict__ prev, int32_t *__restrict__ next, unsigned long long *__restrict__ counter,
-            const int32_t *__restrict__ stop, int32_t *__restrict__ err, int32_t *__restrict__ distinct) {
+            int32_t *__restrict__ err, int32_t *__restrict__ distinct, IterEnd end) {
     __shared__ uint32_t tab[2 << 12];   // keys and counts: 4 x 1024 slots or 4096
     __shared__ uint32_t sred[kRowsWaves];
     __shared__ unsigned long long sred64[kRowsWaves];
-    if (*stop) return;
+    if (*end.stop) return;
     const RowsWork w = rows_work(args);
-    if (w.cls < 0) return;
     uint32_t changed = 0;
     switch (w.cls) {   // uniform
+    case -1: break;   // more blocks than this iteration's rows
     case B_G4: changed = fused_group<4, E>(w, off, nbr, prev, next); break;
     case B_G8: changed = fused_group<8, E>(w, off, nbr, prev, next); break;
     case B_G16: changed = fused_group<16, E>(w, off, nbr, prev, next); break;
@@ -449,7 +449,7 @@ k_hash_rows(RowsArgs<kHashRows> args, const E *__restrict__ off, const int32_t *
         break;
     default: changed = fused_tables<256, 8, 12, E>(w, off, nbr, prev, next, tab, sred, sred64, err, distinct);
     }
-    block_count_add<kRowsWaves>(changed, counter, sred);
+    block_count_end<kRowsWaves>(changed, counter, sred, end);
 }
 
 // ---------------------------------------------------------------------------
@@ -1037,24 +1037,9 @@ k_hub_final(const E *__restrict__ off, const int32_t *__restrict__ nbr, const in
     block_count_add<4>(changed, counter, sred);
 }
 
-// One wave: sums the shards of the change counter, clears them and the
-// frontier's control words (front may be null), records the iteration and
-// applies the stop rule.
-__global__ void __launch_bounds__(kCountShards)
-k_iter_end(unsigned long long *counter, int32_t *stop, long long *iter_counts, int32_t *iters_done, int it,
-           double thr, int64_t *front) {
-    static_assert(kCountShards == kWave, "one lane per shard");
-    if (*stop) return;
-    if (front && threadIdx.x < kFrontCtl) front[threadIdx.x] = 0;
-    unsigned long long c = counter[threadIdx.x * kCountStride];
-    counter[threadIdx.x * kCountStride] = 0ull;
-#pragma unroll
-    for (int s = kWave / 2; s > 0; s >>= 1) c += __shfl_xor(c, s);
-    if (threadIdx.x) return;
-    iter_counts[it] = (long long)c;
-    *(long long *)(stop + kCtlCount) = (long long)c;
-    *iters_done = it + 1;
-    if ((double)c <= thr) *stop = 1;
+__global__ void __launch_bounds__(kCountShards) k_iter_end(unsigned long long *counter, IterEnd e) {
+    if (*e.stop) return;
+    end_iteration(counter, e);
 }
 
 // ---------------------------------------------------------------------------
@@ -1257,8 +1242,9 @@ static void launch_rows(galp_graph *g, const IterView &w, const int32_t *prev, i
     }
     const int grid = rows_plan(g, w, a, B_W128);
     if (!grid) return;
+    g->ended = may_end(g);   // the last kernel of the iteration
     k_hash_rows<E><<<grid, kRowsThreads, 0, g->stream>>>(a, (const E *)w.off, w.nbr, prev, next, g->d_counter,
-                                                         g->d_stop, g->d_err, distinct_out(g));
+                                                         g->d_err, distinct_out(g), iter_end_args(g, g->ended));
 }
 
 int launch_hash_class(galp_graph *g, int b) {
@@ -1347,9 +1333,14 @@ int launch_hash_iteration_incore(galp_graph *g) {
     return g->off64 ? hash_iteration_incore<int64_t>(g) : hash_iteration_incore<int32_t>(g);
 }
 
+IterEnd iter_end_args(const galp_graph *g, bool on) {
+    static_assert(kEndCount == kCtlCount && kEndFront == kFrontCtl, "the control words' layout");
+    return IterEnd{on,           g->iter % kMaxIters, (double)g->n * 1e-5, g->d_stop, g->d_iters_done,
+                   g->d_iter_counts, front_ctl(g), g->h_pinned};
+}
+
 int launch_iter_end(galp_graph *g) {
-    k_iter_end<<<1, kCountShards, 0, g->stream>>>(g->d_counter, g->d_stop, g->d_iter_counts, g->d_iters_done,
-                                       g->iter % kMaxIters, (double)g->n * 1e-5, front_ctl(g));
+    k_iter_end<<<1, kCountShards, 0, g->stream>>>(g->d_counter, iter_end_args(g, true));
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(g->ctx, GALP_EHIP, std::string("iter_end launch: ") + hipGetErrorString(e));
     return GALP_OK;

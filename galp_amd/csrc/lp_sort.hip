@@ -36,6 +36,7 @@
 #include "group_kernel.hpp"
 #include "internal.hpp"
 #include "pipeline.hpp"
+#include "rows_fused.hpp"
 
 namespace galp {
 
@@ -294,6 +295,7 @@ struct RegBitonicPolicy {
     int *sw;                  // NW
     unsigned long long *sred64;   // NW
     int32_t *err;
+    int tid;   // within the row's threads
     uint32_t changed;
 
     __device__ Item item(int64_t i) const {
@@ -305,7 +307,7 @@ struct RegBitonicPolicy {
             it.old = prev[it.v];
             it.valid = true;
             if (it.len > N) {   // never planned into this class
-                if (threadIdx.x == 0) atomicOr(err, 8);
+                if (tid == 0) atomicOr(err, 8);
                 it.len = 0;
             }
         }
@@ -315,7 +317,6 @@ struct RegBitonicPolicy {
 
     __device__ void process(const Item &it, const int32_t (&lab)[EPT]) {
         if (it.len == 0) return;   // uniform per block
-        const int tid = (int)threadIdx.x;
         const int lane = lane_id();
         unsigned long long key[EPT];
 #pragma unroll
@@ -414,10 +415,60 @@ k_sort_reg(const E *__restrict__ off, const int32_t *__restrict__ nbr, const int
     __shared__ uint32_t sred[NW];
     if (*stop) return;
     take_front(front, vlist, v0, nv);
-    RegBitonicPolicy<NW, EPT, E> pol{off, prev, next, vlist, v0, nv, sx, sedge, sw, sred64, err, 0u};
+    RegBitonicPolicy<NW, EPT, E> pol{off, prev, next, vlist, v0, nv, sx, sedge, sw, sred64, err,
+                                     (int)threadIdx.x, 0u};
     pipelined<T, EPT>(pol, nbr, prev, (int64_t)blockIdx.x, (int64_t)gridDim.x, (int)threadIdx.x);
     if constexpr (NW > 1) __syncthreads();
     block_count_add<NW>(pol.changed, counter, sred);
+}
+
+// ---------------------------------------------------------------------------
+// All classes up to degree 1024 in one launch (rows_fused.hpp): the lane
+// groups, and 65..1024 with a wave per row sorted in registers.
+constexpr int kSortRows = B_B1K + 1;
+template <int EPT, typename E>
+__device__ __forceinline__ uint32_t fused_sort(const RowsWork &w, const E *off, const int32_t *nbr,
+                                               const int32_t *prev, int32_t *next, int32_t *err) {
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+    const int64_t first = w.bi * kRowsWaves + wave, stride = w.nb * kRowsWaves;
+    if (first >= w.r.nv) return 0;
+    RegBitonicPolicy<1, EPT, E> pol{off,     prev,    next,    w.r.vlist, w.r.v0, w.r.nv, nullptr,
+                                    nullptr, nullptr, nullptr, err,       lane_id(), 0u};
+    pipelined<kWave, EPT>(pol, nbr, prev, first, stride, lane_id());
+    return pol.changed;
+}
+
+template <int G, typename E>
+__device__ __forceinline__ uint32_t fused_sort_group(const RowsWork &w, const E *off, const int32_t *nbr,
+                                                     const int32_t *prev, int32_t *next) {
+    if (w.bi * (kRowsThreads / G) >= w.r.nv) return 0;
+    if (w.r.vlist)
+        return group_rounds<G, SortGroupResolve, true, E>(off, nbr, prev, next, w.r.vlist, w.r.v0, w.r.nv, w.bi, w.nb);
+    return group_rounds<G, SortGroupResolve, false, E>(off, nbr, prev, next, nullptr, w.r.v0, w.r.nv, w.bi, w.nb);
+}
+
+template <typename E>
+__global__ void __launch_bounds__(kRowsThreads) __attribute__((amdgpu_waves_per_eu(kRowsPerCu)))
+k_sort_rows(RowsArgs<kSortRows> args, const E *__restrict__ off, const int32_t *__restrict__ nbr,
+            const int32_t *__restrict__ prev, int32_t *__restrict__ next, unsigned long long *__restrict__ counter,
+            int32_t *__restrict__ err, IterEnd end) {
+    __shared__ uint32_t sred[kRowsWaves];
+    if (*end.stop) return;
+    const RowsWork w = rows_work(args);
+    uint32_t changed = 0;
+    switch (w.cls) {   // uniform
+    case -1: break;   // more blocks than this iteration's rows
+    case B_G4: changed = fused_sort_group<4, E>(w, off, nbr, prev, next); break;
+    case B_G8: changed = fused_sort_group<8, E>(w, off, nbr, prev, next); break;
+    case B_G16: changed = fused_sort_group<16, E>(w, off, nbr, prev, next); break;
+    case B_G32: changed = fused_sort_group<32, E>(w, off, nbr, prev, next); break;
+    case B_G64: changed = fused_sort_group<64, E>(w, off, nbr, prev, next); break;
+    case B_W128: changed = fused_sort<2, E>(w, off, nbr, prev, next, err); break;
+    case B_W256: changed = fused_sort<4, E>(w, off, nbr, prev, next, err); break;
+    case B_W512: changed = fused_sort<8, E>(w, off, nbr, prev, next, err); break;
+    default: changed = fused_sort<16, E>(w, off, nbr, prev, next, err);
+    }
+    block_count_end<kRowsWaves>(changed, counter, sred, end);
 }
 
 // ---------------------------------------------------------------------------
@@ -1398,6 +1449,24 @@ static int sort_class(galp_graph *g, const IterView &w, int b, const int32_t *pr
     return GALP_OK;
 }
 
+// Classes G4..B1K of a view in one launch.
+template <typename E>
+static void sort_rows(galp_graph *g, const IterView &w, const int32_t *prev, int32_t *next) {
+    static const int kPerBlock[kSortRows] = {64, 32, 16, 8, 4, 4, 4, 4, 4};
+    RowsArgs<kSortRows> a{};
+    a.front = front_list(g, B_G4);
+    for (int b = 0; b < kSortRows; ++b) {
+        const BucketRange &r = w.cls[b];
+        const FrontList fl = front_list(g, b);
+        a.c[b] = RowsClass{g->d_vlist, r.v0, r.nv, nullptr, nullptr, nullptr, fl.list, fl.len, 1.f, kPerBlock[b]};
+    }
+    const int grid = rows_plan(g, w, a, B_W128);
+    if (!grid) return;
+    g->ended = may_end(g);   // the last kernel of the iteration
+    k_sort_rows<E><<<grid, kRowsThreads, 0, g->stream>>>(a, (const E *)w.off, w.nbr, prev, next, g->d_counter,
+                                                         g->d_err, iter_end_args(g, g->ended));
+}
+
 int launch_sort_class(galp_graph *g, int b) {
     const IterView w = full_view(g);
     const int32_t *prev = g->d_lab[g->cur];
@@ -1433,6 +1502,16 @@ template <typename E>
 static int sort_iteration(galp_graph *g, const IterView &w) {
     const int32_t *prev = g->d_lab[g->cur];
     int32_t *next = g->d_lab[g->cur ^ 1];
+    if (fused_rows(g)) {
+        for (int b = B_HUB; b >= B_B2K; --b) {
+            const int rc = sort_class<E>(g, w, b, prev, next);
+            if (rc != GALP_OK) return rc;
+        }
+        sort_rows<E>(g, w, prev, next);
+        const hipError_t ef = hipGetLastError();
+        return ef == hipSuccess ? GALP_OK
+                                : fail(g->ctx, GALP_EHIP, std::string("sort kernel launch: ") + hipGetErrorString(ef));
+    }
     if (!g->ooc && concurrent_classes(g)) return sort_iteration_concurrent<E>(g, w, prev, next);
     if (g->opts.policy == GALP_POLICY_LI) {
         // "load-imbalanced" ablation: every class <= 4096 through the
