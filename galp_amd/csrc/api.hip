@@ -396,15 +396,15 @@ static int upload_impl(galp_graph *g, const galp_csr_view *c) {
     // iteration) and, then, whether the graph is symmetric (the lists of
     // frontier.hip), on the rows in their input numbering.
     GALP_TRY(dev_fill_u32(g, (uint32_t *)g->d_stop, 1, 0u));   // the row check's flag, until the first init
-    const bool lists = !ooc && m >= kFrontMinEdges &&
+    const bool lists = m >= kFrontMinEdges &&
                        (g->opts.method == GALP_METHOD_HASH ? g->opts.variant == 1
-                                                           : g->opts.policy == GALP_POLICY_INCORE);
+                                                           : g->opts.policy != GALP_POLICY_LI);
     bool symmetric = false;
     auto check_rows = [&](const void *d_off, bool off64, const int32_t *d_nbr) {
         GALP_HIP(ctx, hipMemcpyAsync(g->h_pinned, g->d_stop, 4, hipMemcpyDeviceToHost, g->stream));
         GALP_HIP(ctx, hipStreamSynchronize(g->stream));
         g->rows_ascend = g->h_pinned[0] == 0;
-        return lists && g->rows_ascend ? dev_check_symmetric(g, d_off, off64, d_nbr, &symmetric) : GALP_OK;
+        return lists && g->rows_ascend ? dev_check_symmetric(g, d_off, off64, d_nbr, nullptr, &symmetric) : GALP_OK;
     };
     if (g->reorder && !ooc) {
         int64_t *d_off_old = nullptr;
@@ -475,6 +475,7 @@ static int upload_impl(galp_graph *g, const galp_csr_view *c) {
         std::vector<int64_t> hub_item0(hub_nparts.size() + 1, 0);
         for (size_t h = 0; h < hub_nparts.size(); ++h) hub_item0[h + 1] = hub_item0[h] + hub_nparts[h];
         GALP_TRY(ooc_setup(g, c, offi, perm, iperm, vlist, hub_vertices, hub_tile0, hub_item0));
+        if (lists && g->rows_ascend) GALP_TRY(ooc_check_symmetric(g, &symmetric));
     }
     if (g->opts.method == GALP_METHOD_SORT) GALP_TRY(sort_setup(g));
     GALP_HIP(ctx, hipStreamSynchronize(g->stream));
@@ -545,7 +546,7 @@ static int launch_iteration(galp_graph *g) {
     // overwrites the rebuild flag that batch_reset set
     g->ended = false;
     if (g->batch) GALP_TRY(launch_batch_lists(g));
-    if (!first && front_now(g)) GALP_TRY(launch_front(g));
+    if (!first && !g->ooc && front_now(g)) GALP_TRY(launch_front(g));
     switch (g->opts.method) {
     case GALP_METHOD_HASH:
         if (g->opts.dispatch == GALP_DISPATCH_LEARNED) {
@@ -813,7 +814,7 @@ GALP_API int galp_lp_step(galp_graph *g, galp_step_stats *st) {
     if (rc == GALP_OK) {
         g->h_pinned[9] = 0;
         hipError_t e = hipSuccess;
-        if (learned_now(g))
+        if (learned_now(g) && !(g->ooc && g->ooc->on_lists))   // lists: nothing was routed
             e = hipMemcpyAsync(g->h_pinned + 9, g->learn->d_plist_n + kCtrOverflow, 4, hipMemcpyDeviceToHost,
                                g->stream);
         if (e == hipSuccess) e = hipStreamSynchronize(g->stream);

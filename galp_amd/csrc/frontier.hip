@@ -48,7 +48,8 @@ __device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long x)
 }
 
 // ---------------------------------------------------------------------------
-// Symmetry of a CSR whose rows strictly ascend.  Order the vertices by
+// Symmetry of a CSR whose rows strictly ascend (by id, or by iperm[id] for
+// rows in the internal numbering).  Order the vertices by
 // (degree, id): every edge to a lower vertex is looked up in that vertex's
 // (shorter) row by binary search.  Rows hold no vertex twice, so the matches
 // are one to one, and the graph is symmetric when every downward edge has a
@@ -59,8 +60,8 @@ __device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long x)
 constexpr int kSymTile = 2048;
 template <typename E>
 __global__ void __launch_bounds__(256)
-k_check_symmetric(const E *__restrict__ off, const int32_t *__restrict__ nbr, int64_t n, int64_t m,
-                  int32_t *__restrict__ res) {
+k_check_symmetric(const E *__restrict__ off, const int32_t *__restrict__ nbr, const int32_t *__restrict__ iperm,
+                  int64_t n, int64_t m, int32_t *__restrict__ res) {
     __shared__ int64_t srow[2];
     __shared__ long long sbal[256 / kWave];
     long long balance = 0;
@@ -91,10 +92,12 @@ k_check_symmetric(const E *__restrict__ off, const int32_t *__restrict__ nbr, in
                 continue;
             }
             ++balance;
+            const int32_t key = iperm ? iperm[v] : (int32_t)v;
             int64_t lo = b, hi = b + du;   // first position of u's row holding an id >= v
             while (lo < hi) {
                 const int64_t mid = (lo + hi) >> 1;
-                if ((int64_t)nbr[mid] < v) lo = mid + 1;
+                const int32_t x = nbr[mid];
+                if ((iperm ? iperm[x] : x) < key) lo = mid + 1;
                 else hi = mid;
             }
             miss |= lo == b + du || (int64_t)nbr[lo] != v;
@@ -357,7 +360,8 @@ void front_free(galp_graph *g) {
 }
 
 // Whether a CSR on the device (rows strictly ascending) is symmetric.
-int dev_check_symmetric(galp_graph *g, const void *off, bool off64, const int32_t *nbr, bool *symmetric) {
+int dev_check_symmetric(galp_graph *g, const void *off, bool off64, const int32_t *nbr, const int32_t *iperm,
+                        bool *symmetric) {
     *symmetric = true;
     if (!g->m) return GALP_OK;
     int32_t *res = (int32_t *)g->d_counter;   // free until the first init; 16 bytes of it
@@ -365,8 +369,8 @@ int dev_check_symmetric(galp_graph *g, const void *off, bool off64, const int32_
     if (rc != GALP_OK) return rc;
     const int grid = (int)std::min<int64_t>((g->m + kSymTile - 1) / kSymTile,
                                             (int64_t)g->ctx->prop.multiProcessorCount * 8);
-    if (off64) k_check_symmetric<int64_t><<<grid, 256, 0, g->stream>>>((const int64_t *)off, nbr, g->n, g->m, res);
-    else k_check_symmetric<int32_t><<<grid, 256, 0, g->stream>>>((const int32_t *)off, nbr, g->n, g->m, res);
+    if (off64) k_check_symmetric<int64_t><<<grid, 256, 0, g->stream>>>((const int64_t *)off, nbr, iperm, g->n, g->m, res);
+    else k_check_symmetric<int32_t><<<grid, 256, 0, g->stream>>>((const int32_t *)off, nbr, iperm, g->n, g->m, res);
     if (hipGetLastError() != hipSuccess ||
         hipMemcpyAsync(g->h_pinned, res, 16, hipMemcpyDeviceToHost, g->stream) != hipSuccess ||
         hipStreamSynchronize(g->stream) != hipSuccess)
@@ -421,13 +425,14 @@ static void front_launch(galp_graph *g, FrontState *F) {
     const E *off = (const E *)g->d_off;
     const long long *updated = g->d_iter_counts + (g->iter - 1) % kMaxIters;
     const int cus = g->ctx->prop.multiProcessorCount;
-    const int64_t max_push = g->m / kFrontPushDiv;
+    const int64_t max_push = g->m / (g->ooc ? kFrontPushDivOoc : kFrontPushDiv);
+    const int32_t *nbr = g->ooc ? g->ooc->h_nbr : g->d_nbr;   // pinned host memory is mapped
     FrontSpans fs{};
     for (int b = 0; b < NUM_BUCKETS; ++b) fs.v0[b] = g->bucket[b].v0;
     const int grid_c = (int)std::min<int64_t>((g->n + kFrontThreads - 1) / kFrontThreads, cus);
     k_front_count<E><<<grid_c, kFrontThreads, 0, g->stream>>>(off, cur, old, g->n, updated, F->d_ctl, g->d_stop);
     const int grid_m = (int)std::min<int64_t>((g->n + kMarkThreads - 1) / kMarkThreads, (int64_t)cus * 8);
-    k_front_mark<E><<<grid_m, kMarkThreads, 0, g->stream>>>(off, g->d_nbr, cur, old, g->n, max_push, g->d_tile_hub,
+    k_front_mark<E><<<grid_m, kMarkThreads, 0, g->stream>>>(off, nbr, cur, old, g->n, max_push, g->d_tile_hub,
                                                            g->d_hub_tile0, g->d_hub_vid, g->nhub_tiles, updated,
                                                            (uint8_t *)F->d_mark, F->d_hub_sel, g->nhubs, F->d_ctl,
                                                            g->d_stop);

@@ -221,6 +221,9 @@ struct OocState {
     hipStream_t copy_stream = nullptr;
     hipEvent_t ev_copied[2] = {nullptr, nullptr}, ev_free[2] = {nullptr, nullptr};
     bool used[2] = {false, false};
+    int64_t resident[2] = {-1, -1};      // policy 2: the batch each buffer holds (or is being copied into it)
+    int64_t *h_ctl = nullptr;            // pinned: the frontier's control words, then the stop flag
+    bool on_lists = false;               // the last iteration walked the frontier's lists
     int32_t *d_last = nullptr;           // each row's last neighbour (-1: empty), for the first iteration; may be null
 };
 }  // namespace galp
@@ -241,6 +244,14 @@ static_assert(kFrontReady < kFrontCtl && kFrontCtl <= 64, "one wave clears the c
 // edges: 1741 us without, 1786 with; LFR-300K uploaded and run once, 6 M
 // edges: 5.7 ms without, 6.3 with; RMAT-20, 31 M: 5.6 and 3.8 ms).
 constexpr int64_t kFrontPushDiv = 8;
+// Out of core the rows of both steps are read over the host link where they
+// lie, in short pieces, so the lists have to be shorter to beat streaming all
+// batches (a step of 2.5 ms at RMAT-20, 31 M edges, 1.6 ms at LFR-1M, 20 M,
+// 0.6 ms at LFR-600K, 8.9 M).  Lists of x m edges took 5.0 x ms on RMAT-20,
+// 3.9 x on LFR-1M, 2.2 x on LFR-600K and 3.5 x on planted partitions of 17 M
+// edges: they meet the streamed step at x = 0.5, 0.41, 0.27 and 0.4.
+constexpr int64_t kFrontPushDivOoc = 16;
+constexpr int64_t kFrontListDivOoc = 4;
 constexpr int64_t kFrontMinEdges = (int64_t)1 << 23;
 struct FrontState {
     uint32_t *d_mem = nullptr;      // holds all but d_bytes
@@ -483,6 +494,9 @@ int ooc_setup(galp_graph *g, const galp_csr_view *c, const std::vector<int64_t> 
               const std::vector<int32_t> &hub_tile0, const std::vector<int64_t> &hub_item0);
 void ooc_free(galp_graph *g);
 int launch_ooc_iteration(galp_graph *g);
+// Whether an out-of-core graph (rows ascending) is symmetric, on a copy of its
+// rows in device memory; not answered (false) where the card has no ample room.
+int ooc_check_symmetric(galp_graph *g, bool *symmetric);
 // Streams every batch through learn_features_view once (learned dispatch set-up).
 int ooc_features(galp_graph *g);
 
@@ -525,11 +539,12 @@ int front_setup(galp_graph *g);
 void front_free(galp_graph *g);
 bool front_now(const galp_graph *g);   // the iteration being launched may use the lists
 int launch_front(galp_graph *g);
-int dev_check_symmetric(galp_graph *g, const void *off, bool off64, const int32_t *nbr, bool *symmetric);
+int dev_check_symmetric(galp_graph *g, const void *off, bool off64, const int32_t *nbr, const int32_t *iperm,
+                        bool *symmetric);
 inline FrontList front_list(const galp_graph *g, int b) {
     if (!front_now(g)) return FrontList{nullptr, 0, nullptr, nullptr};
     const FrontState *F = g->front;
-    return FrontList{F->d_ctl, g->m / 4 * 3, F->d_lists + g->bucket[b].v0, F->d_ctl + b};
+    return FrontList{F->d_ctl, g->ooc ? g->m / kFrontListDivOoc : g->m / 4 * 3, F->d_lists + g->bucket[b].v0, F->d_ctl + b};
 }
 inline FrontList front_hubs(const galp_graph *g) {   // list: a flag per hub; len: their tiles
     FrontList f = front_list(g, B_HUB);

@@ -18,6 +18,11 @@
 //   policy 2: copies on a second stream, double-buffered: the copy of batch
 //             b+1 overlaps the kernels of batch b; events order each buffer's
 //             reuse after the kernels that read it.
+// What bounds a streamed iteration is the link: all edges once, 50-57 GB/s.
+// Once few rows can still change (frontier.hip) the iteration reads those rows
+// over the link from where they lie, and nothing else.  RMAT-20 (31 M edges,
+// 10 iterations, batches of 2^22 edges): 27.4 ms streaming every iteration,
+// 10.5 with the lists, of which three streamed iterations take 7.
 
 #include <algorithm>
 #include <atomic>
@@ -60,6 +65,7 @@ static std::vector<int64_t> batch_boundaries(const std::vector<int64_t> &off, in
 void ooc_free(galp_graph *g) {
     OocState *O = g->ooc;
     if (!O) return;
+    if (O->copy_stream) (void)hipStreamSynchronize(O->copy_stream);   // batches loaded ahead and not used
     for (int k = 0; k < 2; ++k) {
         if (O->d_buf[k]) (void)hipFree(O->d_buf[k]);
         if (O->d_offb[k]) (void)hipFree(O->d_offb[k]);
@@ -68,6 +74,7 @@ void ooc_free(galp_graph *g) {
     }
     if (O->copy_stream) (void)hipStreamDestroy(O->copy_stream);
     if (O->d_last) (void)hipFree(O->d_last);
+    if (O->h_ctl) (void)hipHostFree(O->h_ctl);
     if (O->h_nbr) (void)hipHostFree(O->h_nbr);
     delete O;
     g->ooc = nullptr;
@@ -162,6 +169,10 @@ int ooc_setup(galp_graph *g, const galp_csr_view *c, const std::vector<int64_t> 
         w.i0 = hub_item0[(size_t)w.h0];
         w.i1 = hub_item0[(size_t)w.h1];
     }
+    if (hipHostMalloc((void **)&O->h_ctl, 8 * (kFrontCtl + 1), hipHostMallocDefault) != hipSuccess) {
+        O->h_ctl = nullptr;
+        return fail(g->ctx, GALP_ENOMEM, "out-of-core control words");
+    }
     O->bufcap = std::max<int64_t>(maxe, 1);
     const size_t esz = g->off64 ? 8 : 4;
     for (int k = 0; k < 2; ++k) {
@@ -188,6 +199,25 @@ int ooc_setup(galp_graph *g, const galp_csr_view *c, const std::vector<int64_t> 
     return GALP_OK;
 }
 
+// Policy 2: queues the copy of batch b into its buffer on the copy stream,
+// after the kernels that read the buffer, unless the buffer holds it.
+static int ooc_copy_async(galp_graph *g, int64_t b) {
+    OocState *O = g->ooc;
+    const int k = (int)(b & 1);
+    if (O->resident[k] == b) return GALP_OK;
+    if (O->used[k] && hipStreamWaitEvent(O->copy_stream, O->ev_free[k], 0) != hipSuccess)
+        return fail(g->ctx, GALP_EHIP, "out-of-core wait");
+    const int64_t e0 = O->e0[(size_t)b], ne = O->e1[(size_t)b] - e0;
+    O->resident[k] = -1;
+    if (ne && hipMemcpyAsync(O->d_buf[k], O->h_nbr + e0, 4 * (size_t)ne, hipMemcpyHostToDevice, O->copy_stream) !=
+                  hipSuccess)
+        return fail(g->ctx, GALP_EHIP, "out-of-core batch copy");
+    if (hipEventRecord(O->ev_copied[k], O->copy_stream) != hipSuccess)
+        return fail(g->ctx, GALP_EHIP, "out-of-core copy event");
+    O->resident[k] = b;
+    return GALP_OK;
+}
+
 template <typename E>
 static int ooc_round(galp_graph *g) {
     OocState *O = g->ooc;
@@ -197,20 +227,18 @@ static int ooc_round(galp_graph *g) {
         const int k = async ? (int)(b & 1) : 0;
         const int64_t e0 = O->e0[(size_t)b], ne = O->e1[(size_t)b] - e0;
         const int64_t lo = O->bbs[(size_t)b], hi = O->bbs[(size_t)b + 1];
-        hipStream_t cs = async ? O->copy_stream : g->stream;
-        if (async && O->used[k]) {   // the kernels that read this buffer are done
-            if (hipStreamWaitEvent(cs, O->ev_free[k], 0) != hipSuccess)
-                return fail(g->ctx, GALP_EHIP, "out-of-core wait");
-        }
-        PendingLaunch pl;
-        if (!async) prof_begin(g, "h2d", 4.0 * (double)ne, &pl);
-        if (ne && hipMemcpyAsync(O->d_buf[k], O->h_nbr + e0, 4 * (size_t)ne, hipMemcpyHostToDevice, cs) != hipSuccess)
-            return fail(g->ctx, GALP_EHIP, "out-of-core batch copy");
-        if (!async) prof_end(g, &pl);
         if (async) {
-            if (hipEventRecord(O->ev_copied[k], cs) != hipSuccess ||
-                hipStreamWaitEvent(g->stream, O->ev_copied[k], 0) != hipSuccess)
+            const int rc = ooc_copy_async(g, b);
+            if (rc != GALP_OK) return rc;
+            if (hipStreamWaitEvent(g->stream, O->ev_copied[k], 0) != hipSuccess)
                 return fail(g->ctx, GALP_EHIP, "out-of-core copy event");
+        } else {
+            PendingLaunch pl;
+            prof_begin(g, "h2d", 4.0 * (double)ne, &pl);
+            if (ne && hipMemcpyAsync(O->d_buf[k], O->h_nbr + e0, 4 * (size_t)ne, hipMemcpyHostToDevice, g->stream) !=
+                          hipSuccess)
+                return fail(g->ctx, GALP_EHIP, "out-of-core batch copy");
+            prof_end(g, &pl);
         }
         const int64_t nv = hi - lo + 1;
         const int grid = (int)std::max<int64_t>(1, std::min<int64_t>((nv + 255) / 256, 1024));
@@ -241,6 +269,10 @@ static int ooc_round(galp_graph *g) {
 int ooc_features(galp_graph *g) {
     OocState *O = g->ooc;
     const int64_t nb = (int64_t)O->views.size();
+    // buffer 0 is written on the graph's stream here: a batch loaded ahead into it comes first
+    if (O->resident[0] >= 0 && hipStreamWaitEvent(g->stream, O->ev_copied[0], 0) != hipSuccess)
+        return fail(g->ctx, GALP_EHIP, "out-of-core copy event");
+    O->resident[0] = -1;
     for (int64_t b = 0; b < nb; ++b) {
         const int64_t e0 = O->e0[(size_t)b], ne = O->e1[(size_t)b] - e0;
         const int64_t lo = O->bbs[(size_t)b], hi = O->bbs[(size_t)b + 1];
@@ -260,8 +292,58 @@ int ooc_features(galp_graph *g) {
     return GALP_OK;
 }
 
+int ooc_check_symmetric(galp_graph *g, bool *symmetric) {
+    *symmetric = false;
+    const size_t bytes = 4 * (size_t)g->m;
+    size_t fr = 0, tot = 0;
+    if (g->opts.mem_budget > 0 || hipMemGetInfo(&fr, &tot) != hipSuccess || fr / 4 < bytes) return GALP_OK;
+    int32_t *d_nbr = nullptr;
+    if (hipMalloc((void **)&d_nbr, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        return GALP_OK;
+    }
+    int rc = GALP_OK;
+    if (hipMemcpyAsync(d_nbr, g->ooc->h_nbr, bytes, hipMemcpyHostToDevice, g->stream) != hipSuccess)
+        rc = fail(g->ctx, GALP_EHIP, "out-of-core symmetry check: copy");
+    if (rc == GALP_OK) rc = dev_check_symmetric(g, g->d_off, g->off64, d_nbr, g->d_iperm, symmetric);
+    (void)hipStreamSynchronize(g->stream);
+    (void)hipFree(d_nbr);
+    return rc;
+}
+
+// An iteration over the rows that can still change (frontier.hip) reads them
+// from the pinned array where they lie, instead of streaming every batch.
+// Which it is, the host has to know before it queues the copies: one wait per
+// iteration, after the list kernels.
 int launch_ooc_iteration(galp_graph *g) {
-    if (!g->ooc) return fail(g->ctx, GALP_ESTATE, "internal: out-of-core state missing");
+    OocState *O = g->ooc;
+    if (!O) return fail(g->ctx, GALP_ESTATE, "internal: out-of-core state missing");
+    O->on_lists = false;
+    if (front_now(g)) {
+        const int rc = launch_front(g);
+        if (rc != GALP_OK) return rc;
+        // the first two batches load while the lists are built and read back;
+        // if the lists are walked they stay for the next streamed iteration
+        if (g->opts.policy == GALP_POLICY_OOC_ASYNC)
+            for (int64_t b = 0; b < 2 && b < (int64_t)O->views.size(); ++b) {
+                const int rcc = ooc_copy_async(g, b);
+                if (rcc != GALP_OK) return rcc;
+            }
+        int64_t *ctl = O->h_ctl;
+        if (hipMemcpyAsync(ctl, g->front->d_ctl, 8 * kFrontCtl, hipMemcpyDeviceToHost, g->stream) != hipSuccess ||
+            hipMemcpyAsync(ctl + kFrontCtl, g->d_stop, 4, hipMemcpyDeviceToHost, g->stream) != hipSuccess ||
+            hipStreamSynchronize(g->stream) != hipSuccess)
+            return fail(g->ctx, GALP_EHIP, "out-of-core list readback");
+        if ((int32_t)ctl[kFrontCtl] != 0) return GALP_OK;   // the run has stopped
+        int64_t edges = 0;
+        for (int b = 0; b < NUM_BUCKETS; ++b) edges += ctl[kFrontEdges + b];
+        if (ctl[kFrontReady] && edges <= front_list(g, 0).max_edges) {   // as front_lists_on
+            O->on_lists = true;
+            IterView w = full_view(g);
+            w.nbr = O->h_nbr;   // mapped
+            return g->opts.method == GALP_METHOD_HASH ? launch_hash_iteration(g, w) : launch_sort_iteration(g, w);
+        }
+    }
     return g->off64 ? ooc_round<int64_t>(g) : ooc_round<int32_t>(g);
 }
 

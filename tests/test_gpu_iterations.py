@@ -208,3 +208,28 @@ def test_changed_rows_only_batch(ctx, settling, method):
         iters = g.batch_iterations()
     assert iters[0] == len(counts)
     assert np.array_equal(labels[:n], final) and np.array_equal(labels[n:2 * n] - n, final)
+
+
+@pytest.mark.parametrize("opts", [dict(policy=_abi.POLICY_OOC_ASYNC, buffer_pow=20),
+                                  dict(policy=_abi.POLICY_OOC_SYNC, buffer_pow=21, reorder=0),
+                                  dict(policy=_abi.POLICY_OOC_ASYNC, buffer_pow=24),
+                                  dict(policy=_abi.POLICY_OOC_ASYNC, buffer_pow=20, method=_abi.METHOD_SORT),
+                                  dict(policy=_abi.POLICY_OOC_ASYNC, buffer_pow=20, dispatch=_abi.DISPATCH_LEARNED)],
+                         ids=["async", "sync-noreorder", "one-batch", "sort", "learned"])
+def test_changed_rows_only_out_of_core(ctx, settling, opts):
+    """Streamed iterations, then lists read from host memory, and from new
+    labels streamed again (the prefetched batches are still in place)."""
+    off, nbr, refs = settling
+    print(f"[lists] {opts}", flush=True)
+    with _abi.Graph(ctx, off, nbr, **opts) as g:
+        if "dispatch" in opts:
+            g.set_mlp(8, _abi.mlp_init(8, 4), 6.0)
+        for _ in range(2):
+            g.init()
+            for it, (ref, cnt) in enumerate(refs):
+                st = g.step()
+                assert st["updated"] == cnt, it + 1
+                assert np.array_equal(g.labels(), ref), it + 1
+        stop = next((i for i, (_, c) in enumerate(refs) if c <= (len(off) - 1) * 1e-5), len(refs) - 1)
+        labels, res = g.run(len(refs) + 3 if stop < len(refs) - 1 else len(refs))
+        assert res["iterations"] == stop + 1 and np.array_equal(labels, refs[stop][0])
