@@ -123,31 +123,67 @@ k_batch_lists(ClassSpans cs, const int32_t *__restrict__ vlist, const int32_t *_
 }
 
 // Per-vertex epilogue: frozen graphs keep prev; changes of the others are
-// counted per graph (wave-aggregated: consecutive ids mostly share a graph).
+// counted per graph.  Bound by the 12 bytes a vertex that it reads.  A block
+// takes a run of consecutive vertices, four per thread and load, and sums in
+// LDS for the kEpiGraphs graphs from its first vertex's on (ids of one graph
+// are consecutive, or any where the rows were renumbered: others go straight
+// to memory), so a graph gets one atomic a block.
+constexpr int kEpiGraphs = 64;
+constexpr int kEpiChunk = 256 * 4 * 4;
 __global__ void __launch_bounds__(256)
 k_batch_epilogue(const int32_t *__restrict__ prev, int32_t *__restrict__ next, const int32_t *__restrict__ gid,
                  const int32_t *__restrict__ gstop, unsigned long long *__restrict__ gcount, int64_t n,
                  const int32_t *__restrict__ stop) {
+    __shared__ uint32_t scnt[kEpiGraphs];
     if (*stop) return;
-    for (int64_t base = (int64_t)blockIdx.x * 256; base < n; base += (int64_t)gridDim.x * 256) {
-        const int64_t v = base + threadIdx.x;
-        bool pending = false;
-        int32_t k = 0;
-        if (v < n) {
-            k = gid[v];
-            const int32_t p = prev[v];
-            if (gstop[k]) next[v] = p;
-            else pending = next[v] != p;
+    for (int64_t c0 = (int64_t)blockIdx.x * kEpiChunk; c0 < n; c0 += (int64_t)gridDim.x * kEpiChunk) {
+        const int32_t k0 = gid[c0];
+        if (threadIdx.x < kEpiGraphs) scnt[threadIdx.x] = 0u;
+        __syncthreads();
+        for (int r = 0; r < kEpiChunk; r += 256 * 4) {
+            const int64_t v = c0 + r + 4 * (int64_t)threadIdx.x;
+            int32_t k[4] = {-1, -1, -1, -1}, p[4] = {0, 0, 0, 0}, q[4] = {0, 0, 0, 0};
+            if (v + 4 <= n) {
+                const int4 kk = *(const int4 *)(gid + v), pp = *(const int4 *)(prev + v), qq = *(const int4 *)(next + v);
+                k[0] = kk.x, k[1] = kk.y, k[2] = kk.z, k[3] = kk.w;
+                p[0] = pp.x, p[1] = pp.y, p[2] = pp.z, p[3] = pp.w;
+                q[0] = qq.x, q[1] = qq.y, q[2] = qq.z, q[3] = qq.w;
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (v + j < n) k[j] = gid[v + j], p[j] = prev[v + j], q[j] = next[v + j];
+            }
+            const int32_t kf = __builtin_amdgcn_readfirstlane(k[0]);
+            if (__ballot(k[0] != kf || k[1] != kf || k[2] != kf || k[3] != kf) == 0ull) {   // the wave in one graph
+                if (kf < 0) continue;
+                if (gstop[kf]) {
+                    *(int4 *)(next + v) = make_int4(p[0], p[1], p[2], p[3]);
+                    continue;
+                }
+                const uint32_t c = wave_reduce_u32((uint32_t)(p[0] != q[0]) + (uint32_t)(p[1] != q[1]) +
+                                                   (uint32_t)(p[2] != q[2]) + (uint32_t)(p[3] != q[3]),
+                                                   [](uint32_t a, uint32_t b) { return a + b; });
+                if (lane_id() == 0 && c) {
+                    if ((uint32_t)(kf - k0) < (uint32_t)kEpiGraphs) atomicAdd(&scnt[kf - k0], c);
+                    else atomicAdd(&gcount[kf], (unsigned long long)c);
+                }
+                continue;
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if (k[j] < 0) continue;
+                if (gstop[k[j]]) {
+                    next[v + j] = p[j];
+                } else if (p[j] != q[j]) {
+                    if ((uint32_t)(k[j] - k0) < (uint32_t)kEpiGraphs) atomicAdd(&scnt[k[j] - k0], 1u);
+                    else atomicAdd(&gcount[k[j]], 1ull);
+                }
+            }
         }
-        unsigned long long ball;
-        while ((ball = __ballot(pending)) != 0ull) {
-            const int leader = __ffsll((long long)ball) - 1;
-            const int32_t kl = __builtin_amdgcn_readlane(k, leader);
-            const bool mine = pending && k == kl;
-            const unsigned long long m = __ballot(mine);
-            if (lane_id() == leader) atomicAdd(&gcount[kl], (unsigned long long)__popcll(m));
-            pending = pending && !mine;
-        }
+        __syncthreads();
+        if (threadIdx.x < kEpiGraphs && scnt[threadIdx.x])
+            atomicAdd(&gcount[k0 + (int32_t)threadIdx.x], (unsigned long long)scnt[threadIdx.x]);
+        __syncthreads();
     }
 }
 
@@ -261,7 +297,7 @@ int launch_batch_end(galp_graph *g) {
     BatchState *B = g->batch;
     const int32_t *prev = g->d_lab[g->cur];
     int32_t *next = g->d_lab[g->cur ^ 1];
-    const int grid = (int)std::max<int64_t>(1, std::min<int64_t>((g->n + 255) / 256,
+    const int grid = (int)std::max<int64_t>(1, std::min<int64_t>((g->n + kEpiChunk - 1) / kEpiChunk,
                                                                  (int64_t)g->ctx->prop.multiProcessorCount * 8));
     k_batch_epilogue<<<grid, 256, 0, g->stream>>>(prev, next, B->d_gid, B->d_gstop, B->d_gcount, g->n, g->d_stop);
     k_batch_stop<<<1, 1024, 0, g->stream>>>(B->d_gcount, B->d_gn, B->d_gstop, B->d_giters, B->ngraphs, g->d_counter,
