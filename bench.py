@@ -515,7 +515,9 @@ def main():
                      "kernel_source_hash": src_hash, "traffic_stale": traffic_stale,
                      "avg_launch_us": round(dom_avg_s * 1e6, 2)},
         "iteration_roofline": {"alg_bytes": b_iter, "achieved_GBps": round(b_iter / per_iter_s / 1e9, 1),
-                               "frac": round(b_iter / per_iter_s / 1e9 / HBM_PEAK_GBS, 4)},
+                               "frac": round(b_iter / per_iter_s / 1e9 / HBM_PEAK_GBS, 4),
+                               "counts": "all m edges of every iteration, also those of rows that cannot change "
+                                         "and are not read; the kernel's roofline counts what it read"},
         **({"gather_ceiling": {
             "kernel": "k_gather_probe", "ms_per_pass": round(probe_ms, 4),
             "gathers_per_s": round(m / (probe_ms * 1e-3), 1), "alg_GBps": round(8.0 * m / (probe_ms * 1e-3) / 1e9, 1),

