@@ -233,3 +233,36 @@ def test_changed_rows_only_out_of_core(ctx, settling, opts):
         stop = next((i for i, (_, c) in enumerate(refs) if c <= (len(off) - 1) * 1e-5), len(refs) - 1)
         labels, res = g.run(len(refs) + 3 if stop < len(refs) - 1 else len(refs))
         assert res["iterations"] == stop + 1 and np.array_equal(labels, refs[stop][0])
+
+
+@pytest.mark.parametrize("reorder", [1, 0])
+@pytest.mark.parametrize("sizes", ["tiny", "edge"])
+def test_batch_counts_per_graph(ctx, sizes, reorder):
+    """Batches whose graphs end anywhere in a block's run of vertices: more
+    than 64 graphs in one run, graphs of one vertex, and graphs that end at,
+    before and behind a run's end (4096 vertices), the last one ragged."""
+    rng = np.random.default_rng(12)
+    ns = [int(x) for x in rng.integers(1, 90, 400)] if sizes == "tiny" else [4096, 4095, 1, 2, 8193, 1, 3]
+    rows, parts, vbase = [], [], [0]
+    for n in ns:
+        a, b = rng.integers(0, n, 3 * n), rng.integers(0, n, 3 * n)
+        nb = [set() for _ in range(n)]
+        for x, y in zip(a.tolist(), b.tolist()):
+            if x != y:
+                nb[x].add(y)
+                nb[y].add(x)
+        own = [sorted(s) for s in nb]
+        parts.append(csr(own))
+        rows += [[u + vbase[-1] for u in r] for r in own]
+        vbase.append(vbase[-1] + n)
+    off, nbr = csr(rows)
+    print(f"[batch] {sizes} reorder={reorder} graphs={len(ns)} n={len(rows)}", flush=True)
+    with _abi.Graph(ctx, off, nbr, reorder=reorder) as g:
+        g.set_batch(vbase)
+        for _ in range(2):
+            labels, _ = g.run(10)
+            iters = g.batch_iterations()
+            for k, (o, u) in enumerate(parts):
+                final, _, counts = oracle.lp_run(o, u, niter=10)
+                assert np.array_equal(labels[vbase[k]:vbase[k + 1]] - vbase[k], final), k
+                assert iters[k] == len(counts), k
