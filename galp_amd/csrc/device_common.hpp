@@ -331,13 +331,23 @@ __device__ __forceinline__ void end_iteration(unsigned long long *counter, const
     publish_ctl(e.host, e.stop, stopped, e.it + 1, (long long)c);
 }
 
+// Sets bits in the graph's error word (states the plan rules out: tables that
+// overflow, rows of the wrong class) and waits until they are there.  The last
+// block of an iteration publishes the word as soon as every block has taken
+// its ticket, and a block takes it behind a barrier that all its waves reach:
+// an atomic without a result could still be on its way then.
+__device__ __forceinline__ void raise_err(int32_t *err, int32_t bits) {
+    int32_t was = atomicOr(err, bits);
+    asm volatile("s_waitcnt vmcnt(0)" : "+v"(was)::"memory");
+}
+
 // block_count_add that ends the iteration when e.on: every block of the grid
 // calls it once, and the last one to come does the bookkeeping, which saves
 // the small graphs a launch per iteration (5 us between two short kernels).
 // Only atomics are ordered here, and each is complete when its result is back,
 // so no block fences or flushes a cache: the count goes to the block's shard,
 // then a ticket to the shard's line, and the last block of each shard takes
-// one of the whole grid.
+// one of the whole grid.  Errors are set by raise_err, which waits as well.
 template <int NW>
 __device__ __forceinline__ void block_count_end(uint32_t mine, unsigned long long *counter, uint32_t *scratch,
                                                 const IterEnd &e) {

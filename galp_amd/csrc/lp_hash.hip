@@ -138,7 +138,7 @@ __device__ __forceinline__ uint32_t lds_insert(uint32_t *skey, uint32_t L, bool 
         }
         h = (h + 1) & MASK;
     }
-    atomicOr(err, 1);
+    raise_err(err, 1);
     return h;
 }
 
@@ -269,7 +269,7 @@ struct LdsVertexPolicy {
             it.old = prev[it.v];
             it.valid = true;
             if (it.len > T * EPT) {   // never planned into this class
-                if (tid == 0) atomicOr(err, 8);
+                if (tid == 0) raise_err(err, 8);
                 it.len = 0;
             }
         }
@@ -984,7 +984,7 @@ k_hub_merge(const HubItem *__restrict__ items, int64_t ibase, int64_t nitems, co
         }
         if (full) {   // start the item over in twice as many rounds
             if (R >= (1u << kHubMergeCapBits)) {
-                if (threadIdx.x == 0) atomicOr(err, 1);
+                if (threadIdx.x == 0) raise_err(err, 1);
                 break;
             }
             R *= 2;

@@ -130,7 +130,7 @@ struct LdsBitonicPolicy {
             it.old = prev[it.v];
             it.valid = true;
             if (it.len > N) {   // never planned into this class
-                if (threadIdx.x == 0) atomicOr(err, 8);
+                if (threadIdx.x == 0) raise_err(err, 8);
                 it.len = 0;
             }
         }
@@ -307,7 +307,7 @@ struct RegBitonicPolicy {
             it.old = prev[it.v];
             it.valid = true;
             if (it.len > N) {   // never planned into this class
-                if (tid == 0) atomicOr(err, 8);
+                if (tid == 0) raise_err(err, 8);
                 it.len = 0;
             }
         }
@@ -639,7 +639,7 @@ struct LdsSortPolicy {
             it.old = prev[it.v];
             it.valid = true;
             if (it.len > N) {   // never planned into this class
-                if (threadIdx.x == 0) atomicOr(err, 8);
+                if (threadIdx.x == 0) raise_err(err, 8);
                 it.len = 0;
             }
         }
@@ -1214,7 +1214,7 @@ k_hs_merge(const int32_t *__restrict__ item_hub, const int32_t *__restrict__ ite
         }
         if (overflow) {   // start the item over in twice as many rounds
             if (R >= 4096u) {
-                if (tid == 0) atomicOr(err, 16);
+                if (tid == 0) raise_err(err, 16);
                 break;
             }
             R *= 2;
