@@ -138,7 +138,7 @@ static void dev_free_all(galp_graph *g) {
                     g->d_out, g->d_hub_vid, g->d_hub_nparts, g->d_item_hub, g->d_item_part, g->d_item_meta,
                     g->d_hub_best, g->d_merge_big, g->d_hub_tile0, g->d_hub_ntiles, g->d_tile_hub,
                     g->d_tile_idx_off,
-                    g->d_tile_idx, g->d_out_key, g->d_out_ent, g->d_counter, g->d_stop, g->d_iter_counts};
+                    g->d_tile_idx, g->d_out_key, g->d_out_ent, g->d_counter, g->d_iter_counts};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     if (g->h_pinned) (void)hipHostFree(g->h_pinned);
@@ -370,8 +370,17 @@ static int upload_impl(galp_graph *g, const galp_csr_view *c) {
     if (!ooc) GALP_TRY(dev_alloc(g, &g->d_nbr, m));
     GALP_TRY(dev_alloc(g, &g->d_lab[0], n));
     GALP_TRY(dev_alloc(g, &g->d_lab[1], n));
-    GALP_TRY(dev_alloc(g, &g->d_counter, kCountShards * kCountStride));
-    GALP_TRY(dev_alloc(g, &g->d_stop, kCtlWords));
+    // the shards of the change counter and the control words, one block; the
+    // memory budget counts the counter and the three words they stand for, not
+    // the 8 KB they are spread over
+    constexpr int64_t kShardWords = (int64_t)kCountShards * kCountStride;
+    if (hipMalloc((void **)&g->d_counter, 8 * kShardWords + 4 * kCtlWords) != hipSuccess) {
+        g->d_counter = nullptr;
+        (void)hipGetLastError();
+        return fail(ctx, GALP_ENOMEM, "control words");
+    }
+    g->device_bytes += 8 + 3 * 4;
+    g->d_stop = (int32_t *)(g->d_counter + kShardWords);
     g->d_iters_done = g->d_stop + 1;
     g->d_err = g->d_stop + 2;
     GALP_HIP(ctx, hipEventCreate(&g->ev[0]));

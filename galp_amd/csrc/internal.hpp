@@ -364,7 +364,7 @@ struct galp_graph {
     // kCtlWords words: the stop flag, the iterations done, an error set by a
     // kernel that hit an impossible state; every iteration's end writes them
     // and its change count (kCtlCount, 64-bit) to h_pinned as well
-    int32_t *d_stop = nullptr;
+    int32_t *d_stop = nullptr;           // behind d_counter's shards, in its allocation
     int32_t *d_iters_done = nullptr;     // d_stop + 1
     int32_t *d_err = nullptr;            // d_stop + 2
     long long *d_iter_counts = nullptr;  // kMaxIters
