@@ -383,7 +383,8 @@ int dev_check_symmetric(galp_graph *g, const void *off, bool off64, const int32_
     return GALP_OK;
 }
 
-// The lists' memory: n marks, n list entries.  Optional: a graph whose memory
+// The lists' memory: n marks, n list entries and, for per-kernel profiling, the
+// classes' bytes per iteration.  Optional: a graph whose memory
 // budget has no room for it, or that leaves less than 64 bytes a vertex free
 // on the card (what learned dispatch or a batch may still ask for), runs
 // every iteration over all rows.
@@ -399,8 +400,11 @@ int front_setup(galp_graph *g) {
     const int64_t words = (g->n + kFrontItems - 1) / kFrontItems;
     const int64_t total = 2 * kFrontCtl + words + g->n + g->nhubs + g->nhub_tiles;
     const std::string err = g->ctx->err;
-    if (dev_alloc(g, &F->d_mem, total) != GALP_OK) {
+    const int64_t before = g->device_bytes;
+    if (dev_alloc(g, &F->d_mem, total) != GALP_OK ||
+        (g->opts.profile && dev_alloc(g, &F->d_bytes, (int64_t)kMaxIters * NUM_BUCKETS) != GALP_OK)) {
         front_free(g);
+        g->device_bytes = before;
         g->ctx->err = err;   // doing without is no failure
         return GALP_OK;
     }
@@ -409,10 +413,6 @@ int front_setup(galp_graph *g) {
     F->d_lists = (int32_t *)(F->d_mark + words);
     F->d_hub_sel = F->d_lists + g->n;
     F->d_tiles = F->d_hub_sel + g->nhubs;
-    if (g->opts.profile) {
-        const int rc = dev_alloc(g, &F->d_bytes, (int64_t)kMaxIters * NUM_BUCKETS);
-        if (rc != GALP_OK) return rc;
-    }
     return dev_fill_u32(g, F->d_mem, total, 0u);
 }
 

@@ -159,6 +159,26 @@ def test_changed_rows_only(ctx, settling, opts):
             assert np.array_equal(g.labels(), lab), it
 
 
+@pytest.mark.parametrize("method", [_abi.METHOD_HASH, _abi.METHOD_SORT])
+def test_lists_need_no_budget(ctx, settling, method):
+    """A budget without room for all of the lists' memory, the last of which
+    holds a profiled graph's byte counts, runs every iteration over all rows."""
+    off, nbr, refs = settling
+    opts = dict(method=method, reorder=0, profile=1)   # renumbering peaks higher than the lists
+    with _abi.Graph(ctx, off, nbr, **opts) as g:
+        total = g.info()["device_bytes"]
+    with _abi.Graph(ctx, off, nbr, mem_budget=total, **opts) as g:
+        g.run(4, want_labels=False)
+        assert "front" in {k["name"] for k in g.profile()}
+    with _abi.Graph(ctx, off, nbr, mem_budget=total - 1, **opts) as g:
+        assert g.info()["device_bytes"] < total
+        g.init()
+        for it, (ref, cnt) in enumerate(refs[:8]):
+            assert g.step()["updated"] == cnt, it + 1
+            assert np.array_equal(g.labels(), ref), it + 1
+        assert "front" not in {k["name"] for k in g.profile()}
+
+
 @pytest.mark.parametrize("capture", [0, 1])
 def test_changed_rows_only_device_loop(ctx, settling, capture):
     off, nbr, refs = settling
