@@ -76,7 +76,8 @@ void prof_begin_dev(galp_graph *g, const char *name, const int64_t *dev_bytes, P
 }
 
 void prof_begin_class(galp_graph *g, const char *name, int b, double alg_bytes, PendingLaunch *pl) {
-    if (g->prof.on && front_now(g) && g->front->d_bytes)
+    // out of core a launch covers one batch, unless the iteration is on the lists
+    if (g->prof.on && front_now(g) && g->front->d_bytes && (!g->ooc || g->ooc->on_lists))
         prof_begin_dev(g, name, g->front->d_bytes + (int64_t)(g->iter % kMaxIters) * NUM_BUCKETS + b, pl);
     else prof_begin(g, name, alg_bytes, pl);
 }

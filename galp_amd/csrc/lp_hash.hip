@@ -1120,8 +1120,6 @@ template <typename E, int TT, int TM, bool LIST>
 static void launch_hubs(galp_graph *g, const IterView &w, const int32_t *prev, int32_t *next) {
     if (w.h1 <= w.h0) return;
     const int64_t nh = w.h1 - w.h0, nt = w.t1 - w.t0, ni = w.i1 - w.i0;
-    double hub_edges = 0.0;
-    if (w.h0 == 0 && w.h1 == g->nhubs) hub_edges = (double)g->bucket[B_HUB].edges;
     const int32_t *sel = learned_now(g) ? g->learn->d_hub_sel : nullptr;
     uint32_t *hdist = distinct_out(g) ? g->learn->d_hub_distinct : nullptr;
     const int64_t *nsel = sel ? g->learn->d_plist_n + kCtrPlainHubs : nullptr;
@@ -1129,7 +1127,7 @@ static void launch_hubs(galp_graph *g, const IterView &w, const int32_t *prev, i
     PendingLaunch pl;
     const FrontList fl = front_hubs(g);
     const int32_t *ftiles = fl.ctl ? g->front->d_tiles : nullptr;
-    prof_begin_class(g, "hub_tile", B_HUB, 8.0 * hub_edges, &pl);
+    prof_begin_class(g, "hub_tile", B_HUB, 8.0 * (double)w.cls[B_HUB].edges, &pl);
     // tiles [t0, t1): the pipeline starts at t0 + blockIdx.x, stops at t1
     k_hub_tile<TT, E, false><<<grid_for(g, nt, 3), TT, 0, g->stream>>>(
         (const E *)w.off, w.nbr, prev, g->d_tile_hub, g->d_hub_tile0, g->d_hub_vid, g->d_hub_nparts,

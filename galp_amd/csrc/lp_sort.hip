@@ -1370,11 +1370,9 @@ template <typename E>
 static int sort_hubs(galp_graph *g, const IterView &w, const int32_t *prev, int32_t *next, int tile_per_cu = 2,
                      int merge_per_cu = 1) {
     const int64_t nt = w.t1 - w.t0, ni = w.i1 - w.i0, nh = w.h1 - w.h0;
-    double hub_edges = 0.0;
-    if (w.h0 == 0 && w.h1 == g->nhubs) hub_edges = (double)g->bucket[B_HUB].edges;
     PendingLaunch pl;
     const FrontList fl = front_hubs(g);
-    prof_begin_class(g, "hub_sort", B_HUB, 8.0 * hub_edges, &pl);
+    prof_begin_class(g, "hub_sort", B_HUB, 8.0 * (double)w.cls[B_HUB].edges, &pl);
     k_hs_tile_wave<E><<<grid_for(g, (nt + kHsWaveT / kWave - 1) / (kHsWaveT / kWave), tile_per_cu), kHsWaveT, 0,
                         g->stream>>>((const E *)w.off, w.nbr, prev, g->d_tile_hub, g->d_hub_tile0, g->d_hub_vid,
                                      g->d_hub_nparts, g->d_tile_idx_off, w.t0, w.t1, g->d_out_key, g->d_out_ent,

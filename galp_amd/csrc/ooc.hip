@@ -157,7 +157,11 @@ int ooc_setup(galp_graph *g, const galp_csr_view *c, const std::vector<int64_t> 
             cut_list(lo, hi, r.v0, r.nv, k0, k1);
             w.cls[cl].v0 = k0;
             w.cls[cl].nv = k1 - k0;
-            w.cls[cl].edges = 0;
+            w.cls[cl].edges = 0;   // read by per-kernel profiling only
+            if (g->opts.profile && g->reorder) w.cls[cl].edges = offi[(size_t)k1] - offi[(size_t)k0];
+            else if (g->opts.profile)
+                for (int64_t k = k0; k < k1; ++k)
+                    w.cls[cl].edges += offi[(size_t)vlist[(size_t)k] + 1] - offi[(size_t)vlist[(size_t)k]];
         }
         // hubs: ascending ids in both numberings
         w.h0 = std::lower_bound(hub_vertices.begin(), hub_vertices.end(), (int32_t)lo) - hub_vertices.begin();

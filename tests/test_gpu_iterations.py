@@ -255,6 +255,39 @@ def test_changed_rows_only_out_of_core(ctx, settling, opts):
         assert res["iterations"] == stop + 1 and np.array_equal(labels, refs[stop][0])
 
 
+ROW_KERNELS = ("g4", "g8", "g16", "g32", "g64", "w128", "w256", "w512", "b1k", "b2k", "b4k", "hub_tile", "hub_sort")
+
+
+@pytest.mark.parametrize("opts", [dict(policy=_abi.POLICY_OOC_ASYNC, buffer_pow=20),
+                                  dict(policy=_abi.POLICY_OOC_SYNC, buffer_pow=21, reorder=0),
+                                  dict(policy=_abi.POLICY_OOC_ASYNC, buffer_pow=24),
+                                  dict(policy=_abi.POLICY_OOC_ASYNC, buffer_pow=20, method=_abi.METHOD_SORT)],
+                         ids=["async", "sync-noreorder", "one-batch", "sort"])
+def test_profiled_bytes_out_of_core(ctx, settling, opts):
+    """The row kernels of an iteration that streams every batch count each
+    edge once (id and label), each row's labels and offsets, and one offset
+    more per kernel; those of an iteration on the lists only what they walk."""
+    off, nbr, refs = settling
+    rows, m = int((np.diff(off) > 0).sum()), len(nbr)
+    with _abi.Graph(ctx, off, nbr, profile=1, **opts) as g:
+        g.init()
+        read = []
+        for it, (ref, cnt) in enumerate(refs):
+            g.profile_reset()
+            assert g.step()["updated"] == cnt, it + 1
+            prof = [k for k in g.profile() if k["name"] in ROW_KERNELS]
+            read.append(sum(k["alg_bytes"] for k in prof))
+            launches = sum(k["launches"] for k in prof)
+            if it in (1, 2):   # streamed: the second without the lists, the third after looking at them
+                hubs = g.info()["bucket_vertices"][11]
+                assert read[it] == 8 * m + 12 * (rows - hubs) + 4 * (launches - hub_launches(prof)), it + 1
+    assert 0 < read[-1] < 0.4 * read[2]
+
+
+def hub_launches(prof):
+    return sum(k["launches"] for k in prof if k["name"].startswith("hub_"))
+
+
 @pytest.mark.parametrize("reorder", [1, 0])
 @pytest.mark.parametrize("sizes", ["tiny", "edge"])
 def test_batch_counts_per_graph(ctx, sizes, reorder):
