@@ -50,7 +50,7 @@ int Profiler::find(const char *name) {
     return (int)aggs.size() - 1;
 }
 
-void prof_begin(galp_graph *g, const char *name, double alg_bytes, PendingLaunch *pl) {
+void prof_begin(galp_graph *g, const char *name, double alg_bytes, PendingLaunch *pl, hipStream_t on) {
     if (!g->prof.on) return;
     auto take = [&]() {
         hipEvent_t e;
@@ -67,7 +67,7 @@ void prof_begin(galp_graph *g, const char *name, double alg_bytes, PendingLaunch
     pl->dev_bytes = nullptr;
     pl->e0 = take();
     pl->e1 = take();
-    if (pl->e0) (void)hipEventRecord(pl->e0, g->stream);
+    if (pl->e0) (void)hipEventRecord(pl->e0, on ? on : g->stream);
 }
 
 void prof_begin_dev(galp_graph *g, const char *name, const int64_t *dev_bytes, PendingLaunch *pl) {
@@ -82,9 +82,9 @@ void prof_begin_class(galp_graph *g, const char *name, int b, double alg_bytes, 
     else prof_begin(g, name, alg_bytes, pl);
 }
 
-void prof_end(galp_graph *g, PendingLaunch *pl) {
+void prof_end(galp_graph *g, PendingLaunch *pl, hipStream_t on) {
     if (!g->prof.on) return;
-    if (pl->e1) (void)hipEventRecord(pl->e1, g->stream);
+    if (pl->e1) (void)hipEventRecord(pl->e1, on ? on : g->stream);
     g->prof.pending.push_back(*pl);
 }
 
@@ -635,6 +635,7 @@ static int queue_init(galp_graph *g) {
     GALP_TRY(dev_init_labels(g));
     GALP_TRY(learn_reset_iteration(g));
     GALP_TRY(batch_reset(g));
+    ooc_forget_batches(g);
     g->cur = 0;
     g->iter = 0;
     g->identity = true;
@@ -790,6 +791,7 @@ GALP_API int galp_lp_set_labels(galp_graph *g, const int32_t *host_labels) {
     GALP_TRY(dev_init_labels(g));   // resets the control words
     GALP_TRY(learn_reset_iteration(g));
     GALP_TRY(batch_reset(g));
+    ooc_forget_batches(g);
     if (g->n) {
         int32_t *dst = g->d_lab[0];
         if (g->reorder) {
@@ -821,6 +823,7 @@ GALP_API int galp_lp_step(galp_graph *g, galp_step_stats *st) {
         rc = launch_iteration(g);
         (void)hipEventRecord(g->ev[1], g->stream);
     }
+    if (rc == GALP_OK) rc = ooc_finish_copies(g);
     if (rc == GALP_OK) {
         g->h_pinned[9] = 0;
         hipError_t e = hipSuccess;
@@ -908,6 +911,7 @@ GALP_API int galp_lp_run(galp_graph *g, int32_t niter, int32_t verbose, int32_t 
             }
         }
         (void)hipEventRecord(g->ev[1], g->stream);
+        if (rc == GALP_OK) rc = ooc_finish_copies(g);
         if (rc == GALP_OK) {
             hipError_t e = hipSuccess;
             if (labels_out && g->reorder && g->n) {   // queued behind the run: one wait for both

@@ -221,7 +221,7 @@ struct OocState {
     hipStream_t copy_stream = nullptr;
     hipEvent_t ev_copied[2] = {nullptr, nullptr}, ev_free[2] = {nullptr, nullptr};
     bool used[2] = {false, false};
-    int64_t resident[2] = {-1, -1};      // policy 2: the batch each buffer holds (or is being copied into it)
+    int64_t resident[2] = {-1, -1};      // policy 2: the batch each buffer holds (or is being copied into it) in this run
     int64_t *h_ctl = nullptr;            // pinned: the frontier's control words, then the stop flag
     bool on_lists = false;               // the last iteration walked the frontier's lists
     int32_t *d_last = nullptr;           // each row's last neighbour (-1: empty), for the first iteration; may be null
@@ -494,6 +494,13 @@ int ooc_setup(galp_graph *g, const galp_csr_view *c, const std::vector<int64_t> 
               const std::vector<int32_t> &hub_tile0, const std::vector<int64_t> &hub_item0);
 void ooc_free(galp_graph *g);
 int launch_ooc_iteration(galp_graph *g);
+// Policy 2: work queued on the graph's stream from here on follows every batch
+// copy queued so far, used or not; each call that steps ends with it, so no
+// copy outlives the call.
+int ooc_finish_copies(galp_graph *g);
+// The next streamed iteration copies every batch, also one that a buffer holds:
+// a run brings its own batches in, like the first one.
+void ooc_forget_batches(galp_graph *g);
 // Whether an out-of-core graph (rows ascending) is symmetric, on a copy of its
 // rows in device memory; not answered (false) where the card has no ample room.
 int ooc_check_symmetric(galp_graph *g, bool *symmetric);
@@ -591,9 +598,10 @@ int dev_map_labels(galp_graph *g, const int32_t *lab, int32_t *out);
 int dev_map_labels_done(galp_graph *g, int cur0, int32_t *out);   // after *d_iters_done iterations from d_lab[cur0]
 int dev_unmap_labels(galp_graph *g, const int32_t *in, int32_t *lab);
 
-// Profiling helpers (api.hip): bracket a launch with events when enabled.
-void prof_begin(galp_graph *g, const char *name, double alg_bytes, PendingLaunch *pl);
-void prof_end(galp_graph *g, PendingLaunch *pl);
+// Profiling helpers (api.hip): bracket a launch with events when enabled, on
+// the graph's stream unless another is named.
+void prof_begin(galp_graph *g, const char *name, double alg_bytes, PendingLaunch *pl, hipStream_t on = nullptr);
+void prof_end(galp_graph *g, PendingLaunch *pl, hipStream_t on = nullptr);
 // As prof_begin, with the launch's algorithmic bytes read from the device
 // when the timings are collected.
 void prof_begin_dev(galp_graph *g, const char *name, const int64_t *dev_bytes, PendingLaunch *pl);

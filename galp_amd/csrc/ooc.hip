@@ -65,7 +65,7 @@ static std::vector<int64_t> batch_boundaries(const std::vector<int64_t> &off, in
 void ooc_free(galp_graph *g) {
     OocState *O = g->ooc;
     if (!O) return;
-    if (O->copy_stream) (void)hipStreamSynchronize(O->copy_stream);   // batches loaded ahead and not used
+    if (O->copy_stream) (void)hipStreamSynchronize(O->copy_stream);   // copies of a call that failed
     for (int k = 0; k < 2; ++k) {
         if (O->d_buf[k]) (void)hipFree(O->d_buf[k]);
         if (O->d_offb[k]) (void)hipFree(O->d_offb[k]);
@@ -203,6 +203,19 @@ int ooc_setup(galp_graph *g, const galp_csr_view *c, const std::vector<int64_t> 
     return GALP_OK;
 }
 
+int ooc_finish_copies(galp_graph *g) {
+    OocState *O = g->ooc;
+    if (!O || !O->copy_stream) return GALP_OK;
+    for (int k = 0; k < 2; ++k)
+        if (hipStreamWaitEvent(g->stream, O->ev_copied[k], 0) != hipSuccess)
+            return fail(g->ctx, GALP_EHIP, "out-of-core copy event");
+    return GALP_OK;
+}
+
+void ooc_forget_batches(galp_graph *g) {
+    if (g->ooc) g->ooc->resident[0] = g->ooc->resident[1] = -1;
+}
+
 // Policy 2: queues the copy of batch b into its buffer on the copy stream,
 // after the kernels that read the buffer, unless the buffer holds it.
 static int ooc_copy_async(galp_graph *g, int64_t b) {
@@ -213,9 +226,12 @@ static int ooc_copy_async(galp_graph *g, int64_t b) {
         return fail(g->ctx, GALP_EHIP, "out-of-core wait");
     const int64_t e0 = O->e0[(size_t)b], ne = O->e1[(size_t)b] - e0;
     O->resident[k] = -1;
+    PendingLaunch pl;
+    prof_begin(g, "h2d", 4.0 * (double)ne, &pl, O->copy_stream);
     if (ne && hipMemcpyAsync(O->d_buf[k], O->h_nbr + e0, 4 * (size_t)ne, hipMemcpyHostToDevice, O->copy_stream) !=
                   hipSuccess)
         return fail(g->ctx, GALP_EHIP, "out-of-core batch copy");
+    prof_end(g, &pl, O->copy_stream);
     if (hipEventRecord(O->ev_copied[k], O->copy_stream) != hipSuccess)
         return fail(g->ctx, GALP_EHIP, "out-of-core copy event");
     O->resident[k] = b;
@@ -274,8 +290,7 @@ int ooc_features(galp_graph *g) {
     OocState *O = g->ooc;
     const int64_t nb = (int64_t)O->views.size();
     // buffer 0 is written on the graph's stream here: a batch loaded ahead into it comes first
-    if (O->resident[0] >= 0 && hipStreamWaitEvent(g->stream, O->ev_copied[0], 0) != hipSuccess)
-        return fail(g->ctx, GALP_EHIP, "out-of-core copy event");
+    if (const int rc = ooc_finish_copies(g); rc != GALP_OK) return rc;
     O->resident[0] = -1;
     for (int64_t b = 0; b < nb; ++b) {
         const int64_t e0 = O->e0[(size_t)b], ne = O->e1[(size_t)b] - e0;
@@ -327,7 +342,7 @@ int launch_ooc_iteration(galp_graph *g) {
         const int rc = launch_front(g);
         if (rc != GALP_OK) return rc;
         // the first two batches load while the lists are built and read back;
-        // if the lists are walked they stay for the next streamed iteration
+        // if the lists are walked they stay for the run's next streamed iteration
         if (g->opts.policy == GALP_POLICY_OOC_ASYNC)
             for (int64_t b = 0; b < 2 && b < (int64_t)O->views.size(); ++b) {
                 const int rcc = ooc_copy_async(g, b);

@@ -284,6 +284,38 @@ def test_profiled_bytes_out_of_core(ctx, settling, opts):
     assert 0 < read[-1] < 0.4 * read[2]
 
 
+@pytest.mark.parametrize("pow2", [20, 24], ids=["nine-batches", "one-batch"])
+def test_out_of_core_copies(ctx, settling, pow2):
+    """Every run copies its batches itself: what an earlier run left in the
+    buffers, or copied ahead and did not use, is not counted on.  The copies
+    are complete when the call returns (else they would not be counted)."""
+    off, nbr, refs = settling
+    m = len(nbr)
+
+    def copied(g):
+        b = sum(k["alg_bytes"] for k in g.profile() if k["name"] == "h2d")
+        g.profile_reset()
+        return b
+
+    with _abi.Graph(ctx, off, nbr, policy=_abi.POLICY_OOC_ASYNC, buffer_pow=pow2, profile=1) as g:
+        per_run = []
+        for _ in range(3):
+            g.run(len(refs), want_labels=False)
+            per_run.append(copied(g))
+        print(f"[ooc] copied per run {per_run}, m={m}", flush=True)
+        assert per_run[0] == per_run[1] == per_run[2]
+        assert per_run[0] == 4 * m if pow2 == 24 else per_run[0] >= 8 * m
+        for _ in range(2):
+            g.set_labels(refs[-1][0])
+            ref, cnt = oracle.lp_iterate(off, nbr, refs[-1][0])
+            assert g.step()["updated"] == cnt and copied(g) == 4 * m
+            assert np.array_equal(g.labels(), ref)
+        for _ in range(2):
+            g.init()
+            for it in range(2):   # the first iteration's closed form needs no batch
+                assert g.step()["updated"] == refs[it][1] and copied(g) == 4 * m * it
+
+
 def hub_launches(prof):
     return sum(k["launches"] for k in prof if k["name"].startswith("hub_"))
 
