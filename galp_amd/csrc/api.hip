@@ -618,7 +618,7 @@ static int run_captured(galp_graph *g, int niter) {
         g->gexec_niter = niter;
     }
     GALP_HIP(g->ctx, hipGraphLaunch(g->gexec, g->stream));
-    if (g->learn && (niter & 1)) g->learn->dcur ^= 1;   // as the eager loop leaves it
+    if (g->learn && g->learn->log_cap && (niter & 1)) g->learn->dcur ^= 1;   // as the eager loop leaves it
     return GALP_OK;
 }
 

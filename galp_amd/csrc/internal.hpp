@@ -157,8 +157,8 @@ struct LearnState {
     int H = 0;                         // hidden width of the attached MLP (0: none)
     float *d_params = nullptr;
     float *d_fdeg = nullptr, *d_fmean = nullptr, *d_fmax = nullptr;   // raw static features
-    int32_t *d_dist[2] = {nullptr, nullptr};   // distinct labels per vertex, double-buffered
-    int dcur = 0;                      // d_dist[dcur]: previous iteration's counts
+    int32_t *d_dist[2] = {nullptr, nullptr};   // distinct labels per vertex
+    int dcur = 0;                      // d_dist[dcur]: previous iteration's counts; alternates while samples are logged
     int64_t big_v0 = 0, big_n = 0;     // big vertex i: vlist ? vlist[big_v0+i] : big_v0+i
     int64_t front_n = 0;               // big vertices the last dispatch routed (an out-of-core batch's share)
     float cand_thresh = 4.0f;          // predicted distinct labels routed to candidates
@@ -523,15 +523,20 @@ inline bool learned_now(const galp_graph *g) {
 
 // Where this iteration's paths record each big row's distinct-label count:
 // the next iteration's dispatch input and the logged training target, so
-// nowhere (null) when the next iteration routes by the degree classes alone
-// and nothing is logged.
+// nowhere when neither wants it.  An iteration on the lists of frontier.hip
+// leaves the counts of the rows it does not walk as they are, which they still
+// are: so the counts stay in one buffer (two only while samples are logged,
+// when no iteration takes the lists), and where a graph has lists they are
+// recorded in every iteration before the last one that routes.
 inline int32_t *distinct_out(const galp_graph *g) {
     const LearnState *L = g->learn;
     if (!L) return nullptr;
+    if (L->log_cap) return L->d_dist[L->dcur ^ 1];
     const int i = g->iter + 1 < 63 ? g->iter + 1 : 63;
-    const bool next_learned = g->opts.dispatch == GALP_DISPATCH_LEARNED &&
-                              (g->ooc || ((g->learn_mask >> i) & 1ull) != 0);
-    return next_learned || L->log_cap ? L->d_dist[L->dcur ^ 1] : nullptr;
+    const uint64_t later = g->learn_mask >> i;   // bit 0: the next iteration
+    const bool wanted = g->opts.dispatch == GALP_DISPATCH_LEARNED &&
+                        (g->ooc || (g->front ? later != 0 : (later & 1ull) != 0));
+    return wanted ? L->d_dist[L->dcur] : nullptr;
 }
 
 // Drops the captured iteration loop after a change to what it launches.

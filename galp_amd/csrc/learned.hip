@@ -1116,11 +1116,11 @@ int launch_learned_front_batch(galp_graph *g, const IterView &w, int64_t lo, int
                     : learned_front<int32_t>(g, (const int32_t *)w.off, w.nbr, lo, nv, lo == 0, true);
 }
 
-// After the iteration's LP kernels: log samples (if enabled), swap counts.
+// After the iteration's LP kernels, if samples are logged: log them, swap counts.
 int learn_after_iteration(galp_graph *g) {
     LearnState *L = g->learn;
-    if (!L) return GALP_OK;
-    if (L->log_cap && L->big_n) {
+    if (!L || !L->log_cap) return GALP_OK;
+    if (L->big_n) {
         k_log_samples<int32_t><<<grid_cap(g, (L->big_n + 255) / 256, 8), 256, 0, g->stream>>>(
             g->d_vlist, L->big_v0, L->big_n, L->d_fdeg, L->d_fmean, L->d_fmax, L->d_dist[L->dcur],
             L->d_dist[L->dcur ^ 1], L->d_log_x, L->d_log_y, L->log_cap, L->d_log_n, g->d_stop);

@@ -216,6 +216,40 @@ def test_changed_rows_only_learned(ctx, settling, net):
             assert np.array_equal(g.labels(), ref), it + 1
 
 
+@pytest.mark.parametrize("mask", [None, 0b1111111], ids=["every", "to-7"])
+def test_counts_of_rows_left_out(ctx, mask):
+    """Distinct-label counts, the network's input: samples logged after
+    iterations on the lists hold each row's count of the iteration before,
+    also for rows that were left out of it."""
+    off, nbr = _abi.gen_lfr(400000, avg_deg=24.0, max_deg=1500, mu=0.3, seed=9)
+    assert len(nbr) >= 1 << 23
+    big = np.nonzero(np.diff(off) > 64)[0]
+    labs = [np.arange(len(off) - 1, dtype=np.int32)]
+    for _ in range(9):
+        labs.append(oracle.lp_iterate(off, nbr, labs[-1])[0])
+
+    def counts(lab):
+        return np.array([len(np.unique(lab[nbr[off[v]:off[v + 1]]])) for v in big])
+
+    with _abi.Graph(ctx, off, nbr, dispatch=_abi.DISPATCH_LEARNED) as g:
+        g.set_mlp(8, _abi.mlp_init(8, 3), 6.0)
+        if mask is not None:   # the last two by the classes alone, which need and keep no counts
+            g.set_learned_iterations(mask | (0b11 << 8))
+        g.init()
+        for it in range(8):
+            g.step()
+        assert np.array_equal(g.labels(), labs[8])
+        g.log_enable(len(big))
+        g.step()
+        x, y = g.log_read()
+        assert np.array_equal(g.labels(), labs[9])
+    before, now = (np.rint(np.exp2(z.astype(np.float64)) - 1).astype(np.int64) for z in (x[:, 3], y))
+    want = np.stack([np.diff(off)[big], counts(labs[7]), counts(labs[8])], 1)
+    got = np.stack([np.rint(np.exp2(x[:, 0].astype(np.float64)) - 1).astype(np.int64), before, now], 1)
+    assert len(got) == len(big)
+    assert np.array_equal(got[np.lexsort(got.T)], want[np.lexsort(want.T)])
+
+
 @pytest.mark.parametrize("method", [_abi.METHOD_HASH, _abi.METHOD_SORT])
 def test_changed_rows_only_batch(ctx, settling, method):
     """The two copies as two graphs of a batch: each stops by its own rule."""
