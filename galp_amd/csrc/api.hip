@@ -827,7 +827,7 @@ GALP_API int galp_lp_step(galp_graph *g, galp_step_stats *st) {
     if (rc == GALP_OK) {
         g->h_pinned[9] = 0;
         hipError_t e = hipSuccess;
-        if (learned_now(g) && !(g->ooc && g->ooc->on_lists))   // lists: nothing was routed
+        if (learned_now(g))
             e = hipMemcpyAsync(g->h_pinned + 9, g->learn->d_plist_n + kCtrOverflow, 4, hipMemcpyDeviceToHost,
                                g->stream);
         if (e == hipSuccess) e = hipStreamSynchronize(g->stream);

@@ -585,6 +585,8 @@ int launch_learned_merge(galp_graph *g);
 // Out-of-core: the dispatch and candidate path of one batch (vertices
 // [lo, hi), the batch's rebased offsets and neighbour buffer in w).
 int launch_learned_front_batch(galp_graph *g, const IterView &w, int64_t lo, int64_t hi);
+// Out-of-core, an iteration on the lists of frontier.hip: clears the counters.
+int learn_route_nothing(galp_graph *g);
 // Static features of the big vertices among [lo, hi) from a batch's rows.
 int learn_features_view(galp_graph *g, const void *offrow, const int32_t *nbr, int64_t lo, int64_t hi);
 int learn_after_iteration(galp_graph *g);

@@ -1083,6 +1083,12 @@ static int learned_front(galp_graph *g, const E *off, const int32_t *nbr, int64_
     return hipGetLastError() == hipSuccess ? GALP_OK : fail(g->ctx, GALP_EHIP, "learned dispatch launch failed");
 }
 
+int learn_route_nothing(galp_graph *g) {
+    LearnState *L = g->learn;
+    k_reset_front<<<1, 64, 0, g->stream>>>(L->d_plist_n, L->d_cand_bytes + g->iter % kMaxIters, 1);
+    return hipGetLastError() == hipSuccess ? GALP_OK : fail(g->ctx, GALP_EHIP, "reset launch failed");
+}
+
 int launch_learned_front(galp_graph *g, bool merge) {
     LearnState *L = g->learn;
     return g->off64

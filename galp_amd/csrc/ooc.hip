@@ -358,6 +358,8 @@ int launch_ooc_iteration(galp_graph *g) {
         for (int b = 0; b < NUM_BUCKETS; ++b) edges += ctl[kFrontEdges + b];
         if (ctl[kFrontReady] && edges <= front_list(g, 0).max_edges) {   // as front_lists_on
             O->on_lists = true;
+            if (learned_now(g))
+                if (const int rcl = learn_route_nothing(g); rcl != GALP_OK) return rcl;
             IterView w = full_view(g);
             w.nbr = O->h_nbr;   // mapped
             return g->opts.method == GALP_METHOD_HASH ? launch_hash_iteration(g, w) : launch_sort_iteration(g, w);

@@ -247,8 +247,10 @@ GALP_API int galp_graph_log_read(galp_graph *g, float *x, float *y, int64_t max,
 /* Raw static features per vertex (original numbering): degree, mean and max
  * neighbour degree, computed for vertices of degree > 64 (0 otherwise). */
 GALP_API int galp_graph_features(galp_graph *g, float *deg, float *mean, float *mx);
-/* Counters of the last iteration routed by the network: [0..12) class list
- * sizes, [12..16) candidate tiles per length class (<= 128, 256, 512, 1024
+/* Counters of the last iteration that learned dispatch was in charge of,
+ * zeros where it routed nothing (the first iteration from labels[i] = i in
+ * closed form, iterations over the rows that can still change): [0..12) class
+ * list sizes, [12..16) candidate tiles per length class (<= 128, 256, 512, 1024
  * edges), [16] candidate overflows, [17] vertices routed to candidates,
  * [18] hubs left to the plain hub path, [19] multi-tile rows routed to
  * candidates, [20..32) sizes of the classes' high-distinct lists ([31], the

@@ -216,6 +216,30 @@ def test_changed_rows_only_learned(ctx, settling, net):
             assert np.array_equal(g.labels(), ref), it + 1
 
 
+@pytest.mark.parametrize("opts", [dict(), dict(reorder=0), dict(policy=_abi.POLICY_OOC_ASYNC, buffer_pow=20)],
+                         ids=["hash", "noreorder", "ooc"])
+def test_dispatch_counters_over_lists(ctx, settling, opts):
+    """The dispatch counters after an iteration are its own: every big row
+    where the network routed it, nothing after the closed form or the lists."""
+    off, nbr, refs = settling
+    deg = np.diff(off)
+    routed = int(((deg > 64) & (deg <= (1024 if "policy" in opts else 1 << 30))).sum())   # one tile out of core
+    with _abi.Graph(ctx, off, nbr, dispatch=_abi.DISPATCH_LEARNED, **opts) as g:
+        g.set_mlp(8, np.zeros(_abi.mlp_num_params(8), np.float32), 6.0)   # predicts 0 labels: every big row
+        for _ in range(2):
+            g.init()
+            for it, (ref, cnt) in enumerate(refs):
+                st = g.step()
+                assert st["updated"] == cnt
+                ds = g.dispatch_stats()
+                assert st["overflowed"] == ds[_abi.DS_OVERFLOW], it + 1
+                if it in (1, 2):   # too many changes for the lists
+                    assert ds[_abi.DS_CAND_VERTS] == routed, it + 1
+                elif it == 0 or it == len(refs) - 1:
+                    assert not ds.any(), it + 1
+            assert np.array_equal(g.labels(), refs[-1][0])
+
+
 @pytest.mark.parametrize("mask", [None, 0b1111111], ids=["every", "to-7"])
 def test_counts_of_rows_left_out(ctx, mask):
     """Distinct-label counts, the network's input: samples logged after
