@@ -143,6 +143,7 @@ def lib():
         "galp_graph_autotune": (ctypes.c_int, [vp, i32, ctypes.c_char_p, vp]),
         "galp_graph_set_learned_iterations": (ctypes.c_int, [vp, ctypes.c_uint64]),
         "galp_graph_set_tuning": (ctypes.c_int, [vp, vp]),
+        "galp_graph_row_launches": (ctypes.c_int, [vp, vp]),
         "galp_batch_iterations": (ctypes.c_int, [vp, vp]),
     }
     for name, (res, args) in sig.items():
@@ -371,6 +372,7 @@ class Graph:
         self.ctx.check(lib().galp_graph_autotune(self.h, reps, os.fsencode(cache_path) if cache_path else None,
                                                  out.ctypes.data))
         self.tuned_streams = int(out[12])   # 1 or 3 streams per iteration (0: not timed)
+        self.tuned_class_kernels = bool(out[15])   # a kernel per class where the size rule has one launch
         # learned dispatch: iterations the judge left to the network
         self.learned_iterations = int(np.uint32(out[13])) | (int(np.uint32(out[14])) << 32)
         return out[:12]
@@ -382,6 +384,13 @@ class Graph:
         o = np.ascontiguousarray(options, np.int32)
         assert len(o) == 12
         self.ctx.check(lib().galp_graph_set_tuning(self.h, o.ctypes.data))
+
+    def row_launches(self):
+        """How the next iteration over every row launches its classes: 0 one
+        launch for the row classes, 1 or 3 a kernel per class on that many streams."""
+        mode = ctypes.c_int32()
+        self.ctx.check(lib().galp_graph_row_launches(self.h, ctypes.byref(mode)))
+        return mode.value
 
     # ---- batched runs ------------------------------------------------------
     def set_batch(self, vbase):

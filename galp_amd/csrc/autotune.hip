@@ -16,9 +16,15 @@
 // where an iteration may run its class kernels on three streams, whole runs
 // are timed on one stream and on three; the choice by size stays unless the
 // other is more than 3 % faster (the overlap helps while the label array
-// stays in the Infinity Cache and can hurt once it does not).  Choices can
-// be cached in a text file, one line per class (class 12 = the stream
-// choice, 1 or 3):
+// stays in the Infinity Cache and can hurt once it does not).  A graph small
+// enough to run its row classes in one launch (rows_fused.hpp) is then timed
+// that way against the class kernels as tuned: the launch wins on skewed
+// graphs (RMAT, LFR: 1.1 to 1.6 times the class kernels' speed at 10 to 31 M
+// edges) and loses where nearly all rows are of one class, which the launch
+// runs at the register and LDS need of the largest (planted partitions of 44
+// edges a row, 17 and 31 M edges: 0.85 and 0.94 times).  Choices can be
+// cached in a text file, one line per class (class 12 = the stream choice, 1
+// or 3; class 13 = the row classes in one launch, 0, or a kernel each, 1):
 //   <arch> <method> <class> <log2 vertices> <log2 edges> <option>
 // and are reused for a graph whose class has the same arch, method and sizes.
 // Under learned dispatch, in core, the tuner then judges the network against
@@ -38,7 +44,8 @@
 namespace galp {
 
 constexpr int kTuneOptions = 3;
-constexpr int kStreamsLine = NUM_BUCKETS;   // the cache line of the stream choice
+constexpr int kStreamsLine = NUM_BUCKETS;    // the cache line of the stream choice
+constexpr int kRowsLine = NUM_BUCKETS + 1;   // and of one launch or a kernel per class
 
 constexpr int kTuneIters = 10;   // iterations of each timed run
 
@@ -119,7 +126,8 @@ static std::vector<CacheLine> read_cache(const char *path) {
         CacheLine c;
         if (!(is >> c.arch >> c.method >> c.cls >> c.lv >> c.le >> c.opt)) continue;
         if ((c.cls >= 0 && c.cls < NUM_BUCKETS && c.opt >= 0 && c.opt < kTuneOptions) ||
-            (c.cls == kStreamsLine && (c.opt == 1 || c.opt == 3)))
+            (c.cls == kStreamsLine && (c.opt == 1 || c.opt == 3)) ||
+            (c.cls == kRowsLine && (c.opt == 0 || c.opt == 1)))
             out.push_back(c);
     }
     return out;
@@ -135,9 +143,18 @@ GALP_API int galp_graph_set_tuning(galp_graph *g, const int32_t *options) {
     if (!g || !options) return GALP_EINVAL;
     for (int b = 0; b < NUM_BUCKETS; ++b)
         if (options[b] < 0 || options[b] >= kTuneOptions) return fail(g->ctx, GALP_EINVAL, "tuning option out of range");
-    for (int b = 0; b < NUM_BUCKETS; ++b) g->tune[b] = (int8_t)options[b];
-    g->class_kernels = true;
+    g->class_kernels = false;
+    for (int b = 0; b < NUM_BUCKETS; ++b) {
+        g->tune[b] = (int8_t)options[b];
+        if (b <= fused_top(g) && options[b]) g->class_kernels = true;
+    }
     invalidate_captured(g);
+    return GALP_OK;
+}
+
+GALP_API int galp_graph_row_launches(galp_graph *g, int32_t *mode) {
+    if (!g || !mode) return GALP_EINVAL;
+    *mode = fused_rows(g) ? 0 : concurrent_classes(g) ? 3 : 1;
     return GALP_OK;
 }
 
@@ -163,6 +180,10 @@ GALP_API int galp_graph_autotune(galp_graph *g, int32_t reps, const char *cache_
     const int32_t capture = g->opts.graph_capture;
     g->opts.graph_capture = 0;
     invalidate_captured(g);
+    const bool class_kernels = g->class_kernels;
+    g->class_kernels = false;
+    const bool fusible = fused_rows(g);   // by size: one launch for the row classes
+    g->class_kernels = true;              // until the choice below
     int rc = GALP_OK;
     bool need[NUM_BUCKETS] = {};
     bool any = false;
@@ -205,6 +226,28 @@ GALP_API int galp_graph_autotune(galp_graph *g, int32_t reps, const char *cache_
         }
         g->streams = (int8_t)mode;
     }
+    bool per_class = !fusible;   // a kernel per class
+    if (rc == GALP_OK && fusible) {
+        const int lv = ilog2(g->n), le = ilog2(g->m);
+        int opt = -1;
+        for (const CacheLine &c : cache)
+            if (c.arch == arch && c.method == g->opts.method && c.cls == kRowsLine && c.lv == lv && c.le == le)
+                opt = c.opt;
+        if (opt < 0) {
+            double tbest[2] = {1e300, 1e300};
+            for (int round = 0; round < reps && rc == GALP_OK; ++round)
+                for (int q = 0; q < 2 && rc == GALP_OK; ++q) {
+                    g->class_kernels = q != 0;
+                    galp_run_result res{};
+                    rc = galp_lp_run(g, kTuneIters, 0, nullptr, &res);
+                    if (rc == GALP_OK) tbest[q] = std::min(tbest[q], res.device_ms);
+                }
+            opt = tbest[1] < 0.97 * tbest[0];
+            if (rc == GALP_OK) fresh.push_back(CacheLine{arch, g->opts.method, kRowsLine, lv, le, opt});
+        }
+        per_class = opt != 0;
+    }
+    g->class_kernels = rc != GALP_OK ? class_kernels : fusible && per_class;
     if (rc == GALP_OK && g->opts.dispatch == GALP_DISPATCH_LEARNED && !g->ooc) {
         // the judge: iteration by iteration, routing by the network against
         // routing by the degree classes alone (the plain dispatcher), on
@@ -247,6 +290,8 @@ GALP_API int galp_graph_autotune(galp_graph *g, int32_t reps, const char *cache_
             const BucketRange &r = g->bucket[b];
             fresh.push_back(CacheLine{arch, g->opts.method, b, ilog2(r.nv), ilog2(r.edges), g->tune[b]});
         }
+    if (!per_class)   // options that nothing uses: as if set by hand to what runs
+        for (int b = 0; b <= fused_top(g); ++b) g->tune[b] = 0;
     g->opts.dispatch = dispatch;
     g->opts.graph_capture = capture;
     invalidate_captured(g);
@@ -263,6 +308,7 @@ GALP_API int galp_graph_autotune(galp_graph *g, int32_t reps, const char *cache_
         for (int b = 0; b < NUM_BUCKETS; ++b) chosen[b] = g->tune[b];
         chosen[kStreamsLine] = g->streams;
         for (int b = kStreamsLine + 1; b < 16; ++b) chosen[b] = 0;
+        chosen[15] = g->class_kernels;
         if (g->opts.dispatch == GALP_DISPATCH_LEARNED) {   // the judge's mask
             chosen[kStreamsLine + 1] = (int32_t)(uint32_t)g->learn_mask;
             chosen[kStreamsLine + 2] = (int32_t)(uint32_t)(g->learn_mask >> 32);

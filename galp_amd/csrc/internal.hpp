@@ -385,7 +385,9 @@ struct galp_graph {
     galp::BatchState *batch = nullptr;
     galp::FrontState *front = nullptr;
     int8_t tune[galp::NUM_BUCKETS] = {};   // kernel configuration per degree class (autotuner)
-    bool class_kernels = false;   // options set by hand: a kernel per class at every size
+    // a kernel per class at every size: the autotuner's choice, or options set
+    // by hand for classes that the one launch covers
+    bool class_kernels = false;
     int8_t streams = 0;   // in-core class kernels: 0 by size, 1 one stream, 3 three (the autotuner's choice)
     // learned dispatch in core: bit i set = iteration i routes by the network,
     // clear = by the degree classes alone (the judge's choice, autotune.hip);
@@ -456,12 +458,21 @@ constexpr int64_t kConcurrentMinEdges = (int64_t)1 << 24;
 constexpr int64_t kConcurrentMaxVertices = (int64_t)1 << 25;
 // All row classes below B4K in one launch (rows_fused.hpp): in core, up to
 // kFusedMaxEdges edges, the default variants, unless single kernels are timed
-// or were chosen by hand (galp_graph_set_tuning).
+// or class kernels were chosen (g->class_kernels).  Ten iterations in one
+// launch each against class kernels on three streams: RMAT-20 of 18 / 24 / 31
+// M edges 1323 / 1632 / 1854 us against 1533 / 1901 / 2145, LFR of 17 / 23 /
+// 29 M 1243 / 1726 / 2061 against 1968 / 2202 / 2569; planted partitions of 17
+// and 31 M, whose rows are nearly all of one class, 1128 and 1915 against 963
+// and 1795, which the size alone does not tell (the autotuner times it).
 // The sort method's kernel holds 16 keys a lane for its largest class and has
 // half the waves of the class kernels: RMAT-20 (31 M edges) 3.89 ms with a
 // kernel per class, 4.08 fused.
 constexpr int64_t kFusedMaxEdges = (int64_t)1 << 25;
 constexpr int64_t kFusedMaxEdgesSort = (int64_t)1 << 24;
+// The classes it covers are b <= kFusedTop (the sort method's: kFusedTopSort).
+constexpr int kFusedTop = B_B2K;
+constexpr int kFusedTopSort = B_B1K;
+inline int fused_top(const galp_graph *g) { return g->opts.method == GALP_METHOD_HASH ? kFusedTop : kFusedTopSort; }
 bool fused_rows(const galp_graph *g);
 // An iteration's last kernel may do its bookkeeping: not in a batch (each
 // graph has its own) nor while samples are logged (the log kernel comes after

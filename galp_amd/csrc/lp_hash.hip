@@ -378,7 +378,7 @@ k_hash_lds(const E *__restrict__ off, const int32_t *__restrict__ nbr,
 // 513..2048 with a block per row.  The resolver and the table kernels adapt to
 // diverse labels by themselves (peel rounds stop), so learned dispatch's two
 // lists of a class run the same code one after the other.
-constexpr int kHashRows = B_B2K + 1;
+constexpr int kHashRows = kFusedTop + 1;
 template <int T, int EPT, int CAPBITS, typename E>
 __device__ __forceinline__ uint32_t fused_tables(const RowsWork &w, const E *off, const int32_t *nbr,
                                                  const int32_t *prev, int32_t *next, uint32_t *tab, uint32_t *sred,

@@ -425,7 +425,7 @@ k_sort_reg(const E *__restrict__ off, const int32_t *__restrict__ nbr, const int
 // ---------------------------------------------------------------------------
 // All classes up to degree 1024 in one launch (rows_fused.hpp): the lane
 // groups, and 65..1024 with a wave per row sorted in registers.
-constexpr int kSortRows = B_B1K + 1;
+constexpr int kSortRows = kFusedTopSort + 1;
 template <int EPT, typename E>
 __device__ __forceinline__ uint32_t fused_sort(const RowsWork &w, const E *off, const int32_t *nbr,
                                                const int32_t *prev, int32_t *next, int32_t *err) {

@@ -267,7 +267,10 @@ GALP_API int galp_graph_dispatch_stats(galp_graph *g, int64_t *out, int32_t max,
  * rounds, reads each class's device time from per-kernel events and keeps
  * its fastest option; then, in core, it times such runs with the class
  * kernels on one stream and on three and keeps the size rule's choice
- * unless the other is more than 3 % faster; under learned dispatch it then
+ * unless the other is more than 3 % faster; on a graph small enough to run
+ * its row classes in one launch it times that launch against the class
+ * kernels so chosen, which have to be more than 3 % faster to replace it;
+ * under learned dispatch it then
  * judges the network against the plain classes per iteration
  * (galp_graph_set_learned_iterations) and, when some iterations go to the
  * classes alone, times the class options again under that mask.  It leaves
@@ -276,10 +279,12 @@ GALP_API int galp_graph_dispatch_stats(galp_graph *g, int64_t *out, int32_t max,
  * were.  cache_path (may be NULL) names a text file of earlier
  * choices keyed by device arch, method and the class's log2 sizes; hits are
  * reused without timing and new choices are appended.  chosen (may be NULL)
- * receives 16 entries: the 12 class options, then the stream choice (1 or 3;
- * 0 where not timed), then the judge's mask (two halves; zeros without
- * learned dispatch), then zeros.  Labels never depend on the choices.  No
- * reference counterpart (fixed block sizes, lfht.cuh:127-165). */
+ * receives 16 entries: the 12 class options as the next run uses them (0 for
+ * the classes that run in one launch), then the stream choice of the class
+ * kernels (1 or 3; 0 where not timed), then the judge's mask (two halves;
+ * zeros without learned dispatch), then 1 where a graph of one-launch size
+ * was given the class kernels, else 0.  Labels never depend on the choices.
+ * No reference counterpart (fixed block sizes, lfht.cuh:127-165). */
 GALP_API int galp_graph_autotune(galp_graph *g, int32_t reps, const char *cache_path, int32_t *chosen);
 /* Learned dispatch in core: which iterations route by the network (bit i
  * for iteration i, bit 63 for every later one); the others run the plain
@@ -290,8 +295,15 @@ GALP_API int galp_graph_autotune(galp_graph *g, int32_t reps, const char *cache_
  * iteration by the network.  Labels never depend on it.  No reference
  * counterpart. */
 GALP_API int galp_graph_set_learned_iterations(galp_graph *g, uint64_t mask);
-/* Sets the option of every class directly (12 entries, each 0..2). */
+/* Sets the option of every class directly (12 entries, each 0..2).  An option
+ * other than the default 0 for a class that a small or mid-sized graph would
+ * run in one launch with others gives it a kernel per class; all such options
+ * 0 give back the choice by size. */
 GALP_API int galp_graph_set_tuning(galp_graph *g, const int32_t *options);
+/* How the next iteration over every row launches its classes: *mode = 0 in one
+ * launch for the classes up to 2048 edges (sort: 1024) and a kernel for each
+ * longer class; 1 or 3 a kernel per class, on one stream or three. */
+GALP_API int galp_graph_row_launches(galp_graph *g, int32_t *mode);
 
 /* ---- batched runs --------------------------------------------------------
  * Declares the uploaded (in-core) CSR to be the disjoint union of ngraphs

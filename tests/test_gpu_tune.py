@@ -134,3 +134,65 @@ def test_autotune_keeps_profile_totals(ctx):
         assert after == before
         labels, _ = g.run(10)
         assert np.array_equal(labels, final)
+
+
+@pytest.mark.parametrize("method", [_abi.METHOD_HASH, _abi.METHOD_SORT])
+def test_tuned_graph_runs_the_choice(ctx, tmp_path, method):
+    """A mid-sized graph runs its rows in one launch (row_launches 0) by
+    default and with the default options set by hand; options for the classes
+    the launch covers take a kernel per class; the autotuner times both, its
+    choice is what runs, and it holds for a graph given the same options and
+    through the cache.  Labels are the oracle's either way."""
+    off, nbr = _abi.gen_rmat(16, 16, seed=27)
+    final, _, _ = oracle.lp_run(off, nbr, niter=10)
+    covered = 10 if method == _abi.METHOD_HASH else 9   # classes of up to 2048 (1024) edges
+    cache = str(tmp_path / "tune.txt")
+
+    def check(g, mode):
+        assert g.row_launches() == mode
+        assert np.array_equal(g.run(10)[0], final)
+
+    with _abi.Graph(ctx, off, nbr, method=method) as g:
+        check(g, 0)
+        g.set_tuning([0] * 4 + [1] + [0] * 7)
+        check(g, 1)
+        g.set_tuning([0] * covered + [1] * (12 - covered))   # classes with a kernel of their own
+        check(g, 0)
+        g.set_tuning([0] * 12)
+        check(g, 0)
+        chosen = g.autotune(reps=3, cache_path=cache)
+        mode = g.tuned_streams if g.tuned_class_kernels else 0
+        print(f"[tune] method {method}: rows in {mode or 'one launch'}, options {chosen.tolist()}", flush=True)
+        check(g, mode)
+        if mode == 0:   # the options of covered classes are not in use
+            assert not chosen[:covered].any()
+            g.set_tuning(chosen)
+            check(g, 0)
+    rows = [x.split() for x in open(cache).read().split("\n") if x.strip()]
+    line = [r for r in rows if r[2] == "13"]
+    assert len(line) == 1 and line[0][5] == str(int(mode != 0))
+    for choice in ("0", "1"):
+        with open(cache, "w") as f:
+            f.write("\n".join(" ".join(r[:5] + [choice]) if r[2] == "13" else " ".join(r) for r in rows) + "\n")
+        with _abi.Graph(ctx, off, nbr, method=method) as g:
+            g.autotune(reps=1, cache_path=cache)
+            assert g.tuned_class_kernels == (choice == "1")
+            check(g, g.tuned_streams if choice == "1" else 0)
+
+
+def test_row_launches_by_size_and_profile(ctx):
+    """Per-kernel profiling takes a kernel per class; so does a sort graph of
+    2^24 edges, three streams wide."""
+    off, nbr = _abi.gen_rmat(14, 16, seed=28)
+    with _abi.Graph(ctx, off, nbr, profile=1) as g:
+        assert g.row_launches() == 1
+    off, nbr = _abi.gen_planted_partition(420000, 256, 18, 4, 3)
+    assert 1 << 24 <= len(nbr) < 1 << 25
+    for method, mode in ((_abi.METHOD_HASH, 0), (_abi.METHOD_SORT, 3)):
+        with _abi.Graph(ctx, off, nbr, method=method) as g:
+            assert g.row_launches() == mode
+            if mode == 0:
+                g.autotune(reps=3)
+                print(f"[tune] PP-420K: rows in {g.row_launches() or 'one launch'}", flush=True)
+                labels, res = g.run(10)
+                assert np.array_equal(labels, oracle.lp_run(off, nbr, niter=10)[0])
