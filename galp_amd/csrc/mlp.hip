@@ -275,9 +275,9 @@ k_mlp_train(float *__restrict__ params, const float *__restrict__ x, const float
     }
 }
 
-// The same training run for H = 32 on the matrix units, bit for bit: an fp32
-// MFMA adds its products to the accumulator in order of k, each by a fused
-// multiply-add, which is what the sums of k_mlp_train compile to.  That
+// The same training run for H = 32 on the matrix units.  An fp32 MFMA adds its
+// products to the accumulator in order of k, each by a fused multiply-add, so
+// the sums run in the order of k_mlp_train's and round as they do.  That
 // kernel waits on LDS (two reads per multiply-add in the sums over samples:
 // 82 us a minibatch of 512); here a minibatch takes 15 us, of which the
 // busiest SIMD's MFMAs are 7.
