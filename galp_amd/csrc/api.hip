@@ -403,18 +403,18 @@ static int upload_impl(galp_graph *g, const galp_csr_view *c) {
         GALP_HIP(ctx, hipMemcpy(g->d_iperm, iperm.data(), 4 * (size_t)n, hipMemcpyHostToDevice));
     }
     // Whether every row's ids strictly ascend (the closed form of the first
-    // iteration) and, then, whether the graph is symmetric (the lists of
-    // frontier.hip), on the rows in their input numbering.
+    // iteration), on the rows in their input numbering, and, then, whether the
+    // graph is symmetric (the lists of frontier.hip).
     GALP_TRY(dev_fill_u32(g, (uint32_t *)g->d_stop, 1, 0u));   // the row check's flag, until the first init
     const bool lists = m >= kFrontMinEdges &&
                        (g->opts.method == GALP_METHOD_HASH ? g->opts.variant == 1
                                                            : g->opts.policy != GALP_POLICY_LI);
     bool symmetric = false;
-    auto check_rows = [&](const void *d_off, bool off64, const int32_t *d_nbr) {
+    auto check_rows = [&] {
         GALP_HIP(ctx, hipMemcpyAsync(g->h_pinned, g->d_stop, 4, hipMemcpyDeviceToHost, g->stream));
         GALP_HIP(ctx, hipStreamSynchronize(g->stream));
         g->rows_ascend = g->h_pinned[0] == 0;
-        return lists && g->rows_ascend ? dev_check_symmetric(g, d_off, off64, d_nbr, nullptr, &symmetric) : GALP_OK;
+        return lists && g->rows_ascend ? dev_check_symmetric(g, g->d_nbr, &symmetric) : GALP_OK;
     };
     if (g->reorder && !ooc) {
         int64_t *d_off_old = nullptr;
@@ -430,7 +430,7 @@ static int upload_impl(galp_graph *g, const galp_csr_view *c) {
         hipError_t e2 = m ? hipMemcpy(d_nbr_old, c->neighbors, 4 * (size_t)m, hipMemcpyHostToDevice) : hipSuccess;
         rc = (e1 == hipSuccess && e2 == hipSuccess) ? dev_permute_rows(g, d_off_old, d_nbr_old, g->d_nbr, g->d_stop)
                                                     : fail(ctx, GALP_EHIP, "upload of the original CSR failed");
-        if (rc == GALP_OK) rc = check_rows(d_off_old, true, d_nbr_old);
+        if (rc == GALP_OK) rc = check_rows();
         hipError_t e3 = hipStreamSynchronize(g->stream);
         (void)hipFree(d_off_old);
         (void)hipFree(d_nbr_old);
@@ -442,7 +442,7 @@ static int upload_impl(galp_graph *g, const galp_csr_view *c) {
             GALP_HIP(ctx, hipMemcpy(g->d_nbr, c->neighbors, 4 * (size_t)m, hipMemcpyHostToDevice));
             GALP_TRY(dev_check_rows(g, g->d_stop));
         }
-        if (!ooc) GALP_TRY(check_rows(g->d_off, g->off64, g->d_nbr));
+        if (!ooc) GALP_TRY(check_rows());
         if (!vlist.empty()) {
             GALP_TRY(dev_alloc(g, &g->d_vlist, (int64_t)vlist.size()));
             GALP_HIP(ctx, hipMemcpy(g->d_vlist, vlist.data(), 4 * vlist.size(), hipMemcpyHostToDevice));
@@ -484,8 +484,8 @@ static int upload_impl(galp_graph *g, const galp_csr_view *c) {
     if (ooc) {
         std::vector<int64_t> hub_item0(hub_nparts.size() + 1, 0);
         for (size_t h = 0; h < hub_nparts.size(); ++h) hub_item0[h + 1] = hub_item0[h] + hub_nparts[h];
-        GALP_TRY(ooc_setup(g, c, offi, perm, iperm, vlist, hub_vertices, hub_tile0, hub_item0));
-        if (lists && g->rows_ascend) GALP_TRY(ooc_check_symmetric(g, &symmetric));
+        GALP_TRY(ooc_setup(g, c, offi, perm, iperm, vlist, hub_vertices, hub_tile0, hub_item0, &symmetric));
+        symmetric = symmetric && lists && g->rows_ascend;
     }
     if (g->opts.method == GALP_METHOD_SORT) GALP_TRY(sort_setup(g));
     GALP_HIP(ctx, hipStreamSynchronize(g->stream));

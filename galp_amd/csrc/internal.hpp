@@ -242,7 +242,8 @@ static_assert(kFrontReady < kFrontCtl && kFrontCtl <= 64, "one wave clears the c
 // ones the three launches of an iteration (12 us) and the set-up (the
 // symmetry check, the memory) cost what the lists save (RMAT-18, 7.6 M
 // edges: 1741 us without, 1786 with; LFR-300K uploaded and run once, 6 M
-// edges: 5.7 ms without, 6.3 with; RMAT-20, 31 M: 5.6 and 3.8 ms).
+// edges: 5.7 ms without, 6.3 with a check that looked every edge up;
+// RMAT-20, 31 M: 5.6 and 3.8 ms).
 constexpr int64_t kFrontPushDiv = 8;
 // Out of core the rows of both steps are read over the host link where they
 // lie, in short pieces, so the lists have to be shorter to beat streaming all
@@ -502,7 +503,7 @@ int launch_sort_class(galp_graph *g, int b);   // one class of the whole graph (
 int ooc_setup(galp_graph *g, const galp_csr_view *c, const std::vector<int64_t> &offi,
               const std::vector<int32_t> &perm, const std::vector<int32_t> &iperm,
               const std::vector<int32_t> &vlist, const std::vector<int32_t> &hub_vertices,
-              const std::vector<int32_t> &hub_tile0, const std::vector<int64_t> &hub_item0);
+              const std::vector<int32_t> &hub_tile0, const std::vector<int64_t> &hub_item0, bool *symmetric);
 void ooc_free(galp_graph *g);
 int launch_ooc_iteration(galp_graph *g);
 // Policy 2: work queued on the graph's stream from here on follows every batch
@@ -512,9 +513,6 @@ int ooc_finish_copies(galp_graph *g);
 // The next streamed iteration copies every batch, also one that a buffer holds:
 // a run brings its own batches in, like the first one.
 void ooc_forget_batches(galp_graph *g);
-// Whether an out-of-core graph (rows ascending) is symmetric, on a copy of its
-// rows in device memory; not answered (false) where the card has no ample room.
-int ooc_check_symmetric(galp_graph *g, bool *symmetric);
 // Streams every batch through learn_features_view once (learned dispatch set-up).
 int ooc_features(galp_graph *g);
 
@@ -562,8 +560,8 @@ int front_setup(galp_graph *g);
 void front_free(galp_graph *g);
 bool front_now(const galp_graph *g);   // the iteration being launched may use the lists
 int launch_front(galp_graph *g);
-int dev_check_symmetric(galp_graph *g, const void *off, bool off64, const int32_t *nbr, const int32_t *iperm,
-                        bool *symmetric);
+int dev_check_symmetric(galp_graph *g, const int32_t *nbr, bool *symmetric, int32_t *last = nullptr,
+                        bool *ascend = nullptr);
 inline FrontList front_list(const galp_graph *g, int b) {
     if (!front_now(g)) return FrontList{nullptr, 0, nullptr, nullptr};
     const FrontState *F = g->front;

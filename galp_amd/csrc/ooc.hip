@@ -25,7 +25,6 @@
 // 10.5 with the lists, of which three streamed iterations take 7.
 
 #include <algorithm>
-#include <atomic>
 #include <cstring>
 #include <vector>
 
@@ -83,7 +82,7 @@ void ooc_free(galp_graph *g) {
 int ooc_setup(galp_graph *g, const galp_csr_view *c, const std::vector<int64_t> &offi,
               const std::vector<int32_t> &perm, const std::vector<int32_t> &iperm,
               const std::vector<int32_t> &vlist, const std::vector<int32_t> &hub_vertices,
-              const std::vector<int32_t> &hub_tile0, const std::vector<int64_t> &hub_item0) {
+              const std::vector<int32_t> &hub_tile0, const std::vector<int64_t> &hub_item0, bool *symmetric) {
     OocState *O = new (std::nothrow) OocState();
     if (!O) return fail(g->ctx, GALP_ENOMEM, "host allocation failed");
     g->ooc = O;
@@ -94,10 +93,6 @@ int ooc_setup(galp_graph *g, const galp_csr_view *c, const std::vector<int64_t> 
         return fail(g->ctx, GALP_ENOMEM, "pinned host buffer for the neighbour array");
     }
     const int32_t *src = c->neighbors;
-    // each row's last neighbour (internal numbering), and whether every row's
-    // input ids strictly ascend: the first iteration then needs no batch
-    std::vector<int32_t> last((size_t)n, -1);
-    std::atomic<bool> ascend{true};
     if (g->reorder) {
         const bool o64 = c->offsets_are_64 != 0;
         parallel_for(0, n, [&](int64_t k) {
@@ -105,26 +100,13 @@ int ooc_setup(galp_graph *g, const galp_csr_view *c, const std::vector<int64_t> 
             const int64_t b = o64 ? ((const int64_t *)c->offsets)[v] : ((const int32_t *)c->offsets)[v];
             const int64_t d = offi[(size_t)k + 1] - offi[(size_t)k];
             int32_t *dst = O->h_nbr + offi[(size_t)k];
-            bool up = true;
-            for (int64_t j = 0; j < d; ++j) {
-                dst[j] = perm[(size_t)src[b + j]];
-                up &= j == 0 || src[b + j - 1] < src[b + j];
-            }
-            if (d) last[(size_t)k] = dst[d - 1];
-            if (!up) ascend.store(false, std::memory_order_relaxed);
+            for (int64_t j = 0; j < d; ++j) dst[j] = perm[(size_t)src[b + j]];
         });
     } else {
         const int64_t chunk = 1 << 22;
         parallel_for(0, (m + chunk - 1) / chunk, [&](int64_t k) {
             const int64_t lo = k * chunk, hi = std::min(m, lo + chunk);
             std::memcpy(O->h_nbr + lo, src + lo, 4 * (size_t)(hi - lo));
-        });
-        parallel_for(0, n, [&](int64_t v) {
-            const int64_t b = offi[(size_t)v], e = offi[(size_t)v + 1];
-            bool up = true;
-            for (int64_t j = b + 1; j < e; ++j) up &= src[j - 1] < src[j];
-            if (e > b) last[(size_t)v] = src[e - 1];
-            if (!up) ascend.store(false, std::memory_order_relaxed);
         });
     }
     // batches and their share of every class and of the hub lists
@@ -191,15 +173,25 @@ int ooc_setup(galp_graph *g, const galp_csr_view *c, const std::vector<int64_t> 
     if (g->opts.policy == GALP_POLICY_OOC_ASYNC &&
         hipStreamCreateWithFlags(&O->copy_stream, hipStreamNonBlocking) != hipSuccess)
         return fail(g->ctx, GALP_EHIP, "out-of-core copy stream");
-    // kept only where the memory budget has room for it: without it the first
-    // iteration streams like the others
+    // Each row's last neighbour, with which the first iteration needs no batch
+    // where every row's ids ascend; that, and whether the graph is symmetric, is
+    // found in the same pass over the link (RMAT-20: 2.3 ms of an upload of 88;
+    // in the host's loop above the check and the records cost 10).  Kept only
+    // where the memory budget has room: without it the first iteration streams
+    // like the others.
     const std::string err = g->ctx->err;
-    if (ascend.load() && dev_alloc(g, &O->d_last, n) == GALP_OK) {
-        if (n && hipMemcpy(O->d_last, last.data(), 4 * (size_t)n, hipMemcpyHostToDevice) != hipSuccess)
-            return fail(g->ctx, GALP_EHIP, "out-of-core last neighbours");
-        g->rows_ascend = true;
+    const int64_t bytes = g->device_bytes;
+    if (dev_alloc(g, &O->d_last, n) != GALP_OK) {
+        g->ctx->err = err;   // doing without is no failure
+        return GALP_OK;
     }
-    g->ctx->err = err;   // doing without is no failure
+    const int rc = dev_check_symmetric(g, O->h_nbr, symmetric, O->d_last, &g->rows_ascend);
+    if (rc != GALP_OK) return rc;
+    if (!g->rows_ascend) {
+        (void)hipFree(O->d_last);
+        O->d_last = nullptr;
+        g->device_bytes = bytes;
+    }
     return GALP_OK;
 }
 
@@ -309,25 +301,6 @@ int ooc_features(galp_graph *g) {
         if (hipStreamSynchronize(g->stream) != hipSuccess) return fail(g->ctx, GALP_EHIP, "feature pass failed");
     }
     return GALP_OK;
-}
-
-int ooc_check_symmetric(galp_graph *g, bool *symmetric) {
-    *symmetric = false;
-    const size_t bytes = 4 * (size_t)g->m;
-    size_t fr = 0, tot = 0;
-    if (g->opts.mem_budget > 0 || hipMemGetInfo(&fr, &tot) != hipSuccess || fr / 4 < bytes) return GALP_OK;
-    int32_t *d_nbr = nullptr;
-    if (hipMalloc((void **)&d_nbr, bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        return GALP_OK;
-    }
-    int rc = GALP_OK;
-    if (hipMemcpyAsync(d_nbr, g->ooc->h_nbr, bytes, hipMemcpyHostToDevice, g->stream) != hipSuccess)
-        rc = fail(g->ctx, GALP_EHIP, "out-of-core symmetry check: copy");
-    if (rc == GALP_OK) rc = dev_check_symmetric(g, g->d_off, g->off64, d_nbr, g->d_iperm, symmetric);
-    (void)hipStreamSynchronize(g->stream);
-    (void)hipFree(d_nbr);
-    return rc;
 }
 
 // An iteration over the rows that can still change (frontier.hip) reads them

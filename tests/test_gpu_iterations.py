@@ -64,6 +64,23 @@ def test_first_iteration(ctx, order, opts):
         assert np.array_equal(g.labels(), ref)
 
 
+@pytest.mark.parametrize("reorder", [1, 0])
+def test_repeats_found_out_of_core(ctx, reorder):
+    """A repeated neighbour at any place of the pass over the ids: inside a
+    thread's eight edges, between two threads, waves, rounds and tiles, first
+    and last in its row.  Its label counts twice, so the closed form is wrong."""
+    n, d = 20000, 9001
+    rest = [[(3 * v + 1) % n] if v % 3 else [] for v in range(n - 2)]
+    for p in [1, 7, 8, 9, 511, 512, 513, 2047, 2048, 2049, 8191, 8192, 8193, d - 1, 0]:
+        row = np.arange(5, 5 + 2 * d, 2)
+        if p:
+            row[p] = row[p - 1]
+        off, nbr = csr([row.tolist(), [1, 2, 3]] + rest)   # p = 0: nothing repeated
+        with _abi.Graph(ctx, off, nbr, policy=_abi.POLICY_OOC_ASYNC, buffer_pow=14, reorder=reorder) as g:
+            g.init()
+            check_steps(g, off, nbr, 2)
+
+
 def test_first_iteration_logs_distinct_counts(ctx):
     """The distinct-label counts logged for the first iteration are the degrees."""
     off, nbr = mixed_rows(2, "ascending")
@@ -202,6 +219,39 @@ def test_one_way_edges_take_every_row(ctx, settling):
         g.init()
         check_steps(g, off2, nbr2, 8)
         assert "front" not in {k["name"] for k in g.profile()}
+
+
+@pytest.mark.parametrize("edit", ["none", "one-way", "swap", "triangle", "last-row"])
+@pytest.mark.parametrize("opts", [dict(), dict(reorder=0), dict(offsets64=1),
+                                  dict(policy=_abi.POLICY_OOC_ASYNC, buffer_pow=20, mem_budget=1 << 30)],
+                         ids=["hash", "noreorder", "off64", "ooc-budget"])
+def test_symmetry_check(ctx, settling, opts, edit):
+    """Lists are used on symmetric graphs, out of core also under a memory
+    budget, and on no other: one edge without its reverse, two edges whose
+    ends are exchanged (all degrees as before), a directed triangle, an edge
+    of the last rows."""
+    off, nbr, _ = settling
+    rows = np.repeat(np.arange(len(off) - 1), np.diff(off))
+    key = rows * np.int64(len(off)) + nbr
+
+    if edit == "one-way":
+        key = np.delete(key, 12345)
+    elif edit == "last-row":
+        key = np.delete(key, len(key) - 1)
+    elif edit == "swap":   # a -> b, c -> d become a -> d, c -> b
+        e, f = 1000, 5000000
+        (a, b), (c, d) = (rows[e], nbr[e]), (rows[f], nbr[f])
+        assert len({a, b, c, d}) == 4
+        key[[e, f]] = a * len(off) + d, c * len(off) + b
+    elif edit == "triangle":
+        tri = np.array([100, 150000, 300000])
+        key = np.concatenate([key, tri * np.int64(len(off)) + np.roll(tri, 1)])
+    key.sort()
+    assert np.all(key[1:] > key[:-1])
+    off2 = np.searchsorted(key // len(off), np.arange(len(off))).astype(np.int64)
+    with _abi.Graph(ctx, off2, (key % len(off)).astype(np.int32), profile=1, **opts) as g:
+        g.run(3, want_labels=False)
+        assert ("front" in {k["name"] for k in g.profile()}) == (edit == "none")
 
 
 @pytest.mark.parametrize("net", ["all-cand", "rand"])
