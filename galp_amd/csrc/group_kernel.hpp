@@ -96,8 +96,8 @@ __device__ __forceinline__ uint32_t group_rounds_lanes(const E *__restrict__ off
 // label and list id loaded through the scalar cache into scalar registers,
 // since they are the same in all lanes.  A round issues three vector memory
 // instructions (ids, gather, label) for six, and holds 25 vector registers for
-// 52, which the fused kernel's mix of classes gains from: LFR-1M learned 2124
-// -> 1973 us.  (The 512-graph batch, bound by the resolver's issue, is
+// 52, which the fused kernel's mix of classes gains from: LFR-1M learned 2127
+// -> 2058 us.  (The 512-graph batch, bound by the resolver's issue, is
 // unchanged, and two rows a wave, for G = 32, lost as much again to selects.)
 template <class Resolve, bool VLIST, typename E>
 __device__ __forceinline__ uint32_t wave_rounds(const E *__restrict__ off, const int32_t *__restrict__ nbr,
@@ -178,7 +178,7 @@ __device__ __forceinline__ uint32_t group_rounds(const E *__restrict__ off, cons
 // hd_total); chosen once per launch, so each choice is its own pipeline.
 // nv_dev, when given, holds the list's length (written on the device by an
 // earlier kernel; nv is then only its capacity).  front: the rows that can
-// still change (frontier.hip), walked instead when its mode word is set.
+// still change (frontier.hip), walked instead when front_lists_on.
 template <int G, class Resolve, class Alt, bool VLIST, typename E>
 __global__ void __launch_bounds__(256)
 k_group(const E *__restrict__ off, const int32_t *__restrict__ nbr,
