@@ -21,8 +21,10 @@
 // What bounds a streamed iteration is the link: all edges once, 50-57 GB/s.
 // Once few rows can still change (frontier.hip) the iteration reads those rows
 // over the link from where they lie, and nothing else.  RMAT-20 (31 M edges,
-// 10 iterations, batches of 2^22 edges): 27.4 ms streaming every iteration,
-// 10.5 with the lists, of which three streamed iterations take 7.
+// 10 iterations, batches of 2^22 edges): 27.3 ms streaming every iteration,
+// 12.1 with the lists, of which three streamed iterations take 7.5.
+// A run copies its own batches: a buffer's batch is used again only within the
+// run that copied it (with at most two batches, from its second iteration on).
 
 #include <algorithm>
 #include <cstring>
